@@ -474,8 +474,13 @@ __global__ void queue_clear_kernel(uint32_t* queue) {
 __global__ void leaf_geom_kernel(const NodeLink* __restrict__ link, const double* __restrict__ x,
                                  const double* __restrict__ y, const double* __restrict__ z,
                                  const double* __restrict__ q, NodeGeom* __restrict__ geom,
+                                 DevBox* __restrict__ boxes, int64_t nsys,
                                  const DevScalars* __restrict__ sc) {
   if (broken(sc)) return;
+  // the signs of the new charges are not collected: a later walk evaluates dipoles
+  for (int64_t s = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; s < nsys;
+       s += (int64_t)gridDim.x * blockDim.x)
+    boxes[s].qsign = kQPositive | kQNegative;
   const int64_t m = sc->nnodes;
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < m;
        i += (int64_t)gridDim.x * blockDim.x) {
@@ -640,8 +645,8 @@ void launch_lists(hipStream_t s, const ListArgs& a, bool record, int blocks,
 
 void launch_leaf_geom(hipStream_t s, const NodeLink* link, const double* x, const double* y,
                       const double* z, const double* q, NodeGeom* geom, int64_t cap,
-                      const DevScalars* sc) {
-  leaf_geom_kernel<<<grid_for(cap), kT, 0, s>>>(link, x, y, z, q, geom, sc);
+                      DevBox* boxes, int64_t nsys, const DevScalars* sc) {
+  leaf_geom_kernel<<<grid_for(cap), kT, 0, s>>>(link, x, y, z, q, geom, boxes, nsys, sc);
 }
 
 void launch_replay(hipStream_t s, const ReplayArgs& a, int blocks) {

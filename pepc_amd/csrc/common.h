@@ -31,7 +31,13 @@ struct DevBox {
   double boxsize[3];
   double cell[3];               // boxsize / 2^20, the refinement length
   double b2[kMaxLevel + 1];     // maxval(boxsize)^2 / 4^l
+  uint32_t qsign;               // kQPositive | kQNegative: signs among the charges
+  uint32_t pad;
 };
+
+// A system whose charges all have one sign has no dipole moments: a node's
+// expansion centre is the |charge|-weighted mean of its particles.
+enum : uint32_t { kQPositive = 1u, kQNegative = 2u };
 
 // Device-wide scalars the host reads once per solve (one small copy).
 struct DevScalars {
@@ -69,9 +75,10 @@ struct __align__(16) NodeLink {
   uint32_t level;
 };
 
-// Moments in the form the M2P kernel evaluates (see walk.hip): charge,
-// dipole, doubled diagonal quadrupole, off-diagonal quadrupole, trace.
-// Slots: 0 q | 1..3 p | 4..6 2*quad | 7 xy | 8 yz | 9 zx | 10 trace
+// Moments in the form the M2P kernel evaluates (see walk.hip): the traceless
+// quadrupole B = -3 (A2 - 2/3 tr I) with A2 = {2 quad, off-diagonals}, the
+// trace of quad, the dipole and the charge.
+// Slots: 0..2 Bxx Byy Bzz | 3 Bxy | 4 Byz | 5 Bzx | 6 tr | 7..9 p | 10 q
 template <typename R>
 struct __align__(16) NodeMoments {
   R v[16];

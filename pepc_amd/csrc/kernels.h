@@ -7,13 +7,14 @@ namespace pepc {
 
 // keys.hip
 int box_partial_blocks(int64_t n);
+constexpr int kBoxPartial = 7;   // doubles per block of launch_box's partial results
 void launch_box(hipStream_t s, int64_t n, const double* x, const double* y, const double* z,
-                int force_cubic, double* partial, DevBox* box, DevScalars* sc);
+                const double* q, int force_cubic, double* partial, DevBox* box, DevScalars* sc);
 // Batched systems: per-system boxes over the ranges [soff[s], soff[s+1]) and
 // the system index of every particle.
 void launch_box_batch(hipStream_t s, int nsys, const int64_t* soff, const double* x,
-                      const double* y, const double* z, int force_cubic, DevBox* boxes,
-                      uint32_t* sys, DevScalars* sc);
+                      const double* y, const double* z, const double* q, int force_cubic,
+                      DevBox* boxes, uint32_t* sys, DevScalars* sc);
 // sys == nullptr: one system with boxes[0].
 // Also writes rec[i] = {x, y, z, q} (input order) for launch_gather_rec.
 void launch_keys(hipStream_t s, int64_t n, const double* x, const double* y, const double* z,
@@ -146,6 +147,7 @@ struct WalkArgs {
   int nqueue = 1;                    // queues: one contiguous range of groups per XCD
   const uint32_t* sys;               // batched systems: system per particle (else nullptr)
   const uint32_t* sysroot;           // batched systems: root node per system
+  const DevBox* boxes;               // one per system (signs among its charges)
   int nbox;                          // periodic: lattice vectors walked per group (else 1)
   const double* vbox;                // periodic: 3 * nbox lattice vectors, (0,0,0) last
   // sinks (targets other than the grown particles; tx == nullptr otherwise):
@@ -164,7 +166,9 @@ void launch_queue_reset(hipStream_t s, uint32_t* queue);   // work-queue heads o
 // list_tile: M2P list capacity in LDS (0 = default: 64 FP32, 32 FP64;
 // FP32 takes 64 or 128, FP64 32 or 64).
 bool walk_list_tile_ok(int precision, int list_tile);
-void launch_walk(hipStream_t s, const WalkArgs& a, int precision, int blocks, int list_tile);
+// max_group: the most targets a group can have.
+void launch_walk(hipStream_t s, const WalkArgs& a, int precision, int blocks, int list_tile,
+                 int max_group);
 void launch_walk_stats(hipStream_t s, const WalkArgs& a);
 int walk_default_blocks(int precision, int list_tile);
 
@@ -287,7 +291,7 @@ void launch_lists(hipStream_t s, const ListArgs& a, bool record, int blocks,
                   unsigned long long* total);
 void launch_leaf_geom(hipStream_t s, const NodeLink* link, const double* x, const double* y,
                       const double* z, const double* q, NodeGeom* geom, int64_t cap,
-                      const DevScalars* sc);
+                      DevBox* boxes, int64_t nsys, const DevScalars* sc);
 struct ReplayArgs {
   const double *x, *y, *z;
   const NodeGeom* geom;

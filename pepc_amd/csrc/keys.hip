@@ -14,12 +14,23 @@ namespace {
 
 constexpr int kBoxThreads = 256;
 
+// Signs of a charge as DevBox::qsign bits; a NaN counts as both.
+__device__ __forceinline__ uint32_t charge_sign(double q) {
+  return (!(q <= 0.0) ? kQPositive : 0u) | (!(q >= 0.0) ? kQNegative : 0u);
+}
+// The bits over a wave, the same in every lane.
+__device__ __forceinline__ uint32_t wave_sign(uint32_t s) {
+  return (__ballot(s & kQPositive) ? kQPositive : 0u) | (__ballot(s & kQNegative) ? kQNegative : 0u);
+}
+
 __global__ __launch_bounds__(kBoxThreads) void box_partial_kernel(
     int64_t n, const double* __restrict__ x, const double* __restrict__ y,
-    const double* __restrict__ z, double* __restrict__ partial, DevScalars* __restrict__ sc) {
+    const double* __restrict__ z, const double* __restrict__ q, double* __restrict__ partial,
+    DevScalars* __restrict__ sc) {
   double mn[3] = {INFINITY, INFINITY, INFINITY};
   double mx[3] = {-INFINITY, -INFINITY, -INFINITY};
   bool nonfinite = false;
+  uint32_t sign = 0u;
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * blockDim.x) {
     double v0 = x[i], v1 = y[i], v2 = z[i];
@@ -27,10 +38,14 @@ __global__ __launch_bounds__(kBoxThreads) void box_partial_kernel(
     mn[0] = fmin(mn[0], v0); mx[0] = fmax(mx[0], v0);
     mn[1] = fmin(mn[1], v1); mx[1] = fmax(mx[1], v1);
     mn[2] = fmin(mn[2], v2); mx[2] = fmax(mx[2], v2);
+    sign |= charge_sign(q[i]);
   }
   if (__ballot(nonfinite) != 0ull && lane_id() == 0) atomicOr(&sc->flags, kFlagBadBox);
   __shared__ double red[6][kBoxThreads / kWave];
+  __shared__ uint32_t rsign[kBoxThreads / kWave];
   const int w = threadIdx.x / kWave;
+  sign = wave_sign(sign);
+  if (lane_id() == 0) rsign[w] = sign;
 #pragma unroll
   for (int d = 0; d < 3; ++d) {
     double a = wave_min(mn[d]), b = wave_max(mx[d]);
@@ -41,14 +56,18 @@ __global__ __launch_bounds__(kBoxThreads) void box_partial_kernel(
     const int d = threadIdx.x;
     double v = red[d][0];
     for (int k = 1; k < kBoxThreads / kWave; ++k) v = d < 3 ? fmin(v, red[d][k]) : fmax(v, red[d][k]);
-    partial[blockIdx.x * 6 + d] = v;
+    partial[blockIdx.x * kBoxPartial + d] = v;
+  } else if (threadIdx.x == 6) {   // the sign bits as a small whole number
+    uint32_t v = rsign[0];
+    for (int k = 1; k < kBoxThreads / kWave; ++k) v |= rsign[k];
+    partial[blockIdx.x * kBoxPartial + 6] = (double)v;
   }
 }
 
 // module_box.f90:65-93 from the coordinate extrema: optional cube, margin
 // boxsize/10000 on both sides, refinement cell, boxlength2 table.
-__device__ void box_finalize(double mn[3], double mx[3], int force_cubic, DevBox* __restrict__ box,
-                             DevScalars* __restrict__ sc) {
+__device__ void box_finalize(double mn[3], double mx[3], uint32_t qsign, int force_cubic,
+                             DevBox* __restrict__ box, DevScalars* __restrict__ sc) {
   if (force_cubic) {  // module_box.f90:71-74
     double lo = fmin(fmin(mn[0], mn[1]), mn[2]);
     double hi = fmax(fmax(mx[0], mx[1]), mx[2]);
@@ -68,6 +87,7 @@ __device__ void box_finalize(double mn[3], double mx[3], int force_cubic, DevBox
   double m = fmax(fmax(box->boxsize[0], box->boxsize[1]), box->boxsize[2]);
   box->b2[0] = m * m;
   for (int l = 1; l <= kMaxLevel; ++l) box->b2[l] = box->b2[l - 1] / 4.0;
+  box->qsign = qsign;
   if (bad) atomicOr(&sc->flags, kFlagBadBox);
 }
 
@@ -76,17 +96,20 @@ __global__ __launch_bounds__(kWave) void box_final_kernel(int nblocks, const dou
                                                          DevScalars* __restrict__ sc) {
   double mn[3] = {INFINITY, INFINITY, INFINITY};
   double mx[3] = {-INFINITY, -INFINITY, -INFINITY};
+  uint32_t sign = 0u;
   for (int b = threadIdx.x; b < nblocks; b += kWave) {
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
-      mn[d] = fmin(mn[d], partial[b * 6 + d]);
-      mx[d] = fmax(mx[d], partial[b * 6 + 3 + d]);
+      mn[d] = fmin(mn[d], partial[b * kBoxPartial + d]);
+      mx[d] = fmax(mx[d], partial[b * kBoxPartial + 3 + d]);
     }
+    sign |= (uint32_t)partial[b * kBoxPartial + 6];
   }
+  sign = wave_sign(sign);
 #pragma unroll
   for (int d = 0; d < 3; ++d) { mn[d] = wave_min(mn[d]); mx[d] = wave_max(mx[d]); }
   if (threadIdx.x != 0) return;
-  box_finalize(mn, mx, force_cubic, box, sc);
+  box_finalize(mn, mx, sign, force_cubic, box, sc);
 }
 
 // Batched systems: one block per system computes that system's box over its
@@ -94,9 +117,11 @@ __global__ __launch_bounds__(kWave) void box_final_kernel(int nblocks, const dou
 // index.  An empty system gets a unit box that no particle refers to.
 __global__ __launch_bounds__(kBoxThreads) void box_segment_kernel(
     int nsys, const int64_t* __restrict__ soff, const double* __restrict__ x,
-    const double* __restrict__ y, const double* __restrict__ z, int force_cubic,
-    DevBox* __restrict__ boxes, uint32_t* __restrict__ sys, DevScalars* __restrict__ sc) {
+    const double* __restrict__ y, const double* __restrict__ z, const double* __restrict__ q,
+    int force_cubic, DevBox* __restrict__ boxes, uint32_t* __restrict__ sys,
+    DevScalars* __restrict__ sc) {
   const int sid = blockIdx.x;
+  uint32_t sign = 0u;
   const int64_t b = soff[sid], e = soff[sid + 1];
   double mn[3] = {INFINITY, INFINITY, INFINITY};
   double mx[3] = {-INFINITY, -INFINITY, -INFINITY};
@@ -108,10 +133,14 @@ __global__ __launch_bounds__(kBoxThreads) void box_segment_kernel(
     mn[1] = fmin(mn[1], v1); mx[1] = fmax(mx[1], v1);
     mn[2] = fmin(mn[2], v2); mx[2] = fmax(mx[2], v2);
     sys[i] = (uint32_t)sid;
+    sign |= charge_sign(q[i]);
   }
   if (__ballot(nonfinite) != 0ull && lane_id() == 0) atomicOr(&sc->flags, kFlagBadBox);
   __shared__ double red[6][kBoxThreads / kWave];
+  __shared__ uint32_t rsign[kBoxThreads / kWave];
   const int w = threadIdx.x / kWave;
+  sign = wave_sign(sign);
+  if (lane_id() == 0) rsign[w] = sign;
 #pragma unroll
   for (int d = 0; d < 3; ++d) {
     double lo = wave_min(mn[d]), hi = wave_max(mx[d]);
@@ -127,10 +156,11 @@ __global__ __launch_bounds__(kBoxThreads) void box_segment_kernel(
       mx[d] = fmax(mx[d], red[3 + d][k]);
     }
   }
+  for (int k = 1; k < kBoxThreads / kWave; ++k) sign |= rsign[k];
   if (e <= b) {
     for (int d = 0; d < 3; ++d) { mn[d] = 0.0; mx[d] = 1.0; }
   }
-  box_finalize(mn, mx, force_cubic, boxes + sid, sc);
+  box_finalize(mn, mx, sign, force_cubic, boxes + sid, sc);
 }
 
 // Hilbert tables packed 3 bits per entry (module_spacefilling.f90:389-390):
@@ -245,16 +275,16 @@ int box_partial_blocks(int64_t n) {
 }
 
 void launch_box(hipStream_t s, int64_t n, const double* x, const double* y, const double* z,
-                int force_cubic, double* partial, DevBox* box, DevScalars* sc) {
+                const double* q, int force_cubic, double* partial, DevBox* box, DevScalars* sc) {
   const int nb = box_partial_blocks(n);
-  box_partial_kernel<<<nb, kBoxThreads, 0, s>>>(n, x, y, z, partial, sc);
+  box_partial_kernel<<<nb, kBoxThreads, 0, s>>>(n, x, y, z, q, partial, sc);
   box_final_kernel<<<1, kWave, 0, s>>>(nb, partial, force_cubic, box, sc);
 }
 
 void launch_box_batch(hipStream_t s, int nsys, const int64_t* soff, const double* x,
-                      const double* y, const double* z, int force_cubic, DevBox* boxes,
-                      uint32_t* sys, DevScalars* sc) {
-  box_segment_kernel<<<nsys, kBoxThreads, 0, s>>>(nsys, soff, x, y, z, force_cubic, boxes, sys, sc);
+                      const double* y, const double* z, const double* q, int force_cubic,
+                      DevBox* boxes, uint32_t* sys, DevScalars* sc) {
+  box_segment_kernel<<<nsys, kBoxThreads, 0, s>>>(nsys, soff, x, y, z, q, force_cubic, boxes, sys, sc);
 }
 
 void launch_keys(hipStream_t s, int64_t n, const double* x, const double* y, const double* z,

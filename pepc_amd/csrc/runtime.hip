@@ -426,9 +426,9 @@ int grow_device_impl(Ctx* c, int64_t n, const double* x, const double* y, const 
   RECORD(c, 0);
   reset_scalars_kernel<<<1, 64, 0, s>>>(c->sc);
   if (nsys > 1)
-    launch_box_batch(s, (int)nsys, c->soff, x, y, z, c->cfg.force_cubic_domain, c->box, c->sys, c->sc);
+    launch_box_batch(s, (int)nsys, c->soff, x, y, z, q, c->cfg.force_cubic_domain, c->box, c->sys, c->sc);
   else
-    launch_box(s, n, x, y, z, c->cfg.force_cubic_domain, c->partial, c->box, c->sc);
+    launch_box(s, n, x, y, z, q, c->cfg.force_cubic_domain, c->partial, c->box, c->sc);
   launch_keys(s, n, x, y, z, q, c->box, sys, c->k0, c->v0, c->prec4);
   launch_sort_keys(s, c->k0, c->v0, c->k1, c->v1, n, c->hist, c->bsum, sys, nsys);
   launch_dup_detect(s, n, c->k0, sys, c->sc);
@@ -486,13 +486,15 @@ int traverse_device_impl(Ctx* c, double* ex, double* ey, double* ez, double* pot
   a.np2p = c->np2p; a.nm2p = c->nm2p; a.gstat = c->gstat; a.queue = c->queue; a.nqueue = c->nxcd;
   a.sys = c->nsys > 1 ? c->sys : nullptr;
   a.sysroot = c->sysroot;
+  a.boxes = c->box;
   if (c->periodic && c->nsys > 1)
     return fail(c, PEPC_GPU_EINVAL, "traverse: periodic boundaries need a single system");
   a.nbox = c->periodic ? c->nbox : 1;
   a.vbox = c->periodic ? c->vbox : nullptr;
   launch_walk_reset(s, a);
   RECORD(c, 2);
-  launch_walk(s, a, c->cfg.precision, c->walk_blocks, c->cfg.list_tile);
+  launch_walk(s, a, c->cfg.precision, c->walk_blocks, c->cfg.list_tile,
+              std::max(c->cfg.group_size, c->cfg.group_pack));
   if (c->periodic && c->far_field)
     launch_lattice_far(s, c->n, c->xs, c->ys, c->zs, c->qs, c->lgeom, c->ml, c->fact, c->linv,
                        c->cfg.sign, c->lpart, c->ldpart, c->lom, c->ldip, c->mu,
@@ -606,7 +608,7 @@ int traverse_sinks_run(Ctx* c, const SinkBufs& b, int64_t m, const double* x, co
   a.sc = c->sc;
   a.theta2 = c->cfg.theta2; a.eps2 = c->cfg.eps2; a.sign = c->cfg.sign;
   a.np2p = b.p2p; a.nm2p = b.m2p; a.gstat = nullptr; a.queue = c->queue; a.nqueue = c->nxcd;
-  a.sys = nullptr; a.sysroot = c->sysroot;
+  a.sys = nullptr; a.sysroot = c->sysroot; a.boxes = c->box;
   a.nbox = c->periodic ? c->nbox : 1;
   a.vbox = c->periodic ? c->vbox : nullptr;
   const double *tx = x, *ty = y, *tz = z;
@@ -629,7 +631,8 @@ int traverse_sinks_run(Ctx* c, const SinkBufs& b, int64_t m, const double* x, co
   a.tx = tx; a.ty = ty; a.tz = tz;
   a.ex = out[0]; a.ey = out[1]; a.ez = out[2]; a.pot = out[3]; a.work = out[4];
   launch_queue_reset(s, c->queue);
-  launch_walk(s, a, c->cfg.precision, c->walk_blocks, c->cfg.list_tile);
+  launch_walk(s, a, c->cfg.precision, c->walk_blocks, c->cfg.list_tile,
+              mode == PEPC_GPU_SINKS_GROUPED ? c->cfg.group_size : 1);
   if (c->periodic && c->far_field) {
     launch_lattice_sources(s, c->n, c->xs, c->ys, c->zs, c->qs, c->lgeom, c->ml, c->fact, c->lpart,
                            c->ldpart, c->lom, c->ldip, c->mu, c->fict, c->lcoef);
@@ -694,7 +697,7 @@ int pepc_gpu_create(void** out, const pepc_gpu_config* cfg) {
       delete c;
       return PEPC_GPU_EHIP;
     }
-  if (dalloc(c, &c->box, 1) || dalloc(c, &c->sc, 1) || dalloc(c, &c->partial, 1024 * 6) ||
+  if (dalloc(c, &c->box, 1) || dalloc(c, &c->sc, 1) || dalloc(c, &c->partial, 1024 * kBoxPartial) ||
       dalloc(c, &c->queue, kQueueWords) ||
       hipHostMalloc((void**)&c->sc_host, sizeof(DevScalars), hipHostMallocDefault) != hipSuccess) {
     free_all(c);
@@ -1470,7 +1473,7 @@ int pepc_gpu_replay_device(void* p, const double* x, const double* y, const doub
   HIPCHECK(c, hipSetDevice(c->cfg.device));
   hipStream_t s = c->stream;
   launch_gather4(s, c->n, c->v0, x, y, z, q, c->xs, c->ys, c->zs, c->qs);
-  launch_leaf_geom(s, c->link, c->xs, c->ys, c->zs, c->qs, c->geom, c->mcap, c->sc);
+  launch_leaf_geom(s, c->link, c->xs, c->ys, c->zs, c->qs, c->geom, c->mcap, c->box, c->nsys, c->sc);
   launch_upward(s, c->tb);
   ReplayArgs a;
   a.x = c->xs; a.y = c->ys; a.z = c->zs;

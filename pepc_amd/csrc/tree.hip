@@ -448,11 +448,12 @@ __device__ __forceinline__ void write_walk_forms(int64_t i, const double* m, dou
   g.cx = m[M_CX]; g.cy = m[M_CY]; g.cz = m[M_CZ]; g.b2 = b2;
   geom[i] = g;
   double w[12];
-  w[0] = m[M_Q];
-  w[1] = m[M_PX]; w[2] = m[M_PY]; w[3] = m[M_PZ];
-  w[4] = 2.0 * m[M_QX]; w[5] = 2.0 * m[M_QY]; w[6] = 2.0 * m[M_QZ];
-  w[7] = m[M_XY]; w[8] = m[M_YZ]; w[9] = m[M_ZX];
-  w[10] = (m[M_QX] + m[M_QY]) + m[M_QZ];
+  const double tr = (m[M_QX] + m[M_QY]) + m[M_QZ];
+  w[0] = 2.0 * tr - 6.0 * m[M_QX]; w[1] = 2.0 * tr - 6.0 * m[M_QY]; w[2] = 2.0 * tr - 6.0 * m[M_QZ];
+  w[3] = -3.0 * m[M_XY]; w[4] = -3.0 * m[M_YZ]; w[5] = -3.0 * m[M_ZX];
+  w[6] = tr;
+  w[7] = m[M_PX]; w[8] = m[M_PY]; w[9] = m[M_PZ];
+  w[10] = m[M_Q];
   w[11] = 0.0;
   if (prec == kWalkFP64) {
     double4* o = reinterpret_cast<double4*>(&wm64[i]);

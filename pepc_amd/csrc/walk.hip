@@ -9,10 +9,10 @@
 // reference's at the same group rule.
 //
 // Mapping to CDNA4.  One 64-lane wavefront owns one group at a time and pulls
-// the next group from a device queue (persistent kernel).  A group of cnt
-// targets occupies T = pow2 >= cnt lanes; the S = 64/T copies ("slices")
-// split every interaction list between them, so small groups still fill the
-// wave.  Traversal is breadth-parallel: each step pops up to 64 nodes from an
+// the next group from a device queue (persistent kernel).  A lane holds one
+// or two of the group's targets (NT); the W lanes that hold them all form a
+// slice, and the S = 64/W slices split every interaction list between them,
+// so small groups still fill the wave.  Traversal is breadth-parallel: each step pops up to 64 nodes from an
 // LDS stack, one node per lane, and decides it against the group's bounding
 // box; only nodes whose decision the box cannot settle run the exact
 // per-target FP64 test (all lanes, one ballot).  Accepted nodes and leaves are
@@ -21,9 +21,20 @@
 //
 // Precision.  FP32 path: coordinates relative to the group's first particle
 // (differences taken in FP64 once per node, then rounded), FP32 kernels with
-// fused multiply-add, per-target compensated (Kahan) accumulation of each
-// batch's partial sums.  FP64 path: absolute coordinates, FP64 kernels,
-// plain FP64 accumulation, as the reference.
+// fused multiply-add, FP32 partial sums per batch added to FP64 running sums
+// (more exact than the compensated FP32 sums they replace, with half the
+// instructions).  FP64 path: absolute coordinates, FP64 kernels, plain FP64
+// accumulation, as the reference.
+//
+// What bounds it: vector-ALU issue.  With four waves per SIMD this chip
+// issues an FP32 instruction every 3 clocks per SIMD and every other kind
+// (FP64, integer, compares, any with a scalar operand) every 4.3 to 4.8; the
+// 4.2M-particle explosion at theta 0.6 issued 4.36e9 VALU instructions at
+// 3.0 clocks each.  So the design counts instructions: traceless moments and
+// no dipole terms for one-signed charges (41 -> 35 per pair), list remainders
+// kept so that passes are full, one ballot transposition for the exact tests
+// and one for the pushes.  3.76e9 instructions, walk 5.88 -> 5.24 ms (FP64
+// 11.56 -> 10.52, theta 0.3 at 500,009 particles 2.90 -> 2.58).
 //
 // Periodic systems (PER): the group walks the tree once per lattice vector
 // vbox of the mirror boxes, with its targets shifted to x - vbox
@@ -45,8 +56,10 @@
 // (module_coulomb_kernels.f90:60-145) around the quadratic form
 // S = d.A.d of the quadrupole tensor; it is the same polynomial in d and the
 // moments (phi = q/r - d.p/r^3 + 3 S/r^5 - tr(A)/r^3 and E = -grad phi with
-// r^2 = d^2 + eps^2), evaluated with fewer operations.
+// r^2 = d^2 + eps^2), evaluated with fewer operations (see m2p).
 #include "kernels.h"
+
+#include <type_traits>
 
 namespace pepc {
 
@@ -62,7 +75,7 @@ constexpr uint32_t kTwigBit = 0x80000000u;
 
 template <typename R> struct Prec;
 template <> struct Prec<float> {
-  using V4 = float4;
+  using V4 = float __attribute__((ext_vector_type(4)));
   // v_rsq_f32 (1 ulp).  Its argument is r^2 = d^2 + eps^2 of an interaction
   // that is not a self term; the input guard of rsqrtf() only matters for
   // denormal arguments, which would need |d| and eps below 1e-19.
@@ -70,48 +83,56 @@ template <> struct Prec<float> {
   static __device__ __forceinline__ float fm(float a, float b, float c) { return fmaf(a, b, c); }
 };
 template <> struct Prec<double> {
-  using V4 = double4;
+  using V4 = double __attribute__((ext_vector_type(4)));
   static __device__ __forceinline__ double rsq(double x) { return rsqrt(x); }
   static __device__ __forceinline__ double fm(double a, double b, double c) { return fma(a, b, c); }
 };
 
 template <typename R>
 struct Acc {
-  R s[4];  // running sums   ex, ey, ez, pot
-  R c[4];  // compensation (FP32 only)
-  R p[4];  // partial sums of the current batch
+  double s[4];  // running sums   ex, ey, ez, pot
+  R p[4];       // partial sums of the current batch
 };
 
-// M2P: entry = {cx,cy,cz,q | px,py,pz,2qx | 2qy,2qz,xy,yz | zx,tr,-,-}; the
-// separation d is target minus centre of charge.  With w = 1/r^2, the matrix
-// A2 = [[2qx,xy,zx],[xy,2qy,yz],[zx,yz,2qz]], g = A2 d, S2 = d.g, a = d.p + tr:
-//   phi = (1/r) (q - w (a - 1.5 w S2))
-//   E   = (w/r) (c d + p - 3 w g),   c = q - 3 w (a - 2.5 w S2)
-// which is phi and -grad phi of module_coulomb_kernels.f90:60-145.
-template <typename R>
-__device__ __forceinline__ void m2p(R dx, R dy, R dz, const typename Prec<R>::V4& b,
-                                    const typename Prec<R>::V4& c, const typename Prec<R>::V4& d,
-                                    R q, R eps2, R* p) {
+// M2P.  With w = 1/r^2, the node's traceless quadrupole B = -3 (A2 - 2/3 tr I)
+// (A2 = 2 Qt, tr = trace Qt), g = B d, X = d.g + 2 tr eps^2 and p = the dipole:
+//   phi = (1/r) (q - w (d.p + 0.5 w X))
+//   E   = (w/r) (c d + p + w g),   c = q - w (3 d.p + 2.5 w X)
+// which is phi and -grad phi of module_coulomb_kernels.f90:60-145: the trace
+// terms of that form cancel against the trace part of d.A2 d up to eps^2.
+// The separation d is target minus centre of charge.
+// Entry: {cx,cy,cz,q | Bxx,Byy,Bzz,Bxy | Byz,Bzx,2 tr eps^2,px | py,pz,-,-}.
+// Without a dipole (DIP = false) its terms and its words are left out.
+template <typename R, bool DIP>
+__device__ __forceinline__ void m2p(R dx, R dy, R dz, R q, const typename Prec<R>::V4& b,
+                                    const typename Prec<R>::V4& c, R py, R pz, R eps2, R* p) {
   using P = Prec<R>;
   const R r2 = P::fm(dz, dz, P::fm(dy, dy, P::fm(dx, dx, eps2)));
   const R rd = P::rsq(r2);
   const R w = rd * rd;
   const R rd3 = rd * w;
-  const R px = b.x, py = b.y, pz = b.z, qx2 = b.w;
-  const R qy2 = c.x, qz2 = c.y, xy = c.z, yz = c.w;
-  const R zx = d.x, tr = d.y;
-  const R gx = P::fm(qx2, dx, P::fm(xy, dy, zx * dz));
-  const R gy = P::fm(qy2, dy, P::fm(xy, dx, yz * dz));
-  const R gz = P::fm(qz2, dz, P::fm(yz, dy, zx * dx));
-  const R s2 = P::fm(dz, gz, P::fm(dy, gy, dx * gx));
-  const R av = P::fm(dz, pz, P::fm(dy, py, P::fm(dx, px, tr)));
-  const R bv = w * s2;
-  p[3] = P::fm(rd, P::fm(-w, P::fm(R(-1.5), bv, av), q), p[3]);
-  const R w3 = R(3) * w;
-  const R cc = P::fm(-w3, P::fm(R(-2.5), bv, av), q);
-  p[0] = P::fm(rd3, P::fm(cc, dx, P::fm(-w3, gx, px)), p[0]);
-  p[1] = P::fm(rd3, P::fm(cc, dy, P::fm(-w3, gy, py)), p[1]);
-  p[2] = P::fm(rd3, P::fm(cc, dz, P::fm(-w3, gz, pz)), p[2]);
+  const R gx = P::fm(b.x, dx, P::fm(b.w, dy, c.y * dz));
+  const R gy = P::fm(b.y, dy, P::fm(b.w, dx, c.x * dz));
+  const R gz = P::fm(b.z, dz, P::fm(c.x, dy, c.y * dx));
+  const R x = P::fm(dz, gz, P::fm(dy, gy, P::fm(dx, gx, c.z)));
+  const R y = w * x;
+  if constexpr (DIP) {
+    const R px = c.w;
+    const R av = P::fm(dz, pz, P::fm(dy, py, dx * px));
+    p[3] = P::fm(rd, P::fm(-w, P::fm(R(0.5), y, av), q), p[3]);
+    const R cc = P::fm(-w, P::fm(R(2.5), y, R(3) * av), q);
+    p[0] = P::fm(rd3, P::fm(cc, dx, P::fm(w, gx, px)), p[0]);
+    p[1] = P::fm(rd3, P::fm(cc, dy, P::fm(w, gy, py)), p[1]);
+    p[2] = P::fm(rd3, P::fm(cc, dz, P::fm(w, gz, pz)), p[2]);
+  } else {
+    const R y2 = w * y;
+    p[3] = P::fm(rd, P::fm(R(-0.5), y2, q), p[3]);
+    const R e1 = rd3 * P::fm(R(-2.5), y2, q);
+    const R e5 = rd3 * w;
+    p[0] = P::fm(e5, gx, P::fm(e1, dx, p[0]));
+    p[1] = P::fm(e5, gy, P::fm(e1, dy, p[1]));
+    p[2] = P::fm(e5, gz, P::fm(e1, dz, p[2]));
+  }
 }
 
 // P2P (module_coulomb_kernels.f90:242-257): phi = q/r, E = q d / r^3.
@@ -130,18 +151,13 @@ __device__ __forceinline__ void p2p(R dx, R dy, R dz, R q, R eps2, bool self, R*
   p[2] = P::fm(qrd3, dz, p[2]);
 }
 
+// Adds a batch's partial sums to the running sums, which are FP64 in both
+// precisions.
 template <typename R>
 __device__ __forceinline__ void fold(Acc<R>& a) {
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
-    if constexpr (sizeof(R) == 4) {   // Kahan step on the batch's partial sum
-      const R y = a.p[k] - a.c[k];
-      const R t = a.s[k] + y;
-      a.c[k] = (t - a.s[k]) - y;
-      a.s[k] = t;
-    } else {
-      a.s[k] += a.p[k];
-    }
+    a.s[k] += (double)a.p[k];
     a.p[k] = R(0);
   }
 }
@@ -155,12 +171,66 @@ __device__ __forceinline__ bool mac_fails(double xt, double yt, double zt, doubl
   return !(theta2 * d2 > b2);
 }
 
+// Orders this wave's LDS accesses for the compiler.  A workgroup is one wave,
+// whose LDS instructions execute in order, so no wait or barrier instruction
+// is needed between one lane's write and another lane's read.
+__device__ __forceinline__ void wave_order() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// A value that is the same in every lane, moved to scalar registers.
+__device__ __forceinline__ uint32_t uniform(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_readfirstlane((int)v);
+}
+__device__ __forceinline__ double uniform(double v) {
+  const int lo = __builtin_amdgcn_readfirstlane(__double2loint(v));
+  const int hi = __builtin_amdgcn_readfirstlane(__double2hiint(v));
+  return __hiloint2double(hi, lo);
+}
+
+template <int kCtrl>
+__device__ __forceinline__ double dpp_move(double v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), kCtrl, 0xF, 0xF, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), kCtrl, 0xF, 0xF, false);
+  return __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double lane_value(double v, int l) {
+  const int lo = __builtin_amdgcn_readlane(__double2loint(v), l);
+  const int hi = __builtin_amdgcn_readlane(__double2hiint(v), l);
+  return __hiloint2double(hi, lo);
+}
+// Minimum over the wave (every lane active), uniform: each row of 16 lanes by
+// DPP, then the four rows through scalar reads; no LDS round trips.
+__device__ __forceinline__ double uniform_min(double v) {
+  v = fmin(v, dpp_move<0xB1>(v));    // quad_perm [1,0,3,2]
+  v = fmin(v, dpp_move<0x4E>(v));    // quad_perm [2,3,0,1]
+  v = fmin(v, dpp_move<0x124>(v));   // row_ror:4
+  v = fmin(v, dpp_move<0x128>(v));   // row_ror:8
+  return uniform(fmin(fmin(lane_value(v, 0), lane_value(v, 16)),
+                      fmin(lane_value(v, 32), lane_value(v, 48))));
+}
+
+// Centre and half width of the interval [lo, hi], the half width rounded up so
+// that lo and hi lie within it of the (rounded) centre.
+struct Span { double c, h; };
+__device__ __forceinline__ Span span_of(double lo, double hi) {
+  Span r;
+  r.c = uniform(0.5 * (lo + hi));
+  r.h = uniform(fmax(hi - r.c, r.c - lo) * (1.0 + 4e-15));
+  return r;
+}
+
 // LM: capacity of the M2P list staged in LDS (the list tile); the P2P list
 // holds kListP entries.  The default tiles (LM * sizeof(R) = 256 bytes per
 // float component: FP32 64, FP64 32) leave LDS for four one-wave workgroups
 // per SIMD; the register budget is held to the same four (at most 128 VGPRs).
 // The larger tiles are LDS-limited to three.
-template <typename R, int LM, bool PER, bool SINK>
+// NT: targets per lane.  Two halve the LDS reads per pair and fill groups of
+// 17 to 64 targets better (1,000,003 particles, G = 64: 1.40 -> 1.19 ms), one
+// fills groups up to 16 better (G = 16 unpacked: 1.76 against 1.64 ms) and
+// then takes two list entries per pass; FP64 has no registers for two.
+template <typename R, int LM, int NT, bool PER, bool SINK>
 __global__ __launch_bounds__(kWave)
 __attribute__((amdgpu_waves_per_eu(LM * sizeof(R) <= 256 ? 4 : 3)))
 void walk_kernel(WalkArgs a) {
@@ -175,11 +245,13 @@ void walk_kernel(WalkArgs a) {
   __shared__ V4 lm[LM][4];
   __shared__ V4 lp[kListP];
   __shared__ uint32_t lpi[kListP];
-  __shared__ uint32_t gsh;
+  __shared__ uint2 opened[kWave];   // {first child, child count | kinds << 8} of a step's opened nodes
 
   const int lane = threadIdx.x;
-  const R eps2 = (R)a.eps2;
+  constexpr bool kPair = sizeof(R) == 4 && NT == 1;
+  const R eps2 = (R)a.eps2, eps22 = (R)(2.0 * a.eps2);
   const double theta2 = a.theta2;
+  const double t_acc = theta2 * (1.0 - 1e-12), t_rej = theta2 * (1.0 + 1e-12);
   const uint32_t ngroups = SINK ? a.nsink_groups : a.sc->ngroups;
   const double* __restrict__ TX = SINK ? a.tx : a.x;
   const double* __restrict__ TY = SINK ? a.ty : a.y;
@@ -193,8 +265,8 @@ void walk_kernel(WalkArgs a) {
   const uint32_t nq = (uint32_t)a.nqueue;
   uint32_t q = blockIdx.x % nq, qleft = nq;   // lane 0's position in the queues
   for (;;) {
+    uint32_t gg = ngroups;
     if (lane == 0) {
-      uint32_t gg = ngroups;
       while (qleft) {
         const uint32_t lo = (uint32_t)((uint64_t)ngroups * q / nq);
         const uint32_t hi = (uint32_t)((uint64_t)ngroups * (q + 1) / nq);
@@ -203,104 +275,124 @@ void walk_kernel(WalkArgs a) {
         q = q + 1 == nq ? 0u : q + 1;
         --qleft;
       }
-      gsh = gg;
     }
-    __syncthreads();
-    const uint32_t g = gsh;
-    __syncthreads();
+    const uint32_t g = uniform(gg);
     if (g >= ngroups) break;
 
-    // Lanes s*cnt .. s*cnt+cnt-1 form slice s (s < S = 64/cnt) and hold the
-    // group's targets in order; the 64 - S*cnt remaining lanes hold copies
-    // of targets for the box and take no part in the sums.
+    // Every lane holds NT of the group's T targets, u and (NT = 2) u + W with
+    // W = ceil(T / NT), and lanes s*W .. s*W+W-1 form slice s (s < S = 64/W).
+    // A lane without a second target repeats its first; the 64 - S*W lanes
+    // past the slices repeat the last slice's entries; both are left out of
+    // the sums.
     uint32_t a0, cnt;
-    if (!SINK || a.gfirst) { a0 = a.gfirst[g]; cnt = a.gcount[g]; }
+    if (!SINK || a.gfirst) { a0 = uniform(a.gfirst[g]); cnt = uniform(a.gcount[g]); }
     else { a0 = g; cnt = 1u; }
     const uint32_t T = cnt;
-    const uint32_t S = kWave / T;
-    const uint32_t s = (uint32_t)lane / T;
-    const uint32_t t = (uint32_t)lane - s * T;
-    const bool valid = s < S;
-    const uint32_t tid = a0 + t;
-    const double xt = TX[tid], yt = TY[tid], zt = TZ[tid];
-    const double ox = TX[a0], oy = TY[a0], oz = TZ[a0];
-    const double lox = wave_min(xt), loy = wave_min(yt), loz = wave_min(zt);
-    const double hix = wave_max(xt), hiy = wave_max(yt), hiz = wave_max(zt);
-    // target position in the kernel's frame (FP64: set per box below)
-    R tx = R(0), ty = R(0), tz = R(0);
-    if constexpr (sizeof(R) == 4) {
-      tx = (R)(xt - ox); ty = (R)(yt - oy); tz = (R)(zt - oz);
+    const uint32_t W = (T + (uint32_t)NT - 1u) / (uint32_t)NT;
+    const bool two = NT == 2 && T > 1u;
+    const uint32_t S = uniform(kWave / W);
+    const uint32_t divS = uniform((4096u + S - 1u) / S);   // r / S = (r * divS) >> 12 for r < 64
+    const uint32_t s = (uint32_t)lane / W;
+    const uint32_t u = (uint32_t)lane - s * W;
+    const uint32_t se = s < S ? s : S - 1u;   // the slice whose entries this lane evaluates
+    bool has1 = false;
+    uint32_t tid[NT];
+    double xt[NT], yt[NT], zt[NT];
+    tid[0] = a0 + u;
+    if constexpr (NT == 2) { has1 = u + W < T; tid[1] = has1 ? tid[0] + W : tid[0]; }
+#pragma unroll
+    for (int j = 0; j < NT; ++j) { xt[j] = TX[tid[j]]; yt[j] = TY[tid[j]]; zt[j] = TZ[tid[j]]; }
+    const double ox = uniform(xt[0]), oy = uniform(yt[0]), oz = uniform(zt[0]);   // lane 0: target a0
+    const double lox = uniform_min(fmin(xt[0], xt[NT - 1])), loy = uniform_min(fmin(yt[0], yt[NT - 1])),
+                 loz = uniform_min(fmin(zt[0], zt[NT - 1]));
+    const double hix = -uniform_min(-fmax(xt[0], xt[NT - 1])), hiy = -uniform_min(-fmax(yt[0], yt[NT - 1])),
+                 hiz = -uniform_min(-fmax(zt[0], zt[NT - 1]));
+    // target positions in the kernel's frame (FP64: set per box below)
+    R tx[NT], ty[NT], tz[NT];
+    Acc<R> acc[NT];
+    double sx[NT], sy[NT], sz[NT];    // targets of the current box: x - vbox
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+      tx[j] = (R)(xt[j] - ox); ty[j] = (R)(yt[j] - oy); tz[j] = (R)(zt[j] - oz);
+      sx[j] = xt[j]; sy[j] = yt[j]; sz[j] = zt[j];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) { acc[j].s[k] = 0.0; acc[j].p[k] = R(0); }
     }
 
-    Acc<R> acc;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) { acc.s[k] = R(0); acc.c[k] = R(0); acc.p[k] = R(0); }
-
+    // Kept remainders (fewer than S entries) shorten the next steps' lists;
+    // above 16 slices, where a list is a few passes at most, lists are emptied.
+    const bool keep_rest = S <= 16u;
+    const bool dipoles = uniform(a.boxes[(!SINK && a.sys) ? a.sys[a0] : 0u].qsign) == 3u;
     uint32_t sp = 0, nm = 0, np = 0, cnt_p2p = 0, cnt_m2p = 0, namb = 0, nsteps = 0;
     uint32_t mac_lane = 0;   // this lane's MAC evaluations, summed over the wave at the end
     bool overflow = false;
-    const uint32_t root = (!SINK && a.sys) ? a.sysroot[a.sys[a0]] : 0u;   // the group's own root
-    double sx = xt, sy = yt, sz = zt;    // targets of the current box: x - vbox
+    const uint32_t root = (!SINK && a.sys) ? uniform(a.sysroot[a.sys[a0]]) : 0u;   // the group's own root
 
-    // Batches: entry k goes to slice k mod S; the loop count is uniform.
-    // FP32: two entries per pass (their LDS reads issued together), then the
-    // tail; FP64 keeps one entry per pass (register pressure).
-    auto flush_m2p = [&]() {
-      uint32_t kk = 0;
-      constexpr bool kPair = sizeof(R) == 4;
-      const uint32_t n2 = (kPair && nm >= 2 * S) ? nm - 2 * S + 1 : 0;
-      if (kPair && valid) {
-        for (; kk < n2; kk += 2 * S) {
-          const uint32_t k = kk + s, k2 = k + S;
+    // Batches: entry k goes to slice k mod S; the passes in which every slice
+    // has an entry run without a mask, the last one with it.
+    auto m2p_pair = [&](auto dip, const V4& e0, const V4& e1, const V4& e2, const V4& e3) __attribute__((always_inline)) {
+      constexpr bool D = decltype(dip)::value;
+      m2p<R, D>(tx[0] - e0.x, ty[0] - e0.y, tz[0] - e0.z, e0.w, e1, e2, e3.x, e3.y, eps2, acc[0].p);
+      if constexpr (NT == 2)
+        if (two)
+          m2p<R, D>(tx[1] - e0.x, ty[1] - e0.y, tz[1] - e0.z, e0.w, e1, e2, e3.x, e3.y, eps2,
+                    acc[1].p);
+    };
+    auto m2p_entry = [&](auto dip, uint32_t k) __attribute__((always_inline)) {
+      const V4 e0 = lm[k][0], e1 = lm[k][1], e2 = lm[k][2], e3 = lm[k][3];
+      m2p_pair(dip, e0, e1, e2, e3);
+    };
+    auto m2p_list = [&](auto dip, uint32_t r) __attribute__((always_inline)) {
+      uint32_t k = r + se, kk = r + S;
+      if constexpr (kPair) {
+        for (; kk + S <= nm; kk += 2 * S, k += 2 * S) {
           const V4 e0 = lm[k][0], e1 = lm[k][1], e2 = lm[k][2], e3 = lm[k][3];
+          const uint32_t k2 = k + S;
           const V4 f0 = lm[k2][0], f1 = lm[k2][1], f2 = lm[k2][2], f3 = lm[k2][3];
-          m2p<R>(tx - (R)e0.x, ty - (R)e0.y, tz - (R)e0.z, e1, e2, e3, (R)e0.w, eps2, acc.p);
-          m2p<R>(tx - (R)f0.x, ty - (R)f0.y, tz - (R)f0.z, f1, f2, f3, (R)f0.w, eps2, acc.p);
+          m2p_pair(dip, e0, e1, e2, e3);
+          m2p_pair(dip, f0, f1, f2, f3);
         }
       }
-      kk = n2 ? ((n2 - 1) / (2 * S) + 1) * 2 * S : 0;
-      for (; kk < nm; kk += S) {
-        const uint32_t k = kk + s;
-        if (valid && k < nm) {
-          const V4 e0 = lm[k][0], e1 = lm[k][1], e2 = lm[k][2], e3 = lm[k][3];
-          m2p<R>(tx - (R)e0.x, ty - (R)e0.y, tz - (R)e0.z, e1, e2, e3, (R)e0.w, eps2, acc.p);
-        }
-      }
-      fold(acc);
+      for (; kk <= nm; kk += S, k += S) m2p_entry(dip, k);
+      if (k < nm) m2p_entry(dip, k);
+    };
+    auto fold_all = [&]() __attribute__((always_inline)) {
+#pragma unroll
+      for (int j = 0; j < NT; ++j) fold(acc[j]);
+    };
+    // Leaves the first nm mod S entries in the list when they still leave
+    // room for `more` (so every pass is a full one), else empties it.
+    auto flush_m2p = [&](uint32_t more) __attribute__((always_inline)) {
+      const uint32_t rest = nm - ((nm * divS) >> 12) * S;
+      const uint32_t r = keep_rest && rest + more <= (uint32_t)LM ? rest : 0u;
+      if (dipoles) m2p_list(std::true_type{}, r);
+      else m2p_list(std::false_type{}, r);
+      fold_all();
+      nm = r;
     };
     // self term: the reference's rule (a zero separation from the leaf's
     // particle) for sinks, the particle index for the grown particles
-    auto p2p_self = [&](uint32_t k) -> bool {
-      if constexpr (SINK) {
-        const uint32_t j = lpi[k];
-        return sx == a.x[j] && sy == a.y[j] && sz == a.z[j];
-      } else {
-        return lpi[k] == tid;   // mirror-box entries hold ~0u
+    auto p2p_entry = [&](uint32_t k) __attribute__((always_inline)) {
+      const V4 e = lp[k];
+      const uint32_t i = lpi[k];   // mirror-box entries hold ~0u
+      bool self[NT];
+#pragma unroll
+      for (int j = 0; j < NT; ++j) {
+        if constexpr (SINK) self[j] = sx[j] == a.x[i] && sy[j] == a.y[i] && sz[j] == a.z[i];
+        else self[j] = i == tid[j];
       }
+      p2p<R>(tx[0] - e.x, ty[0] - e.y, tz[0] - e.z, e.w, eps2, self[0], acc[0].p);
+      if constexpr (NT == 2)
+        if (two) p2p<R>(tx[1] - e.x, ty[1] - e.y, tz[1] - e.z, e.w, eps2, self[1], acc[1].p);
     };
-    // FP32: two entries per pass as for M2P (same per-lane order of terms)
-    auto flush_p2p = [&]() {
-      uint32_t kk = 0;
-      constexpr bool kPair = sizeof(R) == 4;
-      const uint32_t n2 = (kPair && np >= 2 * S) ? np - 2 * S + 1 : 0;
-      if (kPair && valid) {
-        for (; kk < n2; kk += 2 * S) {
-          const uint32_t k = kk + s, k2 = k + S;
-          const V4 e = lp[k], f = lp[k2];
-          const bool self1 = p2p_self(k), self2 = p2p_self(k2);
-          p2p<R>(tx - (R)e.x, ty - (R)e.y, tz - (R)e.z, (R)e.w, eps2, self1, acc.p);
-          p2p<R>(tx - (R)f.x, ty - (R)f.y, tz - (R)f.z, (R)f.w, eps2, self2, acc.p);
-        }
-      }
-      kk = n2 ? ((n2 - 1) / (2 * S) + 1) * 2 * S : 0;
-      for (; kk < np; kk += S) {
-        const uint32_t k = kk + s;
-        if (valid && k < np) {
-          const V4 e = lp[k];
-          p2p<R>(tx - (R)e.x, ty - (R)e.y, tz - (R)e.z, (R)e.w, eps2, p2p_self(k), acc.p);
-        }
-      }
-      fold(acc);
+    auto flush_p2p = [&](uint32_t more) __attribute__((always_inline)) {
+      const uint32_t rest = np - ((np * divS) >> 12) * S;
+      const uint32_t r = keep_rest && rest + more <= (uint32_t)kListP ? rest : 0u;
+      uint32_t k = r + se, kk = r + S;
+      for (; kk <= np; kk += S, k += S) p2p_entry(k);
+      if (k < np) p2p_entry(k);
+      fold_all();
+      np = r;
     };
 
     const int nbox = PER ? a.nbox : 1;
@@ -310,14 +402,21 @@ void walk_kernel(WalkArgs a) {
     const bool central = !PER || (vx == 0.0 && vy == 0.0 && vz == 0.0);
     // targets of this box: x - vbox; group box likewise (rounding is monotone,
     // so the shifted extremes are the extremes of the shifted targets)
-    sx = xt - vx; sy = yt - vy; sz = zt - vz;
-    const double blox = lox - vx, bloy = loy - vy, bloz = loz - vz;
-    const double bhix = hix - vx, bhiy = hiy - vy, bhiz = hiz - vz;
-    const double fox = ox - vx, foy = oy - vy, foz = oz - vz;   // FP32 node frame
-    if constexpr (sizeof(R) == 8) { tx = sx; ty = sy; tz = sz; }
+    if constexpr (PER) {
+#pragma unroll
+      for (int j = 0; j < NT; ++j) { sx[j] = xt[j] - vx; sy[j] = yt[j] - vy; sz[j] = zt[j] - vz; }
+    }
+    const Span bx = span_of(lox - vx, hix - vx), by = span_of(loy - vy, hiy - vy),
+               bz = span_of(loz - vz, hiz - vz);
+    const double fox = PER ? uniform(ox - vx) : ox, foy = PER ? uniform(oy - vy) : oy,
+                 foz = PER ? uniform(oz - vz) : oz;   // FP32 node frame
+    if constexpr (sizeof(R) == 8) {
+#pragma unroll
+      for (int j = 0; j < NT; ++j) { tx[j] = sx[j]; ty[j] = sy[j]; tz[j] = sz[j]; }
+    }
     if (lane == 0) stack[0] = root | kTwigBit;
     sp = 1;
-    __syncthreads();
+    wave_order();
     while (sp > 0) {
       // Up to min(64, LM) nodes are read from the top of the stack (so one
       // step's appends always fit an emptied list, positions nm + rank < LM);
@@ -326,13 +425,16 @@ void walk_kernel(WalkArgs a) {
       constexpr uint32_t kPop = (uint32_t)(LM < kWave ? LM : kWave);
       static_assert(kListP >= kWave, "P2P list must hold one full step");
       const uint32_t m = sp < kPop ? sp : kPop;
-      if (nm + m > (uint32_t)LM) { __syncthreads(); flush_m2p(); nm = 0; }
-      if (np + m > (uint32_t)kListP) { __syncthreads(); flush_p2p(); np = 0; }
       const bool has = (uint32_t)lane < m;
       const uint32_t entry = has ? stack[sp - 1 - lane] : 0u;
       const uint32_t node = entry & ~kTwigBit;
       const bool twig_entry = (entry & kTwigBit) != 0u;
-      __syncthreads();
+      // at most one append per twig and one per leaf (a root counts as a twig
+      // and may be a leaf)
+      const uint32_t nt = (uint32_t)popc64(__ballot(twig_entry)), nl = m - nt + 1u;
+      if (nm + nt > (uint32_t)LM) flush_m2p(nt);
+      if (np + nl > (uint32_t)kListP) flush_p2p(nl);
+      wave_order();
       ++nsteps;
 
       // All of a node's data is requested at once, before any decision, so a
@@ -340,7 +442,7 @@ void walk_kernel(WalkArgs a) {
       // its walk moments and its children's kinds; a leaf has neither.
       NodeGeom gm = {0.0, 0.0, 0.0, 0.0};
       NodeLink lk = {0u, 0u, 0u, 0u};
-      V4 w0, w1, w2;
+      V4 w0 = {}, w1 = {}, w2 = {};
       uint32_t kids = 0u;
       if (has) {
         gm = a.geom[node];
@@ -353,21 +455,22 @@ void walk_kernel(WalkArgs a) {
         else src = reinterpret_cast<const V4*>(&a.wm64[node]);
         w0 = src[0]; w1 = src[1]; w2 = src[2];
       }
-      // Decide from the group's bounding box when possible (margins cover
-      // every rounding of the exact per-target test below).
+      // Decide from the group's bounding box when possible.  The margins
+      // cover every rounding here and in the exact per-target test below: a
+      // distance to the box is either at least the half width, and then has
+      // a relative error of a few ulps, or its error is below the part that
+      // was added to the half width.
       bool acc_ok = false, rej = false;
       uint32_t macc = 0;
       if (has && lk.nchild != 0u) {
-        const double ex = fmax(fmax(blox - gm.cx, gm.cx - bhix), 0.0);
-        const double ey = fmax(fmax(bloy - gm.cy, gm.cy - bhiy), 0.0);
-        const double ez = fmax(fmax(bloz - gm.cz, gm.cz - bhiz), 0.0);
-        const double fx = fmax(fabs(gm.cx - blox), fabs(gm.cx - bhix));
-        const double fy = fmax(fabs(gm.cy - bloy), fabs(gm.cy - bhiy));
-        const double fz = fmax(fabs(gm.cz - bloz), fabs(gm.cz - bhiz));
+#pragma clang fp contract(fast)
+        const double dx = fabs(gm.cx - bx.c), dy = fabs(gm.cy - by.c), dz = fabs(gm.cz - bz.c);
+        const double ex = fmax(dx - bx.h, 0.0), ey = fmax(dy - by.h, 0.0), ez = fmax(dz - bz.h, 0.0);
+        const double fx = dx + bx.h, fy = dy + by.h, fz = dz + bz.h;
         const double dmin2 = ex * ex + ey * ey + ez * ez;
         const double dmax2 = fx * fx + fy * fy + fz * fz;
-        acc_ok = (theta2 * dmin2) * (1.0 - 1e-12) > gm.b2;
-        rej = !acc_ok && (theta2 * dmax2) * (1.0 + 1e-12) <= gm.b2;
+        acc_ok = t_acc * dmin2 > gm.b2;
+        rej = !acc_ok && t_rej * dmax2 <= gm.b2;
         macc = acc_ok ? cnt : (rej ? 1u : 0u);
       }
       // Visit lanes 0 .. k-1 for the largest k whose step leaves at most kCap
@@ -397,39 +500,60 @@ void walk_kernel(WalkArgs a) {
       // nodes are settled per pass.  The nodes' centres and b^2 are staged in
       // the free tail of the M2P list (entries nm .. nm + m - 1, which this
       // step's appends overwrite only after the tests), so each slice reads
-      // its node with one broadcast load per pass.
+      // its node with one broadcast load per pass.  Pass p's failure ballots
+      // are kept in lane p; afterwards each undecided node's lane fetches the
+      // ballots of its pass and cuts out its slice.
       const bool amb_me = twig && !acc_ok && !rej;
       const unsigned long long amb = __ballot(amb_me);
-      const uint32_t na = (uint32_t)popc64(amb);
-      namb += na;
-      if (na) {
+      if (amb) {
+        const uint32_t na = (uint32_t)popc64(amb);
+        namb += na;
         const uint32_t my_rank = mask_rank(amb);
         if (amb_me) {
           double2* st = reinterpret_cast<double2*>(&lm[nm + my_rank][0]);
           st[0] = make_double2(gm.cx, gm.cy);
           st[1] = make_double2(gm.cz, gm.b2);
         }
-        __syncthreads();
-        for (uint32_t base = 0; base < na; base += S) {
-          const uint32_t r = base + s;
-          const bool active = valid && r < na;
-          double2 c0 = make_double2(0.0, 0.0), c1 = c0;
-          if (active) {
-            const double2* st = reinterpret_cast<const double2*>(&lm[nm + r][0]);
-            c0 = st[0];
-            c1 = st[1];
-          }
-          const bool fail = active && mac_fails(sx, sy, sz, c0.x, c0.y, c1.x, c1.y, theta2);
-          const unsigned long long ball = __ballot(fail);
-          if (amb_me && my_rank >= base && my_rank < base + S) {
-            const uint32_t rr = my_rank - base;
-            const unsigned long long fm =
-                (ball >> (rr * T)) & (T == 64 ? ~0ull : ((1ull << T) - 1ull));
-            if (fm == 0ull) { acc_ok = true; macc = cnt; }
-            else { rej = true; macc = (uint32_t)__ffsll((long long)fm); }
+        wave_order();
+        int blo[NT], bhi[NT];
+#pragma unroll
+        for (int j = 0; j < NT; ++j) { blo[j] = 0; bhi[j] = 0; }
+        uint32_t pass = 0;
+        for (uint32_t base = 0; base < na; base += S, ++pass) {
+          // slices past the last node repeat it
+          const uint32_t r = base + s < na ? base + s : na - 1u;
+          const double2* st = reinterpret_cast<const double2*>(&lm[nm + r][0]);
+          const double2 c0 = st[0], c1 = st[1];
+#pragma unroll
+          for (int j = 0; j < NT; ++j) {
+            const bool f = mac_fails(sx[j], sy[j], sz[j], c0.x, c0.y, c1.x, c1.y, theta2);
+            const unsigned long long ball = __ballot(f);
+            blo[j] = (uint32_t)lane == pass ? (int)(uint32_t)ball : blo[j];
+            bhi[j] = (uint32_t)lane == pass ? (int)(uint32_t)(ball >> 32) : bhi[j];
           }
         }
-        __syncthreads();
+        const uint32_t mp = (my_rank * divS) >> 12;
+        const uint32_t sh = (my_rank - mp * S) * W;
+        unsigned long long f[NT];
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+          const uint32_t lo = (uint32_t)__builtin_amdgcn_ds_bpermute((int)(mp << 2), blo[j]);
+          const uint32_t hi = (uint32_t)__builtin_amdgcn_ds_bpermute((int)(mp << 2), bhi[j]);
+          // the node's W bits at the top, the others shifted out
+          f[j] = ((((unsigned long long)hi << 32) | lo) >> sh) << (64u - W);
+        }
+        if (amb_me) {
+          bool any = f[0] != 0ull;
+          if constexpr (NT == 2) any = any || f[1] != 0ull;
+          if (!any) { acc_ok = true; macc = cnt; }
+          else {   // the first failing target, in order
+            rej = true;
+            uint32_t first = (uint32_t)__ffsll((long long)f[0]);
+            if constexpr (NT == 2) first = f[0] ? first : W + (uint32_t)__ffsll((long long)f[1]);
+            macc = first - (64u - W);
+          }
+        }
+        wave_order();
       }
       mac_lane += twig ? macc : 0u;
 
@@ -438,27 +562,23 @@ void walk_kernel(WalkArgs a) {
       const unsigned long long pm = __ballot(leaf);
       if (take_m) {
         const uint32_t pos = nm + mask_rank(am);
+        // w0 = {Bxx,Byy,Bzz,Bxy}, w1 = {Byz,Bzx,tr,px}, w2 = {py,pz,q,-}
         V4 e0;
         if constexpr (sizeof(R) == 4)
-          e0 = make_float4((float)(gm.cx - fox), (float)(gm.cy - foy), (float)(gm.cz - foz), 0.0f);
+          e0 = V4{(float)(gm.cx - fox), (float)(gm.cy - foy), (float)(gm.cz - foz), w2.z};
         else
-          e0 = make_double4(gm.cx, gm.cy, gm.cz, 0.0);
-        // w0 = {q, px, py, pz}, w1 = {2qx, 2qy, 2qz, xy}, w2 = {yz, zx, tr, -}
-        e0.w = w0.x;
-        V4 e1, e2, e3;
-        e1.x = w0.y; e1.y = w0.z; e1.z = w0.w; e1.w = w1.x;
-        e2.x = w1.y; e2.y = w1.z; e2.z = w1.w; e2.w = w2.x;
-        e3.x = w2.y; e3.y = w2.z; e3.z = 0; e3.w = 0;
-        lm[pos][0] = e0; lm[pos][1] = e1; lm[pos][2] = e2; lm[pos][3] = e3;
+          e0 = V4{gm.cx, gm.cy, gm.cz, w2.z};
+        V4 e2 = w1;
+        e2.z *= eps22;
+        lm[pos][0] = e0; lm[pos][1] = w0; lm[pos][2] = e2; lm[pos][3] = w2;
       }
       if (leaf) {
         const uint32_t pos = np + mask_rank(pm);
         V4 e;
         if constexpr (sizeof(R) == 4) {
-          e = make_float4((float)(gm.cx - fox), (float)(gm.cy - foy), (float)(gm.cz - foz),
-                          (float)gm.b2);
+          e = V4{(float)(gm.cx - fox), (float)(gm.cy - foy), (float)(gm.cz - foz), (float)gm.b2};
         } else {
-          e = make_double4(gm.cx, gm.cy, gm.cz, gm.b2);
+          e = V4{gm.cx, gm.cy, gm.cz, gm.b2};
         }
         lp[pos] = e;
         lpi[pos] = (SINK || central) ? lk.first : ~0u;
@@ -466,46 +586,73 @@ void walk_kernel(WalkArgs a) {
       const uint32_t nma = (uint32_t)popc64(am), npa = (uint32_t)popc64(pm);
       nm += nma; np += npa; cnt_m2p += nma; cnt_p2p += npa;
 
-      const uint32_t nc = (twig && !acc_ok) ? lk.nchild : 0u;   // at most 8
-      uint32_t tot;
-      const uint32_t excl = wave_exclusive_scan16(nc, &tot);
-      if (sp + tot > (uint32_t)(kCap + kStackSlack)) { overflow = true; break; }
-      for (uint32_t k = 0; k < nc; ++k)
-        stack[sp + excl + k] = (lk.first + k) | (((kids >> k) & 1u) ? kTwigBit : 0u);
-      sp += tot;
-      __syncthreads();
+      // Children of the opened nodes, eight lanes per node: the nodes' child
+      // runs are compacted in LDS, lane 8 j + c takes child c of the j-th,
+      // and one ballot gives every child its place on the stack.
+      const bool open = twig && !acc_ok;
+      const unsigned long long om = __ballot(open);
+      if (open) opened[mask_rank(om)] = make_uint2(lk.first, lk.nchild | (kids << 8));
+      wave_order();
+      const int no = (int)popc64(om);
+      for (int o = 0; o < no; o += 8) {
+        const int j = o + (lane >> 3);
+        const uint32_t c = (uint32_t)lane & 7u;
+        const uint2 rec = opened[j & (kWave - 1)];
+        const bool child = j < no && c < (rec.y & 0xFFu);
+        const unsigned long long cm = __ballot(child);
+        const uint32_t nc = (uint32_t)popc64(cm);
+        if (sp + nc > (uint32_t)(kCap + kStackSlack)) { overflow = true; break; }
+        if (child)
+          stack[sp + mask_rank(cm)] = (rec.x + c) | (((rec.y >> (8u + c)) & 1u) << 31);
+        sp += nc;
+      }
+      if (overflow) break;
+      wave_order();
     }
     if constexpr (PER && (sizeof(R) == 8 || SINK)) {   // next box shifts the targets
-      __syncthreads();
-      if (nm) flush_m2p();
-      if (np) flush_p2p();
-      nm = 0; np = 0;
+      if (nm) flush_m2p(LM + 1u);
+      if (np) flush_p2p(kListP + 1u);
+      wave_order();
     }
     }   // boxes
-    __syncthreads();
-    if (nm) flush_m2p();
-    if (np) flush_p2p();
+    if (nm) flush_m2p(LM + 1u);
+    if (np) flush_p2p(kListP + 1u);
+    wave_order();
 
-    // combine slices (target t lives in lanes t, t+T, t+2T, ...) in FP64
-    double out[4];
+    // combine the slices in FP64, halving their number per step (slice s adds
+    // slice s + ceil(n/2)): a fixed order
+    for (uint32_t rem = S; rem > 1;) {
+      const uint32_t h = (rem + 1u) >> 1;
+      const int src = (lane + (int)(h * W)) & (kWave - 1);
+      const bool add = s + h < rem;
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const double v0 = (double)acc.s[k] - (double)acc.c[k];
-      double v = v0;
-      for (uint32_t o = 1; o < S; ++o) v += __shfl(v0, (int)(t + o * T));
-      out[k] = v * a.sign;
+      for (int j = 0; j < NT; ++j) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const double v = __shfl(acc[j].s[k], src);
+          acc[j].s[k] += add ? v : 0.0;
+        }
+      }
+      rem = h;
     }
     if (overflow) {
       if (lane == 0) atomicOr(&a.sc->flags, kFlagStackOverflow);
     }
-    if (s == 0 && valid) {
-      a.ex[tid] = out[0];
-      a.ey[tid] = out[1];
-      a.ez[tid] = out[2];
-      a.pot[tid] = out[3];
-      a.work[tid] = (SINK ? 0.0 : 1.0) + (double)(cnt_p2p + cnt_m2p);
-      a.np2p[tid] = cnt_p2p;
-      a.nm2p[tid] = cnt_m2p;
+    const double wk = (SINK ? 0.0 : 1.0) + (double)(cnt_p2p + cnt_m2p);
+    if (s == 0) {
+#pragma unroll
+      for (int j = 0; j < NT; ++j) {
+        if (j == 0 || has1) {
+          const uint32_t t = tid[j];
+          a.ex[t] = acc[j].s[0] * a.sign;
+          a.ey[t] = acc[j].s[1] * a.sign;
+          a.ez[t] = acc[j].s[2] * a.sign;
+          a.pot[t] = acc[j].s[3] * a.sign;
+          a.work[t] = wk;
+          a.np2p[t] = cnt_p2p;
+          a.nm2p[t] = cnt_m2p;
+        }
+      }
     }
     const unsigned long long nmac = SINK ? 0ull : wave_sum((unsigned long long)mac_lane);
     if (!SINK && lane == 0) {   // per-group record, summed by walk_stats_kernel
@@ -513,7 +660,6 @@ void walk_kernel(WalkArgs a) {
       gs[0] = make_uint4((uint32_t)nmac, cnt_p2p, cnt_m2p, namb);
       gs[1] = make_uint4(nsteps, cnt, 0u, 0u);
     }
-    __syncthreads();
   }
 }
 
@@ -642,7 +788,8 @@ __global__ __launch_bounds__(256) void direct_kernel(int64_t n, const double* __
 
 }  // namespace
 
-// Persistent grid: every wavefront the device can hold for this instance.
+// Persistent grid: every wavefront the device can hold for this instance
+// (both targets-per-lane forms have the same LDS and register budget).
 int walk_default_blocks(int precision, int list_tile) {
   int dev = 0, cus = 256;
   if (hipGetDevice(&dev) == hipSuccess) {
@@ -653,12 +800,12 @@ int walk_default_blocks(int precision, int list_tile) {
   hipError_t e;
   if (precision == kWalkFP64)
     e = list_tile == 64
-            ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, walk_kernel<double, 64, false, false>, kWave, 0)
-            : hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, walk_kernel<double, 32, false, false>, kWave, 0);
+            ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, walk_kernel<double, 64, 1, false, false>, kWave, 0)
+            : hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, walk_kernel<double, 32, 1, false, false>, kWave, 0);
   else
     e = list_tile == 128
-            ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, walk_kernel<float, 128, false, false>, kWave, 0)
-            : hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, walk_kernel<float, 64, false, false>, kWave, 0);
+            ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, walk_kernel<float, 128, 1, false, false>, kWave, 0)
+            : hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, walk_kernel<float, 64, 1, false, false>, kWave, 0);
   if (e != hipSuccess || per < 1) per = 8;
   return cus * per;
 }
@@ -675,32 +822,38 @@ bool walk_list_tile_ok(int precision, int list_tile) {
                                 : (list_tile == 64 || list_tile == 128);
 }
 
+// default list tile (0): the smaller of each precision, whose lower LDS use
+// lets one more wavefront per SIMD resident (measured faster on MI355X)
 template <bool PER, bool SINK>
 static void launch_walk_t(hipStream_t s, const WalkArgs& a, int precision, int blocks,
-                          int list_tile) {
-  // default (0): the smaller tile of each precision, whose lower LDS use
-  // lets one more wavefront per SIMD resident (measured faster on MI355X)
+                          int list_tile, int max_group) {
   if (precision == kWalkFP64) {
     if (list_tile == 64)
-      walk_kernel<double, 64, PER, SINK><<<blocks, kWave, 0, s>>>(a);
+      walk_kernel<double, 64, 1, PER, SINK><<<blocks, kWave, 0, s>>>(a);
     else
-      walk_kernel<double, 32, PER, SINK><<<blocks, kWave, 0, s>>>(a);
+      walk_kernel<double, 32, 1, PER, SINK><<<blocks, kWave, 0, s>>>(a);
+  } else if (max_group > 16) {   // two targets per lane, see walk_kernel
+    if (list_tile == 128)
+      walk_kernel<float, 128, 2, PER, SINK><<<blocks, kWave, 0, s>>>(a);
+    else
+      walk_kernel<float, 64, 2, PER, SINK><<<blocks, kWave, 0, s>>>(a);
   } else {
     if (list_tile == 128)
-      walk_kernel<float, 128, PER, SINK><<<blocks, kWave, 0, s>>>(a);
+      walk_kernel<float, 128, 1, PER, SINK><<<blocks, kWave, 0, s>>>(a);
     else
-      walk_kernel<float, 64, PER, SINK><<<blocks, kWave, 0, s>>>(a);
+      walk_kernel<float, 64, 1, PER, SINK><<<blocks, kWave, 0, s>>>(a);
   }
 }
 
-void launch_walk(hipStream_t s, const WalkArgs& a, int precision, int blocks, int list_tile) {
+void launch_walk(hipStream_t s, const WalkArgs& a, int precision, int blocks, int list_tile,
+                 int max_group) {
   const bool sink = a.tx != nullptr;
   if (a.nbox > 1)
-    sink ? launch_walk_t<true, true>(s, a, precision, blocks, list_tile)
-         : launch_walk_t<true, false>(s, a, precision, blocks, list_tile);
+    sink ? launch_walk_t<true, true>(s, a, precision, blocks, list_tile, max_group)
+         : launch_walk_t<true, false>(s, a, precision, blocks, list_tile, max_group);
   else
-    sink ? launch_walk_t<false, true>(s, a, precision, blocks, list_tile)
-         : launch_walk_t<false, false>(s, a, precision, blocks, list_tile);
+    sink ? launch_walk_t<false, true>(s, a, precision, blocks, list_tile, max_group)
+         : launch_walk_t<false, false>(s, a, precision, blocks, list_tile, max_group);
 }
 
 void launch_walk_stats(hipStream_t s, const WalkArgs& a) {
