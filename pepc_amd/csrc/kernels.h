@@ -307,10 +307,18 @@ struct ReplayArgs {
 void launch_replay(hipStream_t s, const ReplayArgs& a, int blocks);
 
 // walk.hip: FP64 direct sum
-// nbox mirror-box vectors vbox (nullptr: open boundaries).
+// How ntest targets against n sources are split: `span` targets per block in
+// 256/span slices, `ranges` ranges of `range` sources.
+struct DirectPlan {
+  int span;
+  int64_t tblocks, ranges, range, partials;
+};
+DirectPlan direct_plan(int64_t n, int64_t ntest);
+// nbox mirror-box vectors vbox (nullptr: open boundaries).  work: room for
+// 4 * ntest * direct_plan(n, ntest).partials doubles, or nullptr (slower).
 void launch_direct(hipStream_t s, int64_t n, const double* x, const double* y, const double* z,
                    const double* q, int64_t ntest, const int64_t* testidx, double eps2, double sign,
-                   double* ex, double* ey, double* ez, double* pot, int nbox = 1,
+                   double* ex, double* ey, double* ez, double* pot, double* work, int nbox = 1,
                    const double* vbox = nullptr);
 
 }  // namespace pepc

@@ -110,6 +110,9 @@ struct Ctx {
   int* lfpt = nullptr;              // merged fictitious-charge points (LatticeGeom::fpt)
   double* lfpos = nullptr;          // their positions and charges (LatticeGeom::fpos)
   double2* lom = nullptr;
+  // direct sum: partial sums
+  double* dwork = nullptr;
+  int64_t dwork_cap = 0;
   // sinks (traversal of other particles)
   int64_t scap = 0, sk_m = 0;
   int sk_mode = 0;
@@ -258,7 +261,7 @@ void free_all(Ctx* c) {
                   c->sk_res[0], c->sk_res[1], c->sk_res[2], c->sk_res[3], c->sk_res[4],
                   c->sk_io[0], c->sk_io[1], c->sk_io[2], c->sk_io[3], c->sk_io[4], c->sk_io[5],
                   c->sk_io[6], c->sk_io[7], c->sk_k0, c->sk_k1, c->sk_v0, c->sk_v1, c->sk_gfirst,
-                  c->sk_gcount, c->sk_p2p, c->sk_m2p, c->sk_hist, c->sk_bsum};
+                  c->sk_gcount, c->sk_p2p, c->sk_m2p, c->sk_hist, c->sk_bsum, c->dwork};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   for (double* p : c->st)
@@ -1095,6 +1098,33 @@ int pepc_gpu_read_walk(void* p, int64_t gcap, uint32_t* gfirst, uint32_t* gcount
   return 0;
 }
 
+// Partial sums of the split direct sum: kept by the context, at most about
+// 19 MB (256 targets x 2304 blocks x 4 sums) plus one sum per target.  nullptr
+// (the unsplit form) when there is no memory for them or when they would have
+// to be allocated on a stream under capture.
+static double* direct_workspace(Ctx* c, hipStream_t s, int64_t n, int64_t ntest) {
+  if (ntest <= 0) return nullptr;
+  const int64_t partials = direct_plan(n, ntest).partials;
+  if (partials == 1) return nullptr;
+  const int64_t need = 4 * ntest * partials;
+  if (need <= c->dwork_cap) return c->dwork;
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  // kernels of earlier calls may still use the smaller buffer: hipFree waits
+  if (c->dwork) (void)hipFree(c->dwork);
+  c->dwork_cap = 0;
+  if (hipMalloc((void**)&c->dwork, sizeof(double) * (size_t)need) != hipSuccess) {
+    (void)hipGetLastError();
+    c->dwork = nullptr;
+    return nullptr;
+  }
+  c->dwork_cap = need;
+  return c->dwork;
+}
+
 // directforce (src/utils/module_directsum.f90:34-172): with periodic
 // boundaries every source in every mirror box, self only in the central box
 // (:80-93), then the lattice far field at the targets from all sources
@@ -1104,11 +1134,13 @@ static void enqueue_direct(Ctx* c, hipStream_t s, int64_t n, const double* x, co
                            const double* z, const double* q, int64_t ntest, const int64_t* testidx,
                            double eps2, double sign, double* ex, double* ey, double* ez,
                            double* pot) {
+  double* work = direct_workspace(c, s, n, ntest);
   if (!c->periodic) {
-    launch_direct(s, n, x, y, z, q, ntest, testidx, eps2, sign, ex, ey, ez, pot);
+    launch_direct(s, n, x, y, z, q, ntest, testidx, eps2, sign, ex, ey, ez, pot, work);
     return;
   }
-  launch_direct(s, n, x, y, z, q, ntest, testidx, eps2, sign, ex, ey, ez, pot, c->nbox, c->vbox);
+  launch_direct(s, n, x, y, z, q, ntest, testidx, eps2, sign, ex, ey, ez, pot, work, c->nbox,
+                c->vbox);
   if (c->far_field && ntest > 0) {
     launch_lattice_sources(s, n, x, y, z, q, c->lgeom, c->ml, c->fact, c->lpart, c->ldpart, c->lom,
                            c->ldip, c->mu, c->fict, c->lcoef);
