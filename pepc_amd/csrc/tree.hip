@@ -17,8 +17,9 @@
 //
 // Upward pass (tree_node_update_from_children, :762-821, with
 // shift_multipoles_up, coulomb/module_interaction_specific.f90:84-140): one
-// launch per level, deepest first, FP64, the reference's operation order with
-// contraction off, so moments are bit-identical to the reference formula.
+// launch per level, deepest first (small trees: by tiles of particles), FP64,
+// the reference's operation order with contraction off, so moments are bit-identical to the
+// reference formula.
 //
 // Groups (walk tiles, module_tree_walk_simple.f90:135-212): the maximal key
 // cells holding at most G particles = children with count <= G of twigs with
@@ -208,16 +209,25 @@ __global__ void levels_kernel(int64_t n, const unsigned long long* __restrict__ 
 }
 
 // ---- BFS node numbering
-// Tiles of kBfsTile sorted particles; wave w of a tile owns the kBfsWave
-// consecutive particles from base + w kBfsWave and takes them 64 at a time,
+// Tiles of bfs_tile(n) sorted particles; wave w of a tile owns the w-th
+// quarter of them and takes them 64 at a time,
 // one per lane, so the nodes one pass writes for a level are consecutive.
 // tab[l * nb + b] counts the nodes of level l owned by tile b's particles,
 // tab[kLevels * nb + l * nb + b] the twigs among them; after the exclusive
 // scan (level-major) the entries are the BFS index of the tile's first node
 // of that level and the twig rank of its first twig there.
-constexpr int kBfsTile = 4096;
-constexpr int kBfsWaves = kT / kWave;           // 4
-constexpr int kBfsWave = kBfsTile / kBfsWaves;  // 1024 particles per wave
+// A tile is short because a wave takes its particles one pass after another:
+// with 4,096 per tile the count took 15 and the emit 41 to 48 us for any
+// system up to a million particles, with 512 they take 3 and 8 us at 32,768
+// particles, 6 and 26 at 1,048,576.  Above that the waves fill the chip, and
+// longer tiles keep the table that bfs_scan_kernel reads short (4,194,304
+// particles: scan 24 us with tiles of 512, 7 with 2,048).
+constexpr int kBfsTileSmall = 512, kBfsTileLarge = 2048;
+constexpr int64_t kBfsLarge = 1 << 20;
+constexpr int kBfsWaves = kT / kWave;           // 4, each a quarter of the tile
+__host__ __device__ constexpr int bfs_tile(int64_t n) {
+  return n <= kBfsLarge ? kBfsTileSmall : kBfsTileLarge;
+}
 constexpr int kLevels = kMaxLevel + 1;
 
 // The wave's node and twig counts per level over its particles: lane l
@@ -227,13 +237,14 @@ __device__ __forceinline__ void bfs_wave_counts(int64_t n, int64_t base,
                                                 const uint8_t* __restrict__ hi, uint32_t& cn,
                                                 uint32_t& ct) {
   const int lane = lane_id();
+  const int passes = bfs_tile(n) / (kBfsWaves * kWave);
   cn = 0;
   ct = 0;
-  for (int it = 0; it < kBfsWave / kWave; ++it) {
+  for (int it = 0; it < passes; ++it) {
     const int64_t a = base + (int64_t)it * kWave + lane;
     const bool valid = a < n;
     const int l0 = valid ? lo[a] : kLevels, l1 = valid ? hi[a] : -1;
-    const int lmin = (int)wave_min_u32((uint32_t)l0), lmax = (int)wave_max_i32(l1);
+    const int lmin = -wave_max_i32(-l0), lmax = wave_max_i32(l1);
     for (int l = lmin; l <= lmax; ++l) {
       const uint32_t c = (uint32_t)popc64(__ballot(l0 <= l && l <= l1));
       const uint32_t d = (uint32_t)popc64(__ballot(l0 <= l && l < l1));
@@ -250,7 +261,8 @@ __global__ __launch_bounds__(kT) void bfs_count_kernel(int64_t n, const uint8_t*
   __shared__ uint32_t wn[kBfsWaves][kLevels], wt[kBfsWaves][kLevels];
   const int w = threadIdx.x / kWave, lane = lane_id();
   uint32_t cn, ct;
-  bfs_wave_counts(n, (int64_t)blockIdx.x * kBfsTile + (int64_t)w * kBfsWave, lo, hi, cn, ct);
+  const int64_t per_wave = bfs_tile(n) / kBfsWaves;
+  bfs_wave_counts(n, ((int64_t)blockIdx.x * kBfsWaves + w) * per_wave, lo, hi, cn, ct);
   if (lane < kLevels) { wn[w][lane] = cn; wt[w][lane] = ct; }
   __syncthreads();
   if (threadIdx.x < kLevels) {
@@ -373,7 +385,8 @@ __global__ __launch_bounds__(kT) void bfs_emit_kernel(
   if (blockIdx.x == 0 && threadIdx.x == 0) fc_rank[sc->ntwig] = sc->nnodes;
   __shared__ uint32_t wn[kBfsWaves][kLevels], wt[kBfsWaves][kLevels];
   const int w = threadIdx.x / kWave, lane = lane_id();
-  const int64_t base = (int64_t)blockIdx.x * kBfsTile + (int64_t)w * kBfsWave;
+  const int64_t per_wave = bfs_tile(n) / kBfsWaves;
+  const int64_t base = ((int64_t)blockIdx.x * kBfsWaves + w) * per_wave;
   uint32_t rn, rt;   // lane l: next node index / twig rank of level l for this wave
   bfs_wave_counts(n, base, lo, hi, rn, rt);
   if (lane < kLevels) { wn[w][lane] = rn; wt[w][lane] = rt; }
@@ -383,13 +396,13 @@ __global__ __launch_bounds__(kT) void bfs_emit_kernel(
     rt = tab[(int64_t)(3 * kLevels + lane) * nb + blockIdx.x];
     for (int k = 0; k < w; ++k) { rn += wn[k][lane]; rt += wt[k][lane]; }
   }
-  for (int it = 0; it < kBfsWave / kWave; ++it) {
+  for (int it = 0; it < (int)(per_wave / kWave); ++it) {
     const int64_t a = base + (int64_t)it * kWave + lane;
     const bool valid = a < n;
     const int l0 = valid ? lo[a] : kLevels, l1 = valid ? hi[a] : -1;
     NodeGeom g = {0.0, 0.0, 0.0, 0.0};
     if (valid) { g.cx = x[a]; g.cy = y[a]; g.cz = z[a]; g.b2 = q[a]; }
-    const int lmin = (int)wave_min_u32((uint32_t)l0), lmax = (int)wave_max_i32(l1);
+    const int lmin = -wave_max_i32(-l0), lmax = wave_max_i32(l1);
     uint32_t child = 0;
     for (int l = lmax; l >= lmin; --l) {
       const bool own = l0 <= l && l <= l1;
@@ -591,6 +604,277 @@ __device__ void twig_moments(int64_t i, uint32_t c0, uint32_t nc, int level, con
   write_walk_forms(i, m, walk_b2(m, b2, u.mac_select), u.prec, u.geom, u.wm32, u.wm64);
 }
 
+// ---- small trees: four lanes per twig, by tiles of particles
+// One wave issues an instruction every eight clocks whatever its lanes do,
+// and thread-per-twig code is about 1,400 instructions long, so a level costs
+// 4 to 5 us however few twigs it has.  Four lanes per twig cut that to a
+// third: lanes 0 to 2 form the components x, y, z (every formula is cyclic in
+// them: lane a takes the centre, dipole and quadrupole component a and the
+// off-diagonal ab with b = a + 1 mod 3), each in the reference's order of
+// operations; the children's distances are rooted two per lane.
+template <int kCtrl>
+__device__ __forceinline__ double quad_move(double v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), kCtrl, 0xF, 0xF, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), kCtrl, 0xF, 0xF, false);
+  return __hiloint2double(hi, lo);
+}
+constexpr int kQuad0 = 0x00, kQuad1 = 0x55, kQuad2 = 0xAA;   // lane 0, 1, 2 of the quad
+constexpr int kQuadNext = 0xC9;                              // lanes 1, 2, 0, 3
+template <int kCtrl>
+__device__ __forceinline__ uint32_t quad_move(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, kCtrl, 0xF, 0xF, false);
+}
+__device__ __forceinline__ uint32_t quad_sum(uint32_t v) {
+  v += quad_move<0xB1>(v);   // [1,0,3,2]
+  return v + quad_move<0x4E>(v);   // [2,3,0,1]
+}
+
+// What a twig's formation needs that the numbering has already written, read
+// ahead of the barrier that its children's moments wait for.
+struct QuadTwig {
+  uint32_t i, c0, nc, leafmask;
+};
+__device__ __forceinline__ QuadTwig quad_twig(uint32_t r, const UpArgs& u) {
+  const uint32_t a = threadIdx.x & 3u;
+  QuadTwig t;
+  t.i = u.node_rank[r];
+  t.c0 = u.fc_rank[r];
+  t.nc = u.fc_rank[r + 1] - t.c0;
+  uint32_t m = 0;
+  if (a < t.nc && u.ntype[t.c0 + a] == 0) m |= 1u << a;
+  if (a + 4u < t.nc && u.ntype[t.c0 + a + 4u] == 0) m |= 16u << a;
+  t.leafmask = quad_sum(m);   // disjoint bits
+  return t;
+}
+
+__device__ __forceinline__ void quad_moments(const QuadTwig& t, int level, const UpArgs& u) {
+  const uint32_t lane = threadIdx.x & 3u;
+  const uint32_t a = lane < 3u ? lane : 0u;   // lane 3 repeats component x
+  const double b2 = u.boxes[u.sys ? u.sys[u.nfirst[t.i]] : 0u].b2[level];
+  double ca[8], cq[8], cw[8], pa[8], qa[8], oa[8];
+#pragma unroll
+  for (uint32_t j = 0; j < 8; ++j) {
+    ca[j] = cq[j] = cw[j] = pa[j] = qa[j] = oa[j] = 0.0;
+    if (j < t.nc) {
+      if (t.leafmask & (1u << j)) {
+        const double* g = reinterpret_cast<const double*>(&u.geom[t.c0 + j]);
+        ca[j] = g[a];
+        cq[j] = g[3];
+        cw[j] = fabs(cq[j]);
+      } else {
+        const double* r = u.mom + (int64_t)(t.c0 + j) * 16;
+        ca[j] = r[M_CX + a];
+        cq[j] = r[M_Q];
+        cw[j] = r[M_AQ];
+        pa[j] = r[M_PX + a];
+        qa[j] = r[M_QX + a];
+        oa[j] = r[M_XY + a];
+      }
+    }
+  }
+  // counts and radii of the two children of this lane
+  uint32_t count = 0;
+  double bm[2] = {0.0, 0.0};
+#pragma unroll
+  for (uint32_t h = 0; h < 2; ++h) {
+    const uint32_t j = lane + 4u * h;
+    if (j < t.nc) {
+      if (t.leafmask & (1u << j)) {
+        count += 1u;
+      } else {
+        count += u.link[t.c0 + j].count;
+        bm[h] = u.mom[(int64_t)(t.c0 + j) * 16 + M_BMAX];
+      }
+      u.parent[t.c0 + j] = t.i;
+    }
+  }
+  count = quad_sum(count);
+  double charge = 0.0, absq = 0.0, coc = 0.0;
+#pragma unroll
+  for (uint32_t j = 0; j < 8; ++j) {
+    if (j < t.nc) {
+      charge = charge + cq[j];
+      absq = absq + cw[j];
+    }
+  }
+  if (absq != 0.0) {
+#pragma unroll
+    for (uint32_t j = 0; j < 8; ++j)
+      if (j < t.nc) coc = coc + (ca[j] * cw[j]);
+    coc = coc / absq;
+  } else {
+#pragma unroll
+    for (uint32_t j = 0; j < 8; ++j)
+      if (j < t.nc) coc = coc + ca[j];
+    coc = coc / (double)t.nc;
+  }
+  double dip = 0.0, quad = 0.0, off = 0.0, d2[2] = {0.0, 0.0};
+#pragma unroll
+  for (uint32_t j = 0; j < 8; ++j) {
+    if (j >= t.nc) continue;
+    const double sa = coc - ca[j];
+    const double sb = quad_move<kQuadNext>(sa), pb = quad_move<kQuadNext>(pa[j]);
+    const double qs = cq[j] * sa, ss = sa * sa;
+    dip = dip + pa[j] + qs;
+    quad = quad + qa[j] + pa[j] * sa + 0.5 * cq[j] * ss;
+    off = off + oa[j] + pa[j] * sb + pb * sa + qs * sb;
+    const double r2 = quad_move<kQuad0>(ss) + quad_move<kQuad1>(ss) + quad_move<kQuad2>(ss);
+    if (lane == (j & 3u)) d2[j >> 2] = r2;
+  }
+  double bmax = 0.0;   // no radius is negative
+  if (lane < t.nc) bmax = sqrt(d2[0]) + bm[0];
+  if (lane + 4u < t.nc) {
+    const double v = sqrt(d2[1]) + bm[1];
+    if (v > bmax) bmax = v;
+  }
+  {
+    const double v = quad_move<0xB1>(bmax);
+    if (v > bmax) bmax = v;
+  }
+  {
+    const double v = quad_move<0x4E>(bmax);
+    if (v > bmax) bmax = v;
+  }
+  const double tr = (quad_move<kQuad0>(quad) + quad_move<kQuad1>(quad)) + quad_move<kQuad2>(quad);
+  double* o = u.mom + (int64_t)t.i * 16;
+  double* g = reinterpret_cast<double*>(&u.geom[t.i]);
+  double w[4];   // this lane's walk moments: slots a, 3 + a, 7 + a; lane 3: 6, 10, 11
+  if (lane < 3u) {
+    o[M_CX + a] = coc;
+    o[M_PX + a] = dip;
+    o[M_QX + a] = quad;
+    o[M_XY + a] = off;
+    g[a] = coc;
+    w[0] = 2.0 * tr - 6.0 * quad;
+    w[1] = -3.0 * off;
+    w[2] = dip;
+  } else {
+    o[M_Q] = charge;
+    o[M_AQ] = absq;
+    o[M_BMAX] = bmax;
+    o[15] = 0.0;
+    double m[16];
+    m[M_BMAX] = bmax;
+    g[3] = walk_b2(m, b2, u.mac_select);
+    w[0] = tr;
+    w[1] = charge;
+    w[2] = 0.0;
+    u.link[t.i].nchild = t.nc;
+    u.link[t.i].count = count;
+    u.kidtwig[t.i] = (uint8_t)(~t.leafmask & ((1u << t.nc) - 1u));
+  }
+  const uint32_t k0 = lane < 3u ? a : 6u, k1 = lane < 3u ? 3u + a : 10u, k2 = lane < 3u ? 7u + a : 11u;
+  if (u.prec == kWalkFP64) {
+    double* v = u.wm64[t.i].v;
+    v[k0] = w[0]; v[k1] = w[1]; v[k2] = w[2];
+  } else {
+    float* v = u.wm32[t.i].v;
+    v[k0] = (float)w[0]; v[k1] = (float)w[1]; v[k2] = (float)w[2];
+  }
+}
+
+// A tile is one of the BFS numbering's.  It owns, at every level, one run of
+// twig ranks (rows of the scanned table), and of those only the last can
+// reach past the tile's end: a cell of level l crosses the end exactly when
+// the first particle behind it starts no node of level l or above (lo > l).
+// So one block forms every twig that lies in its tile, level by level with
+// only workgroup barriers between, and a second kernel of one block the twigs
+// that cross tile ends: two launches in place of one per level.
+// Upward pass 91 -> 42 us for 1,777 particles, 134 -> 63 for 32,768 (with a
+// thread per twig, 95); grow 372 -> 358 us for 131,072.  Larger trees have
+// enough twigs per level for thread-per-twig launches, which need fewer lanes
+// per twig (1,048,576 particles: 333 us by thread-per-twig tiles, 223 by level).
+constexpr int kUpT = 512;
+constexpr int kUpTiles = 256;
+constexpr int64_t kUpTilesMax = (int64_t)kUpTiles * kBfsTileSmall;   // 131,072 particles
+
+struct UpTiles {
+  const uint32_t* twig;   // [level][tile] rank of the tile's first twig of the level, level-major
+  const uint8_t* lo;
+  int64_t n;
+  int nb;                 // tiles
+};
+
+// The tile's twig ranks of the level (the entry behind a level's last tile is
+// the next level's first).
+__device__ __forceinline__ void tile_ranks(const UpTiles& t, int level, int c, uint32_t ntwig,
+                                           uint32_t& b, uint32_t& e) {
+  const int i = level * t.nb + c;
+  b = t.twig[i];
+  e = i + 1 < kLevels * t.nb ? t.twig[i + 1] : ntwig;
+}
+
+// Cells of levels below this one cross the end of the tile.
+__device__ __forceinline__ int cross_level(const UpTiles& t, int c) {
+  const int64_t end = (int64_t)(c + 1) * kBfsTileSmall;
+  return end < t.n ? (int)t.lo[end] : 0;
+}
+
+__global__ __launch_bounds__(kUpT) void upward_tile_kernel(UpTiles t, UpArgs u) {
+  if (tree_broken(u.sc)) return;
+  __shared__ uint32_t rb[kLevels], re[kLevels];
+  const int c = blockIdx.x;
+  if (threadIdx.x < kLevels) {
+    const int l = threadIdx.x;
+    uint32_t b, e;
+    tile_ranks(t, l, c, u.sc->ntwig, b, e);
+    if (e > b && l < cross_level(t, c)) --e;
+    rb[l] = b;
+    re[l] = e;
+  }
+  __syncthreads();
+  const uint32_t mine = threadIdx.x >> 2;
+  QuadTwig next = {0u, 0u, 0u, 0u};
+  bool ready = false;   // `next` holds this thread's first twig of the coming level
+  int l = kMaxLevel;
+  while (l >= 0 && rb[l] >= re[l]) --l;
+  while (l >= 0) {
+    const uint32_t b = rb[l], e = re[l];   // the same for every thread
+    int below = l - 1;
+    while (below >= 0 && rb[below] >= re[below]) --below;
+    for (uint32_t r = b + mine; r < e; r += kUpT / 4) {
+      if (!ready) next = quad_twig(r, u);
+      ready = false;
+      quad_moments(next, l, u);
+    }
+    ready = below >= 0 && rb[below] + mine < re[below];
+    if (ready) next = quad_twig(rb[below] + mine, u);
+    __syncthreads();
+    l = below;
+  }
+}
+
+__global__ __launch_bounds__(kUpT) void upward_cross_kernel(UpTiles t, UpArgs u) {
+  if (tree_broken(u.sc)) return;
+  __shared__ uint32_t re[kLevels][kUpTiles];   // the tile's crossing twig of the level + 1, 0: none
+  __shared__ int top;                          // deepest level of a crossing twig
+  const uint32_t ntwig = u.sc->ntwig;
+  if (threadIdx.x == 0) top = -1;
+  __syncthreads();
+  if (threadIdx.x < kUpTiles) {   // whole waves
+    const int c = threadIdx.x;
+    const int cross = c < t.nb ? cross_level(t, c) : 0;
+    int deepest = -1;
+#pragma unroll
+    for (int l = 0; l < kLevels; ++l) {
+      uint32_t b = 0, e = 0;
+      if (l < cross) tile_ranks(t, l, c, ntwig, b, e);
+      re[l][c] = e > b ? e : 0u;
+      if (e > b) deepest = l;
+    }
+    deepest = wave_max_i32(deepest);
+    if (lane_id() == 0) atomicMax(&top, deepest);
+  }
+  __syncthreads();
+  for (int l = top; l >= 0; --l) {
+    for (int c = threadIdx.x >> 2; c < t.nb; c += kUpT / 4) {
+      const uint32_t e = re[l][c];
+      if (e) quad_moments(quad_twig(e - 1u, u), l, u);
+    }
+    __syncthreads();
+  }
+}
+
 // One launch per level, deepest first, one thread per twig of the level:
 // twig ranks follow the BFS order, so a level's twigs are one contiguous run
 // of ranks, [twig_offset[level], twig_offset[level + 1]).
@@ -779,7 +1063,7 @@ void launch_dupfix(hipStream_t s, int64_t n, unsigned long long* keys, double* x
 }
 
 int64_t bfs_tiles(int64_t n) {
-  const int64_t b = (n + kBfsTile - 1) / kBfsTile;
+  const int64_t b = (n + bfs_tile(n) - 1) / bfs_tile(n);
   return b < 1 ? 1 : b;
 }
 
@@ -810,6 +1094,16 @@ void launch_upward(hipStream_t s, const TreeBuffers& t) {
   u.node_rank = t.node_rank; u.fc_rank = t.fc_rank; u.ntype = t.ntype; u.parent = t.parent;
   u.kidtwig = t.kidtwig;
   u.sc = t.sc;
+  if (t.n <= kUpTilesMax) {
+    UpTiles ut;
+    ut.nb = (int)bfs_tiles(t.n);
+    ut.n = t.n;
+    ut.lo = t.lo;
+    ut.twig = t.tab + 3 * (int64_t)kLevels * ut.nb;
+    upward_tile_kernel<<<(unsigned)ut.nb, kUpT, 0, s>>>(ut, u);
+    if (ut.nb > 1) upward_cross_kernel<<<1, kUpT, 0, s>>>(ut, u);
+    return;
+  }
   // A fixed grid near the resident capacity (six 256-thread blocks per CU of
   // MI355X) with a twig-stride loop: the large levels keep every CU busy and
   // the many small levels launch few idle blocks.
