@@ -114,7 +114,7 @@ void launch_dupfix(hipStream_t s, int64_t n, unsigned long long* keys, double* x
                    long long* kd, unsigned long long* oldkeys, uint32_t* dflag, uint32_t* dlist,
                    uint32_t* bsum, DevScalars* sc);
 void launch_tree_build(hipStream_t s, const TreeBuffers& t, int group_size, int group_pack);
-int64_t bfs_table_words(int64_t n);
+int64_t bfs_table_words(int64_t n);   // enough for every tree of at most n particles
 void launch_leaf_moments(hipStream_t s, const TreeBuffers& t);
 // Tree consistency counters res[7] (zeroed by the caller), see tree.hip.
 void launch_tree_check(hipStream_t s, const NodeLink* link, const uint32_t* parent, int64_t n,

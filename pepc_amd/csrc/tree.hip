@@ -1067,7 +1067,13 @@ int64_t bfs_tiles(int64_t n) {
   return b < 1 ? 1 : b;
 }
 
-int64_t bfs_table_words(int64_t n) { return 4 * (int64_t)kLevels * bfs_tiles(n); }
+// Words for every tree of at most n particles: the tile changes at kBfsLarge,
+// so a tree just below it has more tiles than one just above.
+int64_t bfs_table_words(int64_t n) {
+  int64_t tiles = bfs_tiles(n);
+  if (n > kBfsLarge && bfs_tiles(kBfsLarge) > tiles) tiles = bfs_tiles(kBfsLarge);
+  return 4 * (int64_t)kLevels * tiles;
+}
 
 void launch_tree_build(hipStream_t s, const TreeBuffers& t, int group_size, int group_pack) {
   const int64_t n = t.n, cap = t.cap, nb = bfs_tiles(n);

@@ -33,3 +33,17 @@ def test_tiles(n, clustered):
     assert np.array_equal(link[gg, 2].astype(np.int64), np.asarray(t.leaves, np.int64)[og])
     assert np.array_equal(t.mom[og][:, :15], mom[gg][:, :15])
     sol.close()
+
+
+@pytest.mark.parametrize("n", [940001, 1048576, 1048577])
+def test_table_capacity(n):
+    """Trees on both sides of the change of tile length, in a context whose
+    capacity lies on the other side, are sound."""
+    from pepc_amd.solver import Solver
+    r = np.random.Generator(np.random.PCG64(n))
+    p = r.random((n, 3))
+    sol = Solver(theta2=0.81, eps2=1e-4, precision="fp32", group_size=64, group_pack=64)
+    for m in (n, 1000):
+        st = sol.grow(*(np.ascontiguousarray(p[:m, k]) for k in range(3)), np.ones(m))
+        assert st["nleaf"] == m and sol.check_tree() == 0
+    sol.close()
