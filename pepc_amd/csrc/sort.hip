@@ -9,9 +9,13 @@
 // sort is stable.  Particle keys need 60 bits (the placeholder bit 60 is the
 // same for every key): seven 8-bit passes and one 4-bit pass.
 //
+// Arrays of up to 524,288 keys are sorted by merging instead (see below).
+//
 // Replaces the single-rank presort of slsort_keys (sl_pepc mpi_pepckeys.c:167,
 // sort_radix.c:33-151): for distinct keys both give the same permutation.
 #include "kernels.h"
+
+#include <utility>
 
 namespace pepc {
 
@@ -288,6 +292,98 @@ __global__ __launch_bounds__(kSortThreads) void digit_scan_kernel(uint32_t* __re
     }
   }
   if (threadIdx.x == 0) dtot[blockIdx.x] = tot;
+}
+
+// ---------------------------------------------------------------- merge sort
+// Smaller arrays: blocks of 2,048 pairs sorted in LDS (bitonic; values grow
+// with the position, so ordering by (key, value) is the stable order), then
+// four runs merged per launch, every element finding its place by binary
+// searches in the three other runs.  A radix pass costs two dependent
+// launches of 4 and 8 to 10 us whatever the size, eight times; here it is one
+// launch per factor of four above 2,048.  Whole grow, radix against merging:
+// 184 and 130 us for 1,777 particles, 254 and 186 for 32,768, 359 and 254 for
+// 131,072, 412 and 368 for 524,288; 532 and 553 for 1,048,576, where the
+// searches' scattered reads cost more than the passes.
+constexpr int kMergeT = 1024;
+constexpr int kMergeN = 2 * kMergeT;
+
+// Orders this wave's LDS accesses for the compiler (LDS instructions of one
+// wave execute in order).
+__device__ __forceinline__ void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+__global__ __launch_bounds__(kMergeT) void merge_block_kernel(
+    const unsigned long long* kin, const uint32_t* vin, unsigned long long* kout, uint32_t* vout,
+    int64_t n) {
+  __shared__ unsigned long long sk[kMergeN];
+  __shared__ uint32_t sv[kMergeN];
+  const int64_t base = (int64_t)blockIdx.x * kMergeN;
+  const int cnt = n - base < kMergeN ? (int)(n - base) : kMergeN;
+  int size = 2;
+  while (size < cnt) size *= 2;
+  const int t = threadIdx.x;
+  for (int e = t; e < size; e += kMergeT) {
+    sk[e] = e < cnt ? kin[base + e] : ~0ull;
+    sv[e] = e < cnt ? vin[base + e] : ~0u;
+  }
+  __syncthreads();
+  // A pair of distance j <= 64 lies in the 128 elements of one wave: those
+  // stages need no barrier among themselves.
+  for (int k = 2; k <= size; k *= 2) {
+    for (int j = k / 2; j > 0; j /= 2) {
+      if (t < size / 2) {
+        const int a = 2 * t - (t & (j - 1)), b = a + j;
+        const unsigned long long ka = sk[a], kb = sk[b];
+        const uint32_t va = sv[a], vb = sv[b];
+        const bool greater = ka > kb || (ka == kb && va > vb);
+        if (greater == ((a & k) == 0)) {
+          sk[a] = kb; sk[b] = ka;
+          sv[a] = vb; sv[b] = va;
+        }
+      }
+      const int next = j > 1 ? j / 2 : k;   // distance of the following stage
+      if (j > kWave || next > kWave) __syncthreads();
+      else wave_lds_order();
+    }
+  }
+  __syncthreads();
+  for (int e = t; e < cnt; e += kMergeT) {
+    kout[base + e] = sk[e];
+    vout[base + e] = sv[e];
+  }
+}
+
+// Runs of `run` elements (the last may be shorter), four to a group: element
+// i of a run moves behind the elements of the group's earlier runs that are
+// not greater and of its later runs that are smaller.
+__global__ __launch_bounds__(256) void merge4_kernel(const unsigned long long* __restrict__ kin,
+                                                     const uint32_t* __restrict__ vin,
+                                                     unsigned long long* __restrict__ kout,
+                                                     uint32_t* __restrict__ vout, int n, int run) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= n) return;
+  const unsigned long long key = kin[i];
+  const int r = i / run, first = r & ~3;
+  int pos[3] = {0, 0, 0}, begin[3], len[3];
+  unsigned long long bound[3];   // elements below it come first (keys are below 2^61)
+#pragma unroll
+  for (int q = 0; q < 3; ++q) {
+    const int other = first + q + (first + q >= r ? 1 : 0);
+    const int64_t b = (int64_t)other * run;
+    begin[q] = b < n ? (int)b : n;
+    len[q] = n - begin[q] < run ? n - begin[q] : run;
+    bound[q] = other < r ? key + 1ull : key;
+  }
+  for (int s = run; s > 0; s >>= 1) {
+#pragma unroll
+    for (int q = 0; q < 3; ++q)
+      if (pos[q] + s <= len[q] && kin[begin[q] + pos[q] + s - 1] < bound[q]) pos[q] += s;
+  }
+  const int64_t out = (int64_t)first * run + (i - r * run) + pos[0] + pos[1] + pos[2];
+  kout[out] = key;
+  vout[out] = vin[i];
 }
 
 __global__ __launch_bounds__(256) void gather4_kernel(int64_t n, const uint32_t* __restrict__ perm,
@@ -668,8 +764,27 @@ void launch_radix_pass(hipStream_t s, const unsigned long long* kin, const uint3
   launch_radix_pass_dev(s, kin, vin, kout, vout, n, nullptr, shift, nbits, hist, bsum, nullptr);
 }
 
-// Full sort of particle keys over bits [0, 60).  Input in (k0, v0); the sorted
-// result ends in (k0, v0) again after an even number of passes.  With a system
+// Largest array sorted by merging.
+constexpr int64_t kMergeMax = 524288;
+
+static void launch_merge_sort(hipStream_t s, unsigned long long* k0, uint32_t* v0,
+                              unsigned long long* k1, uint32_t* v1, int64_t n) {
+  int merges = 0;
+  for (int64_t run = kMergeN; run < n; run *= 4) ++merges;
+  unsigned long long *ka = k0, *kb = k1;
+  uint32_t *va = v0, *vb = v1;
+  if (merges % 2) { std::swap(ka, kb); std::swap(va, vb); }   // so the result ends in (k0, v0)
+  merge_block_kernel<<<(unsigned)((n + kMergeN - 1) / kMergeN), kMergeT, 0, s>>>(k0, v0, ka, va, n);
+  int run = kMergeN;
+  for (int m = 0; m < merges; ++m, run *= 4) {
+    merge4_kernel<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(ka, va, kb, vb, (int)n, run);
+    std::swap(ka, kb);
+    std::swap(va, vb);
+  }
+}
+
+// Full sort of particle keys over bits [0, 60), values ascending on input.
+// Input in (k0, v0); the sorted result ends in (k0, v0) again.  With a system
 // index per input particle (sysid != nullptr, values < nsys <= 65536), two more
 // stable passes over its 16 bits order the particles by (system, key); the
 // upper pass only runs when there are more than 256 systems, and then the
@@ -677,6 +792,10 @@ void launch_radix_pass(hipStream_t s, const unsigned long long* kin, const uint3
 void launch_sort_keys(hipStream_t s, unsigned long long* k0, uint32_t* v0, unsigned long long* k1,
                       uint32_t* v1, int64_t n, uint32_t* hist, uint32_t* bsum,
                       const uint32_t* sysid, int64_t nsys) {
+  if (!sysid && n <= kMergeMax) {
+    launch_merge_sort(s, k0, v0, k1, v1, n);
+    return;
+  }
   static const int shifts[8] = {0, 8, 16, 24, 32, 40, 48, 56};
   static const int widths[8] = {8, 8, 8, 8, 8, 8, 8, 4};
   for (int p = 0; p < 8; ++p) {
