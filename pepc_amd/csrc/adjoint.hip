@@ -40,55 +40,56 @@ __device__ __forceinline__ bool broken(const DevScalars* sc) {
 }
 
 // Derivatives of gphi * phi + u . E for one interaction (see header comment).
-// qt = {qx, qy, qz, xy, yz, zx} (Qt_xx = qx, Qt_xy = xy / 2, ...).  Outputs:
-// D = dL/dd, gq, gp, M = dL/dQt as the symmetric matrix {xx, yy, zz, xy, yz, zx}.
-// The adjoint is checked against the oracle to a tolerance, so its terms may
-// contract products and sums into fused multiply-adds.
-__device__ void adjoint_term(const double d[3], double r2, double gphi, const double u[3],
-                             double q, const double p[3], const double qt[6], double D[3],
-                             double& gq, double gp[3], double M[6]) {
+// qt = {xx, yy, zz, xy, yz, zx} of the symmetric matrix Qt, tr its trace.
+// Outputs: D = dL/dd, gq, gp, M = dL/dQt as the symmetric matrix {xx, yy, zz,
+// xy, yz, zx}.  The adjoint is checked against the oracle to a tolerance, so
+// its terms may contract products and sums into fused multiply-adds.
+//
+// The terms of phi = q G + p.grad G + Qt : grad grad G and E = -grad phi,
+// differentiated and collected by vector, with
+//   s1 = gphi r^-3 + 3 ud r^-5,  s2 = 3 gphi r^-5 + 15 ud r^-7,
+//   w = s2 d - 3 r^-5 u:
+//   gp = u r^-3 - s1 d,  M_ab = w_a d_b - 3 r^-5 u_b d_a - s1 delta_ab,
+//   D = cu u - s1 p + 2 Qt w + cd d
+// (one product with Qt for the vector w besides the one for d; about 110 FP64
+// instructions, 134 with separate products for d and u).
+__device__ __forceinline__ void adjoint_term(const double d[3], double r2, double gphi,
+                                             const double u[3], double q, const double p[3],
+                                             const double qt[6], double tr, double D[3],
+                                             double& gq, double gp[3], double M[6]) {
 #pragma clang fp contract(fast)
   const double ri = rsqrt(r2);
   const double ri2 = ri * ri;
   const double r3 = ri * ri2, r5 = r3 * ri2, r7 = r5 * ri2, r9 = r7 * ri2;
   const double ud = u[0] * d[0] + u[1] * d[1] + u[2] * d[2];
-  const double pd = p[0] * d[0] + p[1] * d[1] + p[2] * d[2];
+  const double pt = p[0] * d[0] + p[1] * d[1] + p[2] * d[2] + tr;
   const double up = u[0] * p[0] + u[1] * p[1] + u[2] * p[2];
-  const double hxy = 0.5 * qt[3], hyz = 0.5 * qt[4], hzx = 0.5 * qt[5];
-  const double Qd[3] = {qt[0] * d[0] + hxy * d[1] + hzx * d[2],
-                        hxy * d[0] + qt[1] * d[1] + hyz * d[2],
-                        hzx * d[0] + hyz * d[1] + qt[2] * d[2]};
-  const double Qu[3] = {qt[0] * u[0] + hxy * u[1] + hzx * u[2],
-                        hxy * u[0] + qt[1] * u[1] + hyz * u[2],
-                        hzx * u[0] + hyz * u[1] + qt[2] * u[2]};
-  const double tr = qt[0] + qt[1] + qt[2];
+  const double Qd[3] = {qt[0] * d[0] + qt[3] * d[1] + qt[5] * d[2],
+                        qt[3] * d[0] + qt[1] * d[1] + qt[4] * d[2],
+                        qt[5] * d[0] + qt[4] * d[1] + qt[2] * d[2]};
   const double dQd = d[0] * Qd[0] + d[1] * Qd[1] + d[2] * Qd[2];
   const double uQd = u[0] * Qd[0] + u[1] * Qd[1] + u[2] * Qd[2];
-  // The terms of phi = q G + p.grad G + Qt : grad grad G and E = -grad phi,
-  // differentiated and collected by vector, with
-  //   s1 = gphi r^-3 + 3 ud r^-5,  s2 = 3 gphi r^-5 + 15 ud r^-7:
-  //   gp = u r^-3 - s1 d,  M_ab = s2 d_a d_b - 3 r^-5 (u_a d_b + u_b d_a) - s1 delta_ab,
-  //   D = cu u - s1 p + 2 s2 Qd - 6 r^-5 Qu + cd d.
-  const double s1 = gphi * r3 + 3.0 * ud * r5;
-  const double s2 = 3.0 * gphi * r5 + 15.0 * ud * r7;
-  const double s3 = 15.0 * gphi * r7 + 105.0 * ud * r9;
-  const double pt = pd + tr;
-  const double t5 = 3.0 * r5;
+  const double t5 = 3.0 * r5, t7 = 15.0 * r7;
+  const double s1 = gphi * r3 + ud * t5;
+  const double s2 = gphi * t5 + ud * t7;
+  const double s3 = gphi * t7 + ud * (105.0 * r9);
+  const double tu[3] = {t5 * u[0], t5 * u[1], t5 * u[2]};
+  const double w[3] = {s2 * d[0] - tu[0], s2 * d[1] - tu[1], s2 * d[2] - tu[2]};
   gq = gphi * ri + ud * r3;
 #pragma unroll
-  for (int k = 0; k < 3; ++k) gp[k] = u[k] * r3 - s1 * d[k];
-  const int ma[6] = {0, 1, 2, 0, 1, 2}, mb[6] = {0, 1, 2, 1, 2, 0};
-#pragma unroll
-  for (int k = 0; k < 6; ++k) {
-    const int a = ma[k], b = mb[k];
-    const double v = s2 * d[a] * d[b] - t5 * (u[a] * d[b] + u[b] * d[a]);
-    M[k] = a == b ? v - s1 : v;
+  for (int k = 0; k < 3; ++k) {
+    gp[k] = u[k] * r3 - s1 * d[k];
+    M[k] = w[k] * d[k] - (tu[k] * d[k] + s1);
+    const int l = k == 2 ? 0 : k + 1;
+    M[3 + k] = w[k] * d[l] - tu[l] * d[k];
   }
-  const double cu = q * r3 - t5 * pt + 15.0 * r7 * dQd;
-  const double cd = -q * s1 + pt * s2 - t5 * up - s3 * dQd + 30.0 * r7 * uQd;
+  const double cu = q * r3 - t5 * pt + t7 * dQd;
+  const double cd = pt * s2 - q * s1 - t5 * up - s3 * dQd + 2.0 * (t7 * uQd);
+  const double Qw[3] = {qt[0] * w[0] + qt[3] * w[1] + qt[5] * w[2],
+                        qt[3] * w[0] + qt[1] * w[1] + qt[4] * w[2],
+                        qt[5] * w[0] + qt[4] * w[1] + qt[2] * w[2]};
 #pragma unroll
-  for (int k = 0; k < 3; ++k)
-    D[k] = cu * u[k] - s1 * p[k] + 2.0 * s2 * Qd[k] - 2.0 * t5 * Qu[k] + cd * d[k];
+  for (int k = 0; k < 3; ++k) D[k] = cu * u[k] - s1 * p[k] + 2.0 * Qw[k] + cd * d[k];
 }
 
 // The same for a leaf (p = Qt = 0): D = dL/dd and gq only.
@@ -101,8 +102,9 @@ __device__ __forceinline__ void adjoint_term_p2p(const double d[3], double r2, d
   const double r3 = ri * ri2, r5 = r3 * ri2;
   const double ud = u[0] * d[0] + u[1] * d[1] + u[2] * d[2];
   gq = gphi * ri + ud * r3;
+  const double cu = q * r3, cd = q * (gphi * r3 + ud * (3.0 * r5));
 #pragma unroll
-  for (int k = 0; k < 3; ++k) D[k] = q * ((u[k] - gphi * d[k]) * r3 - 3.0 * ud * d[k] * r5);
+  for (int k = 0; k < 3; ++k) D[k] = cu * u[k] - cd * d[k];
 }
 
 // Lane k's value in every lane (k uniform): register reads, no LDS.
@@ -164,6 +166,31 @@ __device__ __forceinline__ double wsum4(double v0, double v1, double v2, double 
   double x = v0 + v1, y = v2 + v3;
   swap16(x, y);
   return row_sum(x + y);
+}
+
+// Wave sums of up to 16 values on the matrix cores, which the vector-ALU-bound
+// walk leaves idle.  v_mfma_f64_4x4x4_4b keeps A[i][k] of block b in lane
+// 16k + 4b + i, B[k][j] in lane 16k + 4b + j and D[i][j] in lane 16i + 4b + j.
+// With value j of four as A and B's column j ones, D[i][j] collects over k;
+// with that D as B and A's row g ones, row g of the second D collects over i.
+// Afterwards lane 16g + 4b + j holds block b's part of value 4g + j, and two
+// DPP additions sum the four blocks.
+struct LaneSelect {
+  double on[4];   // on[v] = 1 in the lanes with lane % 4 == v, 0 elsewhere
+};
+__device__ __forceinline__ LaneSelect lane_select(int lane) {
+  LaneSelect s;
+#pragma unroll
+  for (int v = 0; v < 4; ++v) s.on[v] = (lane & 3) == v ? 1.0 : 0.0;
+  return s;
+}
+template <int N>
+__device__ __forceinline__ double mfma_collect(const LaneSelect& sel, const double (&v)[N], int g,
+                                               double acc) {
+  double d = 0.0;
+#pragma unroll
+  for (int j = 0; j < N; ++j) d = __builtin_amdgcn_mfma_f64_4x4x4f64(v[j], sel.on[j], d, 0, 0, 0);
+  return __builtin_amdgcn_mfma_f64_4x4x4f64(sel.on[g], d, acc, 0, 0, 0);
 }
 
 // The adjoint buffers are plain device allocations (coarse grained), where the
@@ -259,18 +286,26 @@ struct AdjArgs {
 // stages the popped nodes' interaction data in LDS with the node records (a
 // twig's charge, dipole and quadrupole, a leaf's particle charge): the
 // entries of a step then read LDS only, and the step's one wait on memory
-// also drains the previous step's atomics.  A node's 13 sums (4 for a leaf's
-// particle) are reduce-scattered across the wave (wsum4) and go out as one
-// atomic instruction, one value per lane.  Four waves per SIMD: the 128-VGPR
-// budget costs a few bytes of spill and hides more of each step's latency.
+// also drains the previous step's atomics.  A node's 13 sums are formed on the
+// matrix cores (17 instructions of 17 clocks beside the vector ALUs, in place
+// of 130 vector instructions of the 303 per entry; with the shorter terms 164:
+// 262,144 particles in groups of up to 64 3.43 -> 2.80 ms), a leaf's particle's
+// 4 are reduce-scattered across the wave (wsum4); either goes out as one atomic
+// instruction, one value per lane.  Four waves per SIMD: the 128-VGPR budget
+// costs a few bytes of spill and hides more of each step's latency.
 __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(4)))
 void adjoint_walk_kernel(AdjArgs a) {
   __shared__ uint32_t stack[kStackCap + kStackSlack];
-  __shared__ double smom[kWave][10];   // q, p[3], Qt[6] of popped node k
+  __shared__ double smom[kWave][12];   // q, p[3], Qt[6], trace Qt of popped node k
   __shared__ uint32_t gsh;
   const int lane = threadIdx.x;
   const uint32_t ngroups = a.sc->ngroups;
   const double eps2 = a.eps2;
+  const LaneSelect sel = lane_select(lane);
+  // slot of nadj that this lane adds: row 0 slots 0..3, row 1 4..7, row 2 8..9,
+  // row 3 10..12 (-1: none)
+  const int srow = lane >> 4, scol = lane & 15;
+  const int node_slot = scol >= (srow == 2 ? 2 : srow == 3 ? 3 : 4) ? -1 : srow == 3 ? 10 + scol : 4 * srow + scol;
   // Work units: a group's walk is cut at its root into one unit per child of
   // the root (the acceptance decisions do not depend on the order of the
   // walk, so the units' entries are the group's), which evens out the end of
@@ -331,8 +366,11 @@ void adjoint_walk_kernel(AdjArgs a) {
           smom[lane][0] = mm[3];
 #pragma unroll
           for (int j = 0; j < 3; ++j) smom[lane][1 + j] = mm[5 + j];
+          const double qx = mm[8], qy = mm[9], qz = mm[10];
+          smom[lane][4] = qx; smom[lane][5] = qy; smom[lane][6] = qz;
 #pragma unroll
-          for (int j = 0; j < 6; ++j) smom[lane][4 + j] = mm[8 + j];
+          for (int j = 0; j < 3; ++j) smom[lane][7 + j] = 0.5 * mm[11 + j];   // Qt_xy = xy / 2, ...
+          smom[lane][10] = qx + qy + qz;
         } else {
           smom[lane][0] = a.q[mylk.first];
         }
@@ -382,25 +420,18 @@ void adjoint_walk_kernel(AdjArgs a) {
         const double q = smom[k][0];
         const double p[3] = {smom[k][1], smom[k][2], smom[k][3]};
         const double qt[6] = {smom[k][4], smom[k][5], smom[k][6], smom[k][7], smom[k][8], smom[k][9]};
-        adjoint_term(d, r2, gphi, u, q, p, qt, D, gq, gp, M);
-        if (!valid) {
-          D[0] = D[1] = D[2] = 0.0; gq = 0.0; gp[0] = gp[1] = gp[2] = 0.0;
-#pragma unroll
-          for (int j = 0; j < 6; ++j) M[j] = 0.0;
-        }
+        adjoint_term(d, r2, gphi, u, q, p, qt, smom[k][10], D, gq, gp, M);
+        // (lanes without a target have gphi = u = 0: every derivative is 0)
         tD[0] += D[0]; tD[1] += D[1]; tD[2] += D[2];
-        // the node's 13 sums (slots 0..12): register c holds values 4c..4c+3,
-        // and lane 16 r + c adds value 4c + row_value(r)
-        const double s0 = wsum4(gq, gp[0], gp[1], gp[2]);
-        const double s1 = wsum4(M[0], M[1], M[2], M[3]);
-        const double s2 = wsum4(M[4], M[5], D[0], D[1]);
-        const double s3 = wsum4(D[2], 0.0, 0.0, 0.0);
-        const int c = lane & 15;
-        const int j = 4 * c + row_value(lane >> 4);
-        if (c < 4 && j < 13) {
-          const double sv = c == 0 ? s0 : c == 1 ? s1 : c == 2 ? s2 : s3;
-          unsafeAtomicAdd(&a.nadj[(size_t)node * 16 + j], sv);
-        }
+        // the node's 13 sums, one per lane of the four rows
+        const double v0[4] = {gq, gp[0], gp[1], gp[2]}, v1[4] = {M[0], M[1], M[2], M[3]};
+        const double v2[2] = {M[4], M[5]}, v3[3] = {D[0], D[1], D[2]};
+        double sv = mfma_collect(sel, v0, 0, 0.0);
+        sv = mfma_collect(sel, v1, 1, sv);
+        sv = mfma_collect(sel, v2, 2, sv);
+        sv = mfma_collect(sel, v3, 3, sv);
+        sv = dpp_add<0x128>(dpp_add<0x124>(sv));   // row_ror:4, then row_ror:8
+        if (node_slot >= 0) unsafeAtomicAdd(&a.nadj[(size_t)node * 16 + node_slot], sv);
       }
       __syncthreads();
     }
