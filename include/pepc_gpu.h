@@ -202,6 +202,16 @@ int pepc_gpu_sorted_device(void *ctx, const uint64_t **keys, const uint32_t **pe
 int pepc_gpu_restore_device(void *ctx, int64_t count, const double *const *in,
                             double *const *out);
 
+/* Fields between the sorted order of the last grow (ex, ey, ez, pot, as
+ * pepc_gpu_traverse_device writes them) and the input order with one row of
+ * three per particle (e[3 i + c], phi[i]): restore_fields sorted -> input,
+ * sort_fields input -> sorted.  Device arrays, no overlap between inputs and
+ * outputs.  Asynchronous on the context's stream. */
+int pepc_gpu_restore_fields_device(void *ctx, const double *ex, const double *ey, const double *ez,
+                                   const double *pot, double *e, double *phi);
+int pepc_gpu_sort_fields_device(void *ctx, const double *e, const double *phi, double *ex,
+                                double *ey, double *ez, double *pot);
+
 /* Host copies of the sorted particle arrays of the last grow (each may be
  * NULL): keys[n], perm[n] (input index of sorted particle i), x,y,z,q[n]. */
 int pepc_gpu_read_sorted(void *ctx, uint64_t *keys, int64_t *perm, double *x, double *y,

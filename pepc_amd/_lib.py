@@ -27,7 +27,8 @@ EXPORTS = [
     "pepc_gpu_timings", "pepc_gpu_grow_batch_device", "pepc_gpu_state_set", "pepc_gpu_run",
     "pepc_gpu_state_get", "pepc_gpu_state_device", "pepc_gpu_read_energies",
     "pepc_gpu_adjoint_device", "pepc_gpu_autotune", "pepc_gpu_get_config", "pepc_gpu_freeze",
-    "pepc_gpu_replay_device", "pepc_gpu_restore_device", "pepc_gpu_periodic_default",
+    "pepc_gpu_replay_device", "pepc_gpu_restore_device",
+    "pepc_gpu_restore_fields_device", "pepc_gpu_sort_fields_device", "pepc_gpu_periodic_default",
     "pepc_gpu_set_periodic", "pepc_gpu_lattice_get", "pepc_gpu_constrain_periodic_device",
     "pepc_gpu_traverse_sinks_device", "pepc_gpu_traverse_sinks", "pepc_gpu_read_sink_counts",
     "pepc_gpu_check_tree", "pepc_gpu_direct", "pepc_gpu_reserve_nodes", "pepc_gpu_read_box",
@@ -137,6 +138,8 @@ def load(path: str = LIB_PATH):
     L.pepc_gpu_get_config.argtypes = [_vp, C.POINTER(Config)]
     L.pepc_gpu_freeze.argtypes = [_vp, C.POINTER(_i64)]
     L.pepc_gpu_restore_device.argtypes = [_vp, _i64, C.POINTER(_vp), C.POINTER(_vp)]
+    L.pepc_gpu_restore_fields_device.argtypes = [_vp] * 7
+    L.pepc_gpu_sort_fields_device.argtypes = [_vp] * 7
     L.pepc_gpu_replay_device.argtypes = [_vp] * 9
     L.pepc_gpu_periodic_default.argtypes = [C.POINTER(Periodic)]
     L.pepc_gpu_periodic_default.restype = None

@@ -9,8 +9,9 @@ The Barnes-Hut acceptance decisions are piecewise constant in the positions,
 so this is the derivative of the solve wherever the decisions do not change
 (everywhere at theta = 0).
 
-The permutation between input order and the solver's key order is applied
-with torch index operations; every arithmetic step is in libpepc_gpu.so.
+The permutation between input order and the solver's key order stays on the
+device (pepc_gpu_restore_fields_device and its reverse); every arithmetic step
+is in libpepc_gpu.so.
 """
 from __future__ import annotations
 
@@ -20,45 +21,40 @@ import torch
 class _CoulombField(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, y, z, q, solver):
+        if x.device != solver.device:
+            raise ValueError(f"coulomb_field: inputs on {x.device}, solver on {solver.device}")
         solver.grow(x.detach(), y.detach(), z.detach(), q.detach())
-        res = solver.traverse()
-        perm = torch.from_numpy(solver.sorted_host()[1]).to(x.device)
-        n = perm.numel()
-        e = torch.empty((n, 3), dtype=torch.float64, device=x.device)
-        pot = torch.empty(n, dtype=torch.float64, device=x.device)
-        e[perm] = res.e.T
-        pot[perm] = res.pot
+        # one wait for the walk and the restore: when this returns, nothing of
+        # it is left on the stream that a grow on another stream could overtake
+        res = solver.traverse(sync=False)
+        e, pot = solver.restore_fields(res.e, res.pot)
+        solver.sync()
         solver._generation = getattr(solver, "_generation", 0) + 1
         ctx.solver = solver
         ctx.generation = solver._generation
-        ctx.save_for_backward(perm, x.detach(), y.detach(), z.detach(), q.detach())
+        ctx.save_for_backward(x.detach(), y.detach(), z.detach(), q.detach())
         return e, pot
 
     @staticmethod
     def backward(ctx, ge, gpot):
-        perm, x, y, z, q = ctx.saved_tensors
+        x, y, z, q = ctx.saved_tensors
         solver = ctx.solver
         if getattr(solver, "_generation", None) != ctx.generation:
             # the solver grew another tree since this forward: rebuild this
-            # one (the build is deterministic, so tree and lists are the same)
+            # one (the build is deterministic, so tree, order and lists are
+            # the same)
             solver.grow(x, y, z, q)
             solver._generation += 1
             ctx.generation = solver._generation
-        n = perm.numel()
-        dev = perm.device
+        n = x.numel()
         if ge is None:
-            ge = torch.zeros((n, 3), dtype=torch.float64, device=dev)
+            ge = torch.zeros((n, 3), dtype=torch.float64, device=solver.device)
         if gpot is None:
-            gpot = torch.zeros(n, dtype=torch.float64, device=dev)
-        ges = ge.to(torch.float64)[perm].T.contiguous()
-        gps = gpot.to(torch.float64)[perm].contiguous()
-        gx, gy, gz, gq = solver.adjoint(ges, gps)
-        outs = []
-        for g in (gx, gy, gz, gq):
-            o = torch.empty_like(g)
-            o[perm] = g
-            outs.append(o)
-        return outs[0], outs[1], outs[2], outs[3], None
+            gpot = torch.zeros(n, dtype=torch.float64, device=solver.device)
+        ges, gps = solver.sort_fields(ge, gpot)
+        grads = solver.restore(*solver.adjoint(ges, gps, sync=False), sync=False)
+        solver.sync()
+        return (*grads, None)
 
 
 def coulomb_field(x, y, z, q, solver):

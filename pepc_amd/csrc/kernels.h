@@ -61,6 +61,12 @@ void launch_tie_order(hipStream_t s, int64_t n, int64_t nsys, const int64_t* sof
 // out[perm[i]] = in[i] (back to input order)
 void launch_scatter_back(hipStream_t s, int64_t n, const uint32_t* perm, const double* in,
                          double* out);
+// Fields between sorted order and input order (rows of three), both ways.
+void launch_restore_fields(hipStream_t s, int64_t n, const uint32_t* perm, const double* ex,
+                           const double* ey, const double* ez, const double* pot, double* e,
+                           double* phi);
+void launch_sort_fields(hipStream_t s, int64_t n, const uint32_t* perm, const double* e,
+                        const double* phi, double* ex, double* ey, double* ez, double* pot);
 // Sorted SoA particles from the 32-byte records: xs[i] = rec[perm[i]].x, ...
 void launch_gather_rec(hipStream_t s, int64_t n, const uint32_t* perm, const double4* rec,
                        double* xs, double* ys, double* zs, double* qs);

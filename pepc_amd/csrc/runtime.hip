@@ -1013,6 +1013,32 @@ int pepc_gpu_restore_device(void* p, int64_t count, const double* const* in, dou
   return 0;
 }
 
+int pepc_gpu_restore_fields_device(void* p, const double* ex, const double* ey, const double* ez,
+                                   const double* pot, double* e, double* phi) {
+  Ctx* c = as_ctx(p);
+  if (!c) return PEPC_GPU_EINVAL;
+  if (!c->grown) return fail(c, PEPC_GPU_EINVAL, "restore_fields: no tree (call grow first)");
+  if (!ex || !ey || !ez || !pot || !e || !phi)
+    return fail(c, PEPC_GPU_EINVAL, "restore_fields: null argument");
+  HIPCHECK(c, hipSetDevice(c->cfg.device));
+  launch_restore_fields(c->stream, c->n, c->v0, ex, ey, ez, pot, e, phi);
+  HIPCHECK(c, hipGetLastError());
+  return 0;
+}
+
+int pepc_gpu_sort_fields_device(void* p, const double* e, const double* phi, double* ex, double* ey,
+                                double* ez, double* pot) {
+  Ctx* c = as_ctx(p);
+  if (!c) return PEPC_GPU_EINVAL;
+  if (!c->grown) return fail(c, PEPC_GPU_EINVAL, "sort_fields: no tree (call grow first)");
+  if (!ex || !ey || !ez || !pot || !e || !phi)
+    return fail(c, PEPC_GPU_EINVAL, "sort_fields: null argument");
+  HIPCHECK(c, hipSetDevice(c->cfg.device));
+  launch_sort_fields(c->stream, c->n, c->v0, e, phi, ex, ey, ez, pot);
+  HIPCHECK(c, hipGetLastError());
+  return 0;
+}
+
 int pepc_gpu_read_sorted(void* p, uint64_t* keys, int64_t* perm, double* x, double* y, double* z,
                          double* q) {
   Ctx* c = as_ctx(p);

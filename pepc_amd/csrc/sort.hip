@@ -440,6 +440,37 @@ __global__ __launch_bounds__(256) void scatter_back_kernel(int64_t n, const uint
   out[perm[i]] = in[i];
 }
 
+// Memory bound: 32 bytes read and 32 written per particle, one side of them
+// scattered by the permutation in runs of 24 and 8 bytes. They take the place
+// of a permutation that went to the host and back and of four indexed torch
+// operations each way: a differentiable solve with its backward pass over
+// 262,144 particles went from 5.1 to 4.0 ms.
+__global__ __launch_bounds__(256) void restore_fields_kernel(
+    int64_t n, const uint32_t* __restrict__ perm, const double* __restrict__ ex,
+    const double* __restrict__ ey, const double* __restrict__ ez, const double* __restrict__ pot,
+    double* __restrict__ e, double* __restrict__ phi) {
+  const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const int64_t p = perm[i];
+  e[3 * p] = ex[i];
+  e[3 * p + 1] = ey[i];
+  e[3 * p + 2] = ez[i];
+  phi[p] = pot[i];
+}
+
+__global__ __launch_bounds__(256) void sort_fields_kernel(
+    int64_t n, const uint32_t* __restrict__ perm, const double* __restrict__ e,
+    const double* __restrict__ phi, double* __restrict__ ex, double* __restrict__ ey,
+    double* __restrict__ ez, double* __restrict__ pot) {
+  const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const int64_t p = perm[i];
+  ex[i] = e[3 * p];
+  ey[i] = e[3 * p + 1];
+  ez[i] = e[3 * p + 2];
+  pot[i] = phi[p];
+}
+
 // ---------------------------------------------------------------- tie order
 // Order of equal keys as the reference's local presort leaves it.
 //
@@ -817,6 +848,17 @@ void launch_sort_keys(hipStream_t s, unsigned long long* k0, uint32_t* v0, unsig
 void launch_scatter_back(hipStream_t s, int64_t n, const uint32_t* perm, const double* in,
                          double* out) {
   scatter_back_kernel<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(n, perm, in, out);
+}
+
+void launch_restore_fields(hipStream_t s, int64_t n, const uint32_t* perm, const double* ex,
+                           const double* ey, const double* ez, const double* pot, double* e,
+                           double* phi) {
+  restore_fields_kernel<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(n, perm, ex, ey, ez, pot, e, phi);
+}
+
+void launch_sort_fields(hipStream_t s, int64_t n, const uint32_t* perm, const double* e,
+                        const double* phi, double* ex, double* ey, double* ez, double* pot) {
+  sort_fields_kernel<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(n, perm, e, phi, ex, ey, ez, pot);
 }
 
 void launch_gather_rec(hipStream_t s, int64_t n, const uint32_t* perm, const double4* rec,

@@ -263,7 +263,7 @@ class Solver:
             self.sync()
         return out
 
-    def restore(self, *arrays):
+    def restore(self, *arrays, sync=True):
         """Device arrays in sorted order (e.g. traverse results) back to the
         input order of the last grow; returns new tensors."""
         t = self.torch
@@ -277,8 +277,39 @@ class Solver:
         self._bind_stream()
         self._check(self.lib.pepc_gpu_restore_device(self.h, k, pin, pout))
         self._keep_restore = ins
-        t.cuda.synchronize(self.device)
+        if sync:
+            t.cuda.synchronize(self.device)
         return outs
+
+    def restore_fields(self, e, pot):
+        """Fields e (3, n) and potentials in sorted order to input order, one
+        row of three per particle: (n, 3) and (n,).  Asynchronous."""
+        t = self.torch
+        n = self.n
+        e, pot = self._dev(e), self._dev(pot)
+        if e.shape != (3, n) or pot.shape != (n,):
+            raise ValueError("restore_fields: e must be (3, n) and pot (n,)")
+        out = (t.empty((n, 3), dtype=t.float64, device=self.device),
+               t.empty(n, dtype=t.float64, device=self.device))
+        self._bind_stream()
+        self._check(self.lib.pepc_gpu_restore_fields_device(
+            self.h, _ptr(e[0]), _ptr(e[1]), _ptr(e[2]), _ptr(pot), _ptr(out[0]), _ptr(out[1])))
+        return out
+
+    def sort_fields(self, e, pot):
+        """The reverse of restore_fields.  Asynchronous."""
+        t = self.torch
+        n = self.n
+        e, pot = self._dev(e), self._dev(pot)
+        if e.shape != (n, 3) or pot.shape != (n,):
+            raise ValueError("sort_fields: e must be (n, 3) and pot (n,)")
+        out = (t.empty((3, n), dtype=t.float64, device=self.device),
+               t.empty(n, dtype=t.float64, device=self.device))
+        self._bind_stream()
+        self._check(self.lib.pepc_gpu_sort_fields_device(
+            self.h, _ptr(e), _ptr(pot), _ptr(out[0][0]), _ptr(out[0][1]), _ptr(out[0][2]),
+            _ptr(out[1])))
+        return out
 
     # -------------------------------------------------------------- timestep
     def state_set(self, x, y, z, v, q, m, offsets=None, max_records=1024):
