@@ -45,7 +45,7 @@ struct DevScalars {
   uint32_t nnodes;
   uint32_t ntwig;
   uint32_t ngroups;
-  uint32_t dup_scan_n;          // particles the duplicate fix-up scans (0 without duplicates)
+  uint32_t pad0;
   uint32_t maxlevel_used;
   uint32_t level_offset[kMaxLevel + 2];   // first node of every level; [kMaxLevel + 1] = nnodes
   uint32_t twig_offset[kMaxLevel + 2];    // first twig rank of every level; [kMaxLevel + 1] = ntwig

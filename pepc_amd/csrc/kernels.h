@@ -31,11 +31,10 @@ void launch_sink_groups(hipStream_t s, int64_t m, int g, uint32_t* gfirst, uint3
 int64_t scan_blocks(int64_t n);
 int64_t sort_blocks(int64_t n);
 // Exclusive scan of n values (in place allowed); *total gets the sum when
-// total != nullptr.  With ndev != nullptr only the first min(n, *ndev) values
-// are scanned (the count is read on the device; n sizes the grid).  With
-// flags, each value counts as 1 when nonzero and 0 otherwise.
+// total != nullptr.  With flags, each value counts as 1 when nonzero and 0
+// otherwise.
 void launch_scan(hipStream_t s, const uint32_t* in, uint32_t* out, int64_t n, uint32_t* bsum,
-                 uint32_t* total, const uint32_t* ndev = nullptr, bool flags = false);
+                 uint32_t* total, bool flags = false);
 void launch_radix_pass(hipStream_t s, const unsigned long long* kin, const uint32_t* vin,
                        unsigned long long* kout, uint32_t* vout, int64_t n, int shift, int nbits,
                        uint32_t* hist, uint32_t* bsum);
@@ -51,13 +50,17 @@ void launch_sort_keys(hipStream_t s, unsigned long long* k0, uint32_t* v0, unsig
 // Reorders runs of equal keys in perm (after launch_sort_keys and
 // launch_dup_detect) into the order the reference's in-place MSD presort
 // gives them; nothing to do (one uniform load per block) when dup_count is 0.
-// Scratch: kin[n] (keys by input index), ord/ord2[n], cls[n], and the
-// per-pass slot lists fp[n] (positions) and fec[n] (element | class << 32).
+// Then moves the equal keys in ks apart (module_domains.f90:248-297) and puts
+// the particles whose key changed at the new cells' centres (in rec, input
+// order).  Scratch: kin[n] (keys by input index), ord/ord2[n], cls[n],
+// list[n], and the per-pass slot lists fp[n] (positions) and fec[n]
+// (element | class << 32).
 // One block per system (soff: nsys + 1 offsets when nsys > 1).
 void launch_tie_order(hipStream_t s, int64_t n, int64_t nsys, const int64_t* soff,
-                      const unsigned long long* ks, uint32_t* perm, unsigned long long* kin,
+                      unsigned long long* ks, uint32_t* perm, unsigned long long* kin,
                       uint32_t* ord, uint32_t* ord2, uint16_t* cls, uint32_t* fp,
-                      unsigned long long* fec, DevScalars* sc);
+                      unsigned long long* fec, uint32_t* list, const DevBox* boxes, double4* rec,
+                      DevScalars* sc);
 // out[perm[i]] = in[i] (back to input order)
 void launch_scatter_back(hipStream_t s, int64_t n, const uint32_t* perm, const double* in,
                          double* out);
@@ -115,10 +118,6 @@ struct TreeBuffers {
 
 void launch_dup_detect(hipStream_t s, int64_t n, const unsigned long long* keys, const uint32_t* sys,
                        DevScalars* sc);
-void launch_dupfix(hipStream_t s, int64_t n, unsigned long long* keys, double* x, double* y,
-                   double* z, const DevBox* boxes, const uint32_t* sys, const int64_t* soff,
-                   long long* kd, unsigned long long* oldkeys, uint32_t* dflag, uint32_t* dlist,
-                   uint32_t* bsum, DevScalars* sc);
 void launch_tree_build(hipStream_t s, const TreeBuffers& t, int group_size, int group_pack);
 int64_t bfs_table_words(int64_t n);   // enough for every tree of at most n particles
 void launch_leaf_moments(hipStream_t s, const TreeBuffers& t);

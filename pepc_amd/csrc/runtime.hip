@@ -37,13 +37,12 @@ struct Ctx {
 
   // particles
   double *in[4] = {nullptr, nullptr, nullptr, nullptr};   // host-path input copies
-  unsigned long long *k0 = nullptr, *k1 = nullptr, *oldkeys = nullptr;
+  unsigned long long *k0 = nullptr, *k1 = nullptr, *tie_ent = nullptr;
   uint32_t *v0 = nullptr, *v1 = nullptr;
   double *xs = nullptr, *ys = nullptr, *zs = nullptr, *qs = nullptr;
   double4* prec4 = nullptr;         // {x, y, z, q} records, input order
   uint8_t *lo = nullptr, *hi = nullptr;
-  uint32_t *cnt = nullptr, *gmark = nullptr, *dflag = nullptr, *dlist = nullptr;
-  long long* kd = nullptr;
+  uint32_t *cnt = nullptr, *gmark = nullptr, *tie_pos = nullptr, *dlist = nullptr;
   uint32_t *gfirst = nullptr, *gcount = nullptr, *gstat = nullptr, *queue = nullptr;
   uint32_t *np2p = nullptr, *nm2p = nullptr;
   double *res[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};   // host-path outputs
@@ -247,9 +246,9 @@ int dalloc(Ctx* c, T** p, int64_t count) {
   } while (0)
 
 void free_all(Ctx* c) {
-  void* ptrs[] = {c->in[0], c->in[1], c->in[2], c->in[3], c->k0, c->k1, c->oldkeys, c->v0, c->v1,
-                  c->xs, c->ys, c->zs, c->qs, c->lo, c->hi, c->cnt, c->gmark, c->dflag, c->dlist,
-                  c->kd, c->gfirst, c->gcount, c->gstat, c->queue, c->np2p, c->nm2p, c->res[0], c->res[1],
+  void* ptrs[] = {c->in[0], c->in[1], c->in[2], c->in[3], c->k0, c->k1, c->tie_ent, c->v0, c->v1,
+                  c->xs, c->ys, c->zs, c->qs, c->lo, c->hi, c->cnt, c->gmark, c->tie_pos, c->dlist,
+                  c->gfirst, c->gcount, c->gstat, c->queue, c->np2p, c->nm2p, c->res[0], c->res[1],
                   c->res[2], c->res[3], c->res[4], c->tab, c->ntype, c->kidtwig,
                   c->fc_rank, c->node_rank, c->nfirst, c->link, c->geom,
                   c->mom64, c->wm32, c->wm64, c->hist, c->bsum, c->partial, c->box, c->sc,
@@ -316,13 +315,12 @@ int ensure_particles(Ctx* c, int64_t n) {
     return fail(c, PEPC_GPU_EINVAL, "node pool of node_factor * n nodes exceeds 31-bit node indices");
   if (mc < c->node_min) mc = c->node_min;
   if (mc < nc) mc = nc;   // every particle is a leaf (and the grow borrows node arrays of n entries)
-  ALLOC(c, c->k0, nc); ALLOC(c, c->k1, nc); ALLOC(c, c->oldkeys, nc);
+  ALLOC(c, c->k0, nc); ALLOC(c, c->k1, nc); ALLOC(c, c->tie_ent, nc);
   ALLOC(c, c->v0, nc); ALLOC(c, c->v1, nc);
   ALLOC(c, c->xs, nc); ALLOC(c, c->ys, nc); ALLOC(c, c->zs, nc); ALLOC(c, c->qs, nc);
   ALLOC(c, c->prec4, nc);
   ALLOC(c, c->lo, nc); ALLOC(c, c->hi, nc);
-  ALLOC(c, c->cnt, nc); ALLOC(c, c->gmark, nc); ALLOC(c, c->dflag, nc); ALLOC(c, c->dlist, nc);
-  ALLOC(c, c->kd, nc);
+  ALLOC(c, c->cnt, nc); ALLOC(c, c->gmark, nc); ALLOC(c, c->tie_pos, nc); ALLOC(c, c->dlist, nc);
   ALLOC(c, c->gfirst, nc); ALLOC(c, c->gcount, nc); ALLOC(c, c->gstat, 8 * nc);
   ALLOC(c, c->sys, nc);
   ALLOC(c, c->np2p, nc); ALLOC(c, c->nm2p, nc);
@@ -435,15 +433,13 @@ int grow_device_impl(Ctx* c, int64_t n, const double* x, const double* y, const 
   launch_keys(s, n, x, y, z, q, c->box, sys, c->k0, c->v0, c->prec4);
   launch_sort_keys(s, c->k0, c->v0, c->k1, c->v1, n, c->hist, c->bsum, sys, nsys);
   launch_dup_detect(s, n, c->k0, sys, c->sc);
-  // equal keys into the reference presort's order (the sort's ping-pong
-  // buffers, the group scratch arrays and the duplicate fix-up's arrays,
-  // all written afresh before their own use, are free here)
+  // equal keys into the reference presort's order and apart (the sort's
+  // ping-pong buffers and the group scratch arrays, all written afresh before
+  // their own use, are free here)
   launch_tie_order(s, n, nsys, c->soff, c->k0, c->v0, c->k1, c->v1, c->cnt,
-                   reinterpret_cast<uint16_t*>(c->gmark), c->dflag,
-                   reinterpret_cast<unsigned long long*>(c->kd), c->sc);
+                   reinterpret_cast<uint16_t*>(c->gmark), c->tie_pos, c->tie_ent, c->dlist, c->box,
+                   c->prec4, c->sc);
   launch_gather_rec(s, n, c->v0, c->prec4, c->xs, c->ys, c->zs, c->qs);
-  launch_dupfix(s, n, c->k0, c->xs, c->ys, c->zs, c->box, sys, nsys > 1 ? c->soff : nullptr, c->kd,
-                c->oldkeys, c->dflag, c->dlist, c->bsum, c->sc);
   TreeBuffers t;
   t.n = n;
   t.cap = c->mcap;

@@ -44,18 +44,10 @@ __device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t v, uint32_t* t
   return off + inc - v;
 }
 
-// With ndev != nullptr the scanned length is min(n, *ndev), read on the
-// device (n only sizes the grid); entries past it are neither read nor written.
-__device__ __forceinline__ int64_t scan_len(int64_t n, const uint32_t* ndev) {
-  return (ndev && (int64_t)*ndev < n) ? (int64_t)*ndev : n;
-}
-
 __global__ __launch_bounds__(kScanThreads) void scan_reduce_kernel(const uint32_t* __restrict__ in,
                                                                     int64_t n,
                                                                     uint32_t* __restrict__ bsum,
-                                                                    const uint32_t* __restrict__ ndev,
                                                                     bool flags) {
-  n = scan_len(n, ndev);
   const int64_t base = (int64_t)blockIdx.x * kScanTile;
   uint32_t s = 0;
 #pragma unroll
@@ -93,10 +85,8 @@ __global__ __launch_bounds__(kScanThreads) void scan_apply_kernel(const uint32_t
                                                                    uint32_t* __restrict__ out,
                                                                    int64_t n,
                                                                    const uint32_t* __restrict__ bsum,
-                                                                   const uint32_t* __restrict__ ndev,
                                                                    bool flags) {
   __shared__ uint32_t tile[kScanTile];
-  n = scan_len(n, ndev);
   const int64_t base = (int64_t)blockIdx.x * kScanTile;
   if (base >= n) return;   // uniform over the block
 #pragma unroll
@@ -500,17 +490,133 @@ __global__ __launch_bounds__(256) void sort_fields_kernel(
 // that hold a tie, and writes the final order of each such bucket into the
 // permutation.  Runs only when the sort left equal adjacent keys (dup_count
 // from dup_detect); one block per system.
+//
+// The equal keys are then moved apart in the same launch (fix_duplicates), so
+// a system without any pays for one launch that returns at once; with the
+// fix-up in seven more launches a solve of 32,768 particles took 411 us in
+// place of 388, one of 1,777 particles 326 in place of 311.  With equal keys
+// the steps are a chain of memory accesses, so a wave looks for the gaps: a
+// third of 1,777 particles at one point took 62 ms with one thread, 8 with it.
 constexpr int kTieThreads = 256;
 constexpr int kTieWidth = 10;           // sl_tune_intern.h:22 (sort_radix_width_default)
 constexpr int kTieThreshold = 256;      // sl_tune_intern.h:30 (sort_radix_threshold_rec)
 constexpr int kTieClasses = 1 << kTieWidth;
 constexpr int kTieDepth = 8;            // 64 bits in 10-bit digits: at most 7 passes
 
+// key_to_intcoord_hilbert / key_to_coord, module_spacefilling.f90:445-565.
+constexpr int kC3[8] = {0, 1, 3, 2, 6, 7, 5, 4};
+constexpr int kGX[8] = {5, 6, 0, 5, 5, 0, 6, 5};
+constexpr int kGR[8] = {0, 0, 0, 5, 0, 0, 6, 5};
+
+__device__ void key_to_intcoord(unsigned long long key, long long ic[3]) {
+  const int lev = level_of_key(key);
+  ic[0] = ic[1] = ic[2] = 0;
+  for (int i = 0; i < lev; ++i) {
+    const int h = (int)((key >> (3 * i)) & 7ull);
+    const int cval = kC3[h], rev = kGR[h], ex = kGX[h];
+    if (i > 0) {
+      for (int j = 0; j < 3; ++j)
+        if ((rev >> j) & 1) ic[j] = (~ic[j]) & ((1ll << i) - 1);
+      for (int j = 0; j < 2; ++j) {
+        if (!((ex >> j) & 1)) continue;
+        for (int k = j + 1; k < 3; ++k)
+          if ((ex >> k) & 1) { long long t = ic[j]; ic[j] = ic[k]; ic[k] = t; }
+      }
+    }
+    for (int j = 0; j < 3; ++j) ic[j] |= (long long)((cval >> j) & 1) << i;
+  }
+  for (int j = 0; j < 3; ++j) ic[j] <<= (kMaxLevel - lev);
+}
+
+// module_domains.f90:248-297 for one system of n particles (keys ks[0..n)),
+// in the reference's loop order, by one wave: it visits the nd positions of
+// list, those that start with a successor of the same key.  Only they are
+// ever modified to a smaller key difference, so this equals visiting every
+// position.  The reference's table of key differences kd(i) always equals
+// ks[i] - ks[i - 1] (1-based i; 1 at the last position, which no step reads),
+// so the keys stand for it.  A step's search for the nearest gap and its
+// shift take 64 positions at a time; the steps themselves are a chain.
+// lo/hi[r] keep the positions that step r moved.
+constexpr int kDupNear = 4;
+
+__device__ void dup_serial(long long n, unsigned long long* ks, const uint32_t* list, uint32_t nd,
+                           uint32_t* lo, uint32_t* hi, DevScalars* sc) {
+  const int lane = lane_id();
+  const bool full = (long long)(ks[n - 1] - ks[0]) + 1 < n;   // :254-262
+  if (full && lane == 0) atomicOr(&sc->flags, kFlagDupKeys);
+  uint32_t pos = 0, mylo = 1, myhi = 0;   // lane l: of step l of 64
+  for (uint32_t r = 0; r < nd; ++r) {
+    const int l = (int)(r % kWave);
+    if (l == 0) pos = r + lane < nd ? list[r + lane] : 0u;
+    long long from = 1, to = 0;   // positions moved (0-based)
+    const long long i1 = (long long)__builtin_amdgcn_readlane((int)pos, l) + 1;   // 1-based as in the source
+    if (!full) {
+      const long long jmax = (n - i1) > i1 ? (n - i1) : i1;
+      // the step's own difference, loaded with the first gaps
+      const bool equal = (long long)(ks[i1] - ks[i1 - 1]) < 1;
+      // first a few gaps, which one or two cache lines hold
+      for (long long j0 = 1, w = kDupNear; j0 <= jmax; j0 += w, w = kWave) {
+        const long long j = j0 + (lane < w ? lane : 0);
+        const bool has_dn = i1 - j >= 1, has_up = i1 + j <= n - 1;
+        const long long dn = has_dn ? i1 - j : 1, up = has_up ? i1 + j : 1;
+        const unsigned long long kd1 = ks[dn], kd0 = ks[dn - 1], ku1 = ks[up], ku0 = ks[up - 1];
+        if (!equal) break;
+        const bool down = has_dn && (long long)(kd1 - kd0) > 1;
+        const bool hit = down || (has_up && (long long)(ku1 - ku0) > 1);
+        const unsigned long long m = __ballot(hit);
+        if (m) {
+          const int first = __ffsll(m) - 1;
+          const bool d = (__ballot(down) >> first) & 1ull;
+          from = d ? i1 - (j0 + first) : i1;
+          to = d ? i1 - 1 : i1 + (j0 + first) - 1;
+          const unsigned long long by = d ? ~0ull : 1ull;   // -1 or +1
+          for (long long t = from + lane; t <= to; t += kWave) ks[t] += by;
+          break;
+        }
+      }
+      // the next step's loads in every lane see this step's stores
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+    }
+    if (lane == l) { mylo = (uint32_t)from; myhi = (uint32_t)to; }
+    if (l == kWave - 1 || r + 1 == nd) {
+      const uint32_t at = r - l + lane;
+      if (at < nd) { lo[at] = mylo; hi[at] = myhi; }
+    }
+  }
+}
+
+// The system's particles [b, e): moves equal keys apart and puts every
+// particle whose key changed (kin holds the keys in input order) at its new
+// key's cell centre, in the records that the sorted particles are taken from.
+// list[0..nd): the duplicates' positions in [b, e), increasing.  The steps'
+// ranges are usually a position or two, so each thread replays whole steps.
+__device__ void fix_duplicates(int64_t b, int64_t e, unsigned long long* ks, const uint32_t* perm,
+                               const unsigned long long* kin, const uint32_t* list, uint32_t nd,
+                               uint32_t* lo, uint32_t* hi, const DevBox* box, double4* rec,
+                               DevScalars* sc) {
+  __syncthreads();
+  if (threadIdx.x < kWave) dup_serial(e - b, ks + b, list, nd, lo, hi, sc);
+  __syncthreads();
+  for (uint32_t r = threadIdx.x; r < nd; r += blockDim.x) {
+    for (int64_t t = lo[r]; t <= (int64_t)hi[r]; ++t) {
+      const unsigned long long key = ks[b + t];
+      const uint32_t p = perm[b + t];
+      if (key == kin[p]) continue;
+      long long ic[3];
+      key_to_intcoord(key, ic);
+      rec[p].x = ((double)ic[0] + 0.5) * box->cell[0] + box->boxmin[0];
+      rec[p].y = ((double)ic[1] + 0.5) * box->cell[1] + box->boxmin[1];
+      rec[p].z = ((double)ic[2] + 0.5) * box->cell[2] + box->boxmin[2];
+    }
+  }
+}
+
 __global__ __launch_bounds__(kTieThreads) void tie_order_kernel(
-    int64_t n, const int64_t* __restrict__ soff, const unsigned long long* __restrict__ ks,
-    uint32_t* __restrict__ perm, unsigned long long* __restrict__ kin, uint32_t* __restrict__ ord,
-    uint32_t* __restrict__ ord2, uint16_t* __restrict__ cls, uint32_t* __restrict__ fp,
-    unsigned long long* __restrict__ fec, DevScalars* __restrict__ sc) {
+    int64_t n, const int64_t* __restrict__ soff, unsigned long long* ks, uint32_t* perm,
+    unsigned long long* kin, uint32_t* ord, uint32_t* ord2, uint16_t* __restrict__ cls,
+    uint32_t* __restrict__ fp, unsigned long long* __restrict__ fec, uint32_t* list,
+    const DevBox* __restrict__ boxes, double4* rec, DevScalars* __restrict__ sc) {
   if (sc->dup_count == 0) return;
   const int tid = threadIdx.x;
   const int64_t b = soff ? soff[blockIdx.x] : 0;
@@ -523,15 +629,36 @@ __global__ __launch_bounds__(kTieThreads) void tie_order_kernel(
   __shared__ unsigned long long skey[kTieThreshold];
   __shared__ int64_t fs[kTieDepth], fe[kTieDepth], fcur[kTieDepth];
   __shared__ int frh[kTieDepth], fnext[kTieDepth];
-  __shared__ int depth, any;
+  __shared__ int depth;
   __shared__ int64_t found;
 
-  if (tid == 0) any = 0;
+  // the positions with a successor of the same key, in increasing order
+  list += b;
+  if (tid == 0) run_base = 0;
   __syncthreads();
-  for (int64_t i = b + tid; i + 1 < e; i += kTieThreads)
-    if (ks[i + 1] == ks[i]) any = 1;
+  {
+    constexpr int kPer = 8;   // consecutive positions per thread per chunk
+    for (int64_t base = b; base + 1 < e; base += (int64_t)kTieThreads * kPer) {
+      const int64_t i0 = base + (int64_t)tid * kPer;
+      unsigned long long k[kPer + 1];
+#pragma unroll
+      for (int j = 0; j <= kPer; ++j) k[j] = i0 + j < e ? ks[i0 + j] : 0ull;
+      uint32_t nf = 0;
+#pragma unroll
+      for (int j = 0; j < kPer; ++j) nf += i0 + j + 1 < e && k[j + 1] == k[j] ? 1u : 0u;
+      uint32_t tot;
+      uint32_t off = run_base + block_exclusive_scan(nf, &tot);
+#pragma unroll
+      for (int j = 0; j < kPer; ++j)
+        if (i0 + j + 1 < e && k[j + 1] == k[j]) list[off++] = (uint32_t)(i0 + j - b);
+      __syncthreads();
+      if (tid == 0) run_base += tot;
+      __syncthreads();
+    }
+  }
+  const uint32_t nd = run_base;   // replaced by the passes below
   __syncthreads();
-  if (!any) return;
+  if (nd == 0) return;
 
   // keys in input order (the sort's input of this system is [b, e) too) and
   // the initial order of the top segment
@@ -746,29 +873,33 @@ __global__ __launch_bounds__(kTieThreads) void tie_order_kernel(
     }
     __syncthreads();
   }
+  fix_duplicates(b, e, ks, perm, kin, list, nd, ord + b, ord2 + b, boxes + (soff ? blockIdx.x : 0),
+                 rec, sc);
 }
 
 }  // namespace
 
 void launch_tie_order(hipStream_t s, int64_t n, int64_t nsys, const int64_t* soff,
-                      const unsigned long long* ks, uint32_t* perm, unsigned long long* kin,
+                      unsigned long long* ks, uint32_t* perm, unsigned long long* kin,
                       uint32_t* ord, uint32_t* ord2, uint16_t* cls, uint32_t* fp,
-                      unsigned long long* fec, DevScalars* sc) {
+                      unsigned long long* fec, uint32_t* list, const DevBox* boxes, double4* rec,
+                      DevScalars* sc) {
   if (n < 2) return;
   tie_order_kernel<<<(unsigned)(nsys > 1 ? nsys : 1), kTieThreads, 0, s>>>(
-      n, nsys > 1 ? soff : nullptr, ks, perm, kin, ord, ord2, cls, fp, fec, sc);
+      n, nsys > 1 ? soff : nullptr, ks, perm, kin, ord, ord2, cls, fp, fec, list, boxes,
+      rec, sc);
 }
 
 int64_t scan_blocks(int64_t n) { return (n + kScanTile - 1) / kScanTile; }
 int64_t sort_blocks(int64_t n) { return (n + kSortTile - 1) / kSortTile; }
 
 void launch_scan(hipStream_t s, const uint32_t* in, uint32_t* out, int64_t n, uint32_t* bsum,
-                 uint32_t* total, const uint32_t* ndev, bool flags) {
+                 uint32_t* total, bool flags) {
   if (n <= 0) return;
   const int64_t nb = scan_blocks(n);
-  scan_reduce_kernel<<<(unsigned)nb, kScanThreads, 0, s>>>(in, n, bsum, ndev, flags);
+  scan_reduce_kernel<<<(unsigned)nb, kScanThreads, 0, s>>>(in, n, bsum, flags);
   scan_small_kernel<<<1, kScanThreads, 0, s>>>(bsum, (int)nb, total);
-  scan_apply_kernel<<<(unsigned)nb, kScanThreads, 0, s>>>(in, out, n, bsum, ndev, flags);
+  scan_apply_kernel<<<(unsigned)nb, kScanThreads, 0, s>>>(in, out, n, bsum, flags);
 }
 
 // One stable pass over bits [shift, shift + nbits), output in (kout, vout).

@@ -54,125 +54,6 @@ __global__ void dup_detect_kernel(int64_t n, const unsigned long long* __restric
   if (lane_id() == 0 && c) atomicAdd(&sc->dup_count, c);
 }
 
-__global__ void dup_prepare_kernel(int64_t n, const unsigned long long* __restrict__ keys,
-                                   const uint32_t* __restrict__ sys,
-                                   long long* __restrict__ kd, unsigned long long* __restrict__ old,
-                                   uint32_t* __restrict__ flag, DevScalars* __restrict__ sc) {
-  if (blockIdx.x == 0 && threadIdx.x == 0) sc->dup_scan_n = sc->dup_count ? (uint32_t)n : 0u;
-  if (sc->dup_count == 0) return;
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    // the last particle of a range behaves as the last particle of a rank
-    long long d = (i + 1 < n && same_sys(sys, i, i + 1)) ? (long long)(keys[i + 1] - keys[i]) : 1ll;
-    kd[i] = d;
-    old[i] = keys[i];
-    flag[i] = d < 1 ? 1u : 0u;
-  }
-}
-
-__global__ void dup_compact_kernel(int64_t n, const long long* __restrict__ kd,
-                                   const uint32_t* __restrict__ rank, uint32_t* __restrict__ list,
-                                   const DevScalars* __restrict__ sc) {
-  if (sc->dup_count == 0) return;
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x)
-    if (kd[i] < 1) list[rank[i]] = (uint32_t)i;
-}
-
-// module_domains.f90:248-297, one thread, in the reference's loop order.
-// Only positions that start as duplicates are ever modified to a smaller
-// key difference, so visiting the compacted list in order equals visiting
-// every position.  With batched systems the loop runs on each system's range
-// (base pointer and length of that range), systems in increasing order.
-__global__ void dup_serial_kernel(int64_t n_all, unsigned long long* __restrict__ keys_all,
-                                  long long* __restrict__ kd_all, const uint32_t* __restrict__ list,
-                                  const uint32_t* __restrict__ sys, const int64_t* __restrict__ soff,
-                                  DevScalars* __restrict__ sc) {
-  const uint32_t nd = sc->dup_count;
-  if (nd == 0 || threadIdx.x != 0) return;
-  int64_t cur = -1;
-  long long n = n_all;
-  unsigned long long* keys = keys_all;
-  long long* kd = kd_all;
-  for (uint32_t r = 0; r < nd; ++r) {
-    const int64_t gi = list[r];
-    const int64_t sid = sys ? (int64_t)sys[gi] : 0;
-    if (sid != cur) {
-      cur = sid;
-      const int64_t b = sys ? soff[sid] : 0;
-      n = sys ? (long long)(soff[sid + 1] - b) : n_all;
-      keys = keys_all + b;
-      kd = kd_all + b;
-      if ((long long)(keys[n - 1] - keys[0]) + 1 < n) {   // :254-262
-        atomicOr(&sc->flags, kFlagDupKeys);
-        return;
-      }
-    }
-    const long long i1 = (long long)(gi - (keys - keys_all)) + 1;   // 1-based as in the source
-    if (kd[i1 - 1] >= 1) continue;
-    const long long jmax = (n - i1) > i1 ? (n - i1) : i1;
-    for (long long j = 1; j <= jmax; ++j) {
-      const long long dn = i1 - j < 1 ? 1 : i1 - j;
-      const long long up = i1 + j < n - 1 ? i1 + j : n - 1;
-      if (kd[dn - 1] > 1 && i1 - j >= 1) {
-        for (long long t = i1 - j + 1; t <= i1; ++t) keys[t - 1] -= 1ull;
-        kd[i1 - 1] += 1;
-        kd[i1 - j - 1] -= 1;
-        break;
-      } else if (kd[up - 1] > 1 && i1 + j <= n - 1) {
-        for (long long t = i1 + 1; t <= i1 + j; ++t) keys[t - 1] += 1ull;
-        kd[i1 - 1] += 1;
-        kd[i1 + j - 1] -= 1;
-        break;
-      }
-    }
-  }
-}
-
-// key_to_intcoord_hilbert / key_to_coord, module_spacefilling.f90:445-565.
-constexpr int kC3[8] = {0, 1, 3, 2, 6, 7, 5, 4};
-constexpr int kGX[8] = {5, 6, 0, 5, 5, 0, 6, 5};
-constexpr int kGR[8] = {0, 0, 0, 5, 0, 0, 6, 5};
-
-__device__ void key_to_intcoord(unsigned long long key, long long ic[3]) {
-  const int lev = level_of_key(key);
-  ic[0] = ic[1] = ic[2] = 0;
-  for (int i = 0; i < lev; ++i) {
-    const int h = (int)((key >> (3 * i)) & 7ull);
-    const int cval = kC3[h], rev = kGR[h], ex = kGX[h];
-    if (i > 0) {
-      for (int j = 0; j < 3; ++j)
-        if ((rev >> j) & 1) ic[j] = (~ic[j]) & ((1ll << i) - 1);
-      for (int j = 0; j < 2; ++j) {
-        if (!((ex >> j) & 1)) continue;
-        for (int k = j + 1; k < 3; ++k)
-          if ((ex >> k) & 1) { long long t = ic[j]; ic[j] = ic[k]; ic[k] = t; }
-      }
-    }
-    for (int j = 0; j < 3; ++j) ic[j] |= (long long)((cval >> j) & 1) << i;
-  }
-  for (int j = 0; j < 3; ++j) ic[j] <<= (kMaxLevel - lev);
-}
-
-__global__ void dup_recoord_kernel(int64_t n, const unsigned long long* __restrict__ keys,
-                                   const unsigned long long* __restrict__ old,
-                                   double* __restrict__ x, double* __restrict__ y,
-                                   double* __restrict__ z, const DevBox* __restrict__ boxes,
-                                   const uint32_t* __restrict__ sys,
-                                   const DevScalars* __restrict__ sc) {
-  if (sc->dup_count == 0) return;
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    if (keys[i] == old[i]) continue;
-    const DevBox* __restrict__ box = boxes + (sys ? sys[i] : 0u);
-    long long ic[3];
-    key_to_intcoord(keys[i], ic);
-    x[i] = ((double)ic[0] + 0.5) * box->cell[0] + box->boxmin[0];
-    y[i] = ((double)ic[1] + 0.5) * box->cell[1] + box->boxmin[1];
-    z[i] = ((double)ic[2] + 0.5) * box->cell[2] + box->boxmin[2];
-  }
-}
-
 // ------------------------------------------------------------ build
 // Every kernel after the node count is known bails out once an earlier stage
 // raised a flag that makes the node arrays inconsistent, so no index read
@@ -1051,17 +932,6 @@ void launch_dup_detect(hipStream_t s, int64_t n, const unsigned long long* keys,
   dup_detect_kernel<<<grid_for(n), kT, 0, s>>>(n, keys, sys, sc);
 }
 
-void launch_dupfix(hipStream_t s, int64_t n, unsigned long long* keys, double* x, double* y,
-                   double* z, const DevBox* boxes, const uint32_t* sys, const int64_t* soff,
-                   long long* kd, unsigned long long* oldkeys, uint32_t* dflag, uint32_t* dlist,
-                   uint32_t* bsum, DevScalars* sc) {
-  dup_prepare_kernel<<<grid_for(n), kT, 0, s>>>(n, keys, sys, kd, oldkeys, dflag, sc);
-  launch_scan(s, dflag, dflag, n, bsum, nullptr, &sc->dup_scan_n);
-  dup_compact_kernel<<<grid_for(n), kT, 0, s>>>(n, kd, dflag, dlist, sc);
-  dup_serial_kernel<<<1, 1, 0, s>>>(n, keys, kd, dlist, sys, soff, sc);
-  dup_recoord_kernel<<<grid_for(n), kT, 0, s>>>(n, keys, oldkeys, x, y, z, boxes, sys, sc);
-}
-
 int64_t bfs_tiles(int64_t n) {
   const int64_t b = (n + bfs_tile(n) - 1) / bfs_tile(n);
   return b < 1 ? 1 : b;
@@ -1086,7 +956,7 @@ void launch_tree_build(hipStream_t s, const TreeBuffers& t, int group_size, int 
   launch_upward(s, t);
   group_mark_kernel<<<grid_for(n), kT, 0, s>>>(group_size, group_pack, t.link, t.nfirst, t.node_rank,
                                                t.gmark, t.sc);
-  launch_scan(s, t.gmark, t.cnt, n, t.bsum, &t.sc->ngroups, nullptr, true);
+  launch_scan(s, t.gmark, t.cnt, n, t.bsum, &t.sc->ngroups, true);
   group_emit_kernel<<<grid_for(n), kT, 0, s>>>(n, t.gmark, t.cnt, t.gfirst, t.gcount);
   if (t.sys) sysroot_kernel<<<grid_for(t.nsys), kT, 0, s>>>(t.sys, t.nfirst, t.sysroot, t.sc);
 }
