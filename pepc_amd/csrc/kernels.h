@@ -6,15 +6,15 @@
 namespace pepc {
 
 // keys.hip
-int box_partial_blocks(int64_t n);
 constexpr int kBoxPartial = 7;   // doubles per block of launch_box's partial results
-void launch_box(hipStream_t s, int64_t n, const double* x, const double* y, const double* z,
-                const double* q, int force_cubic, double* partial, DevBox* box, DevScalars* sc);
-// Batched systems: per-system boxes over the ranges [soff[s], soff[s+1]) and
-// the system index of every particle.
-void launch_box_batch(hipStream_t s, int nsys, const int64_t* soff, const double* x,
-                      const double* y, const double* z, const double* q, int force_cubic,
-                      DevBox* boxes, uint32_t* sys, DevScalars* sc);
+constexpr int kBoxParts = 4096;  // blocks of launch_box with partial results
+// Boxes of nsys systems (soff: their ranges when nsys > 1; sys then gets the
+// system index of every particle).  One system: also clears the scalars; a
+// batch needs them cleared before.  partial: kBoxParts * kBoxPartial doubles,
+// tickets: kBoxParts words, zero between calls.
+void launch_box(hipStream_t s, int64_t n, int nsys, const int64_t* soff, const double* x,
+                const double* y, const double* z, const double* q, int force_cubic,
+                double* partial, uint32_t* tickets, DevBox* boxes, uint32_t* sys, DevScalars* sc);
 // sys == nullptr: one system with boxes[0].
 // Also writes rec[i] = {x, y, z, q} (input order) for launch_gather_rec.
 void launch_keys(hipStream_t s, int64_t n, const double* x, const double* y, const double* z,
@@ -31,10 +31,13 @@ void launch_sink_groups(hipStream_t s, int64_t m, int g, uint32_t* gfirst, uint3
 int64_t scan_blocks(int64_t n);
 int64_t sort_blocks(int64_t n);
 // Exclusive scan of n values (in place allowed); *total gets the sum when
-// total != nullptr.  With flags, each value counts as 1 when nonzero and 0
-// otherwise.
+// total != nullptr.
 void launch_scan(hipStream_t s, const uint32_t* in, uint32_t* out, int64_t n, uint32_t* bsum,
-                 uint32_t* total, bool flags = false);
+                 uint32_t* total);
+// Group g is the g-th nonzero mark: gfirst[g] its particle, gcount[g] its
+// value; *ngroups their number.
+void launch_group_list(hipStream_t s, int64_t n, const uint32_t* gmark, uint32_t* bsum,
+                       uint32_t* gfirst, uint32_t* gcount, uint32_t* ngroups);
 void launch_radix_pass(hipStream_t s, const unsigned long long* kin, const uint32_t* vin,
                        unsigned long long* kout, uint32_t* vout, int64_t n, int shift, int nbits,
                        uint32_t* hist, uint32_t* bsum);
@@ -87,7 +90,6 @@ struct TreeBuffers {
   const double *x, *y, *z, *q;       // sorted particles
   uint8_t* lo;                       // L(a): level of the first node of particle a
   uint8_t* hi;                       // leaf level of particle a
-  uint32_t* cnt;                     // per-particle scratch (group marks -> group ranks)
   uint32_t* tab;                     // (level, tile) node and twig counts and their scans, bfs_table_words(n)
   uint32_t* fc_rank;                 // first child by twig rank (+1 sentinel)
   uint32_t* node_rank;               // node index by twig rank
@@ -161,13 +163,16 @@ struct WalkArgs {
   const double *tx = nullptr, *ty = nullptr, *tz = nullptr;
   uint32_t nsink_groups = 0;
 };
-void launch_walk_reset(hipStream_t s, const WalkArgs& a);
 // Work queues of the persistent walk: up to kMaxQueues heads, each on a
 // 64-byte line of its own (kQueueWords words in all).
 constexpr int kMaxQueues = 8;
 constexpr int kQueueStride = 16;
 constexpr int kQueueWords = kMaxQueues * kQueueStride;
-void launch_queue_reset(hipStream_t s, uint32_t* queue);   // work-queue heads only
+// Zeroes n words.  The work-queue heads are zero between walks: launch_walk_stats
+// leaves them so, and a walk of sinks is followed by this.
+void launch_zero_words(hipStream_t s, uint32_t* words, int n);
+// dst (pinned host memory) = src
+void launch_publish(hipStream_t s, const DevScalars* src, DevScalars* dst);
 // list_tile: M2P list capacity in LDS (0 = default: 64 FP32, 32 FP64;
 // FP32 takes 64 or 128, FP64 32 or 64).
 bool walk_list_tile_ok(int precision, int list_tile);

@@ -18,62 +18,26 @@ constexpr int kBoxThreads = 256;
 __device__ __forceinline__ uint32_t charge_sign(double q) {
   return (!(q <= 0.0) ? kQPositive : 0u) | (!(q >= 0.0) ? kQNegative : 0u);
 }
+// A coordinate that is not finite, beside the sign bits.
+constexpr uint32_t kBoxNonfinite = 4u;
+static_assert(((kQPositive | kQNegative) & kBoxNonfinite) == 0u, "bits of their own");
 // The bits over a wave, the same in every lane.
 __device__ __forceinline__ uint32_t wave_sign(uint32_t s) {
-  return (__ballot(s & kQPositive) ? kQPositive : 0u) | (__ballot(s & kQNegative) ? kQNegative : 0u);
-}
-
-__global__ __launch_bounds__(kBoxThreads) void box_partial_kernel(
-    int64_t n, const double* __restrict__ x, const double* __restrict__ y,
-    const double* __restrict__ z, const double* __restrict__ q, double* __restrict__ partial,
-    DevScalars* __restrict__ sc) {
-  double mn[3] = {INFINITY, INFINITY, INFINITY};
-  double mx[3] = {-INFINITY, -INFINITY, -INFINITY};
-  bool nonfinite = false;
-  uint32_t sign = 0u;
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    double v0 = x[i], v1 = y[i], v2 = z[i];
-    nonfinite |= !isfinite(v0) || !isfinite(v1) || !isfinite(v2);
-    mn[0] = fmin(mn[0], v0); mx[0] = fmax(mx[0], v0);
-    mn[1] = fmin(mn[1], v1); mx[1] = fmax(mx[1], v1);
-    mn[2] = fmin(mn[2], v2); mx[2] = fmax(mx[2], v2);
-    sign |= charge_sign(q[i]);
-  }
-  if (__ballot(nonfinite) != 0ull && lane_id() == 0) atomicOr(&sc->flags, kFlagBadBox);
-  __shared__ double red[6][kBoxThreads / kWave];
-  __shared__ uint32_t rsign[kBoxThreads / kWave];
-  const int w = threadIdx.x / kWave;
-  sign = wave_sign(sign);
-  if (lane_id() == 0) rsign[w] = sign;
-#pragma unroll
-  for (int d = 0; d < 3; ++d) {
-    double a = wave_min(mn[d]), b = wave_max(mx[d]);
-    if (lane_id() == 0) { red[d][w] = a; red[3 + d][w] = b; }
-  }
-  __syncthreads();
-  if (threadIdx.x < 6) {
-    const int d = threadIdx.x;
-    double v = red[d][0];
-    for (int k = 1; k < kBoxThreads / kWave; ++k) v = d < 3 ? fmin(v, red[d][k]) : fmax(v, red[d][k]);
-    partial[blockIdx.x * kBoxPartial + d] = v;
-  } else if (threadIdx.x == 6) {   // the sign bits as a small whole number
-    uint32_t v = rsign[0];
-    for (int k = 1; k < kBoxThreads / kWave; ++k) v |= rsign[k];
-    partial[blockIdx.x * kBoxPartial + 6] = (double)v;
-  }
+  return (__ballot(s & kQPositive) ? kQPositive : 0u) |
+         (__ballot(s & kQNegative) ? kQNegative : 0u) |
+         (__ballot(s & kBoxNonfinite) ? kBoxNonfinite : 0u);
 }
 
 // module_box.f90:65-93 from the coordinate extrema: optional cube, margin
 // boxsize/10000 on both sides, refinement cell, boxlength2 table.
-__device__ void box_finalize(double mn[3], double mx[3], uint32_t qsign, int force_cubic,
+__device__ void box_finalize(double mn[3], double mx[3], uint32_t sign, int force_cubic,
                              DevBox* __restrict__ box, DevScalars* __restrict__ sc) {
   if (force_cubic) {  // module_box.f90:71-74
     double lo = fmin(fmin(mn[0], mn[1]), mn[2]);
     double hi = fmax(fmax(mx[0], mx[1]), mx[2]);
     for (int d = 0; d < 3; ++d) { mn[d] = lo; mx[d] = hi; }
   }
-  bool bad = false;
+  bool bad = (sign & kBoxNonfinite) != 0u;
   for (int d = 0; d < 3; ++d) {
     double size0 = mx[d] - mn[d];
     double lo = mn[d] - size0 / 10000.0;
@@ -87,55 +51,43 @@ __device__ void box_finalize(double mn[3], double mx[3], uint32_t qsign, int for
   double m = fmax(fmax(box->boxsize[0], box->boxsize[1]), box->boxsize[2]);
   box->b2[0] = m * m;
   for (int l = 1; l <= kMaxLevel; ++l) box->b2[l] = box->b2[l - 1] / 4.0;
-  box->qsign = qsign;
+  box->qsign = sign & (kQPositive | kQNegative);
   if (bad) atomicOr(&sc->flags, kFlagBadBox);
 }
 
-__global__ __launch_bounds__(kWave) void box_final_kernel(int nblocks, const double* __restrict__ partial,
-                                                         int force_cubic, DevBox* __restrict__ box,
-                                                         DevScalars* __restrict__ sc) {
-  double mn[3] = {INFINITY, INFINITY, INFINITY};
-  double mx[3] = {-INFINITY, -INFINITY, -INFINITY};
-  uint32_t sign = 0u;
-  for (int b = threadIdx.x; b < nblocks; b += kWave) {
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-      mn[d] = fmin(mn[d], partial[b * kBoxPartial + d]);
-      mx[d] = fmax(mx[d], partial[b * kBoxPartial + 3 + d]);
-    }
-    sign |= (uint32_t)partial[b * kBoxPartial + 6];
-  }
-  sign = wave_sign(sign);
-#pragma unroll
-  for (int d = 0; d < 3; ++d) { mn[d] = wave_min(mn[d]); mx[d] = wave_max(mx[d]); }
-  if (threadIdx.x != 0) return;
-  box_finalize(mn, mx, sign, force_cubic, box, sc);
-}
-
-// Batched systems: one block per system computes that system's box over its
-// particle range [soff[s], soff[s+1]) and tags the range with the system
-// index.  An empty system gets a unit box that no particle refers to.
-__global__ __launch_bounds__(kBoxThreads) void box_segment_kernel(
-    int nsys, const int64_t* __restrict__ soff, const double* __restrict__ x,
+// Bounding boxes, one launch: `parts` blocks per system reduce the system's
+// particles [soff[s], soff[s+1]) (the whole array without soff), and the block
+// that finishes a system last joins their results.  Extrema and sign bits do
+// not depend on the order of joining.  An empty system gets a unit box that
+// no particle refers to.  The results of other blocks, which may run on
+// another XCD, are published and read at device scope; tickets[s] counts the
+// system's finished blocks and is left at zero.
+// With clear, the scalars start from zero here (one system: its last block
+// writes them all).
+// Memory bound; for one system it is one launch in place of three (reset,
+// partial boxes, box), 2 us each, and a batch, which had one block per system,
+// spreads its largest systems: 256 systems of 1,024 to 65,536 particles
+// 148 -> 48 us.
+__global__ __launch_bounds__(kBoxThreads) void box_kernel(
+    int64_t n, int parts, const int64_t* __restrict__ soff, const double* __restrict__ x,
     const double* __restrict__ y, const double* __restrict__ z, const double* __restrict__ q,
-    int force_cubic, DevBox* __restrict__ boxes, uint32_t* __restrict__ sys,
-    DevScalars* __restrict__ sc) {
-  const int sid = blockIdx.x;
-  uint32_t sign = 0u;
-  const int64_t b = soff[sid], e = soff[sid + 1];
+    int force_cubic, double* partial, uint32_t* tickets, DevBox* __restrict__ boxes,
+    uint32_t* __restrict__ sys, DevScalars* __restrict__ sc, bool clear) {
+  const unsigned sid = blockIdx.x / (unsigned)parts, part = blockIdx.x % (unsigned)parts;
+  const int64_t b = soff ? soff[sid] : 0, e = soff ? soff[sid + 1] : n;
   double mn[3] = {INFINITY, INFINITY, INFINITY};
   double mx[3] = {-INFINITY, -INFINITY, -INFINITY};
-  bool nonfinite = false;
-  for (int64_t i = b + threadIdx.x; i < e; i += blockDim.x) {
+  uint32_t sign = 0u;   // DevBox::qsign bits and kBoxNonfinite
+  for (int64_t i = b + part * (int64_t)kBoxThreads + threadIdx.x; i < e;
+       i += (int64_t)parts * kBoxThreads) {
     double v0 = x[i], v1 = y[i], v2 = z[i];
-    nonfinite |= !isfinite(v0) || !isfinite(v1) || !isfinite(v2);
+    if (!isfinite(v0) || !isfinite(v1) || !isfinite(v2)) sign |= kBoxNonfinite;
     mn[0] = fmin(mn[0], v0); mx[0] = fmax(mx[0], v0);
     mn[1] = fmin(mn[1], v1); mx[1] = fmax(mx[1], v1);
     mn[2] = fmin(mn[2], v2); mx[2] = fmax(mx[2], v2);
-    sys[i] = (uint32_t)sid;
+    if (sys) sys[i] = sid;
     sign |= charge_sign(q[i]);
   }
-  if (__ballot(nonfinite) != 0ull && lane_id() == 0) atomicOr(&sc->flags, kFlagBadBox);
   __shared__ double red[6][kBoxThreads / kWave];
   __shared__ uint32_t rsign[kBoxThreads / kWave];
   const int w = threadIdx.x / kWave;
@@ -147,19 +99,59 @@ __global__ __launch_bounds__(kBoxThreads) void box_segment_kernel(
     if (lane_id() == 0) { red[d][w] = lo; red[3 + d][w] = hi; }
   }
   __syncthreads();
-  if (threadIdx.x != 0) return;
-  for (int d = 0; d < 3; ++d) {
-    mn[d] = red[d][0];
-    mx[d] = red[3 + d][0];
-    for (int k = 1; k < kBoxThreads / kWave; ++k) {
-      mn[d] = fmin(mn[d], red[d][k]);
-      mx[d] = fmax(mx[d], red[3 + d][k]);
+  if (w != 0) return;   // the rest is the first wave's
+  double v = 0.0;       // lane d < 6: extremum d; lane 6: the bits as a whole number
+  const int d = threadIdx.x;
+  if (d < 6) {
+    v = red[d][0];
+    for (int k = 1; k < kBoxThreads / kWave; ++k) v = d < 3 ? fmin(v, red[d][k]) : fmax(v, red[d][k]);
+  } else if (d == 6) {
+    uint32_t m = rsign[0];
+    for (int k = 1; k < kBoxThreads / kWave; ++k) m |= rsign[k];
+    v = (double)m;
+  }
+  if (parts > 1) {
+    double* mine = partial + (int64_t)blockIdx.x * kBoxPartial;
+    if (d < kBoxPartial) __hip_atomic_store(mine + d, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    // The stores are device-scope themselves, so before the ticket they only
+    // have to be complete; a release would write back the XCD's whole L2
+    // (4,096 blocks of a batch: 238 us).
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    uint32_t order = 0u;
+    if (d == 0)
+      order = __hip_atomic_fetch_add(tickets + sid, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    order = __builtin_amdgcn_readfirstlane(order);
+    if (order + 1u != (unsigned)parts) return;
+    if (d == 0) __hip_atomic_store(tickets + sid, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const double* all = partial + (int64_t)sid * parts * kBoxPartial;
+    sign = 0u;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) { mn[k] = INFINITY; mx[k] = -INFINITY; }
+    for (int p = d; p < parts; p += kWave) {
+      double u[kBoxPartial];
+#pragma unroll
+      for (int k = 0; k < kBoxPartial; ++k)
+        u[k] = __hip_atomic_load(all + p * kBoxPartial + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+      for (int k = 0; k < 3; ++k) { mn[k] = fmin(mn[k], u[k]); mx[k] = fmax(mx[k], u[3 + k]); }
+      sign |= (uint32_t)u[6];
     }
+    sign = wave_sign(sign);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) { mn[k] = wave_min(mn[k]); mx[k] = wave_max(mx[k]); }
+  } else {
+#pragma unroll
+    for (int k = 0; k < 3; ++k) { mn[k] = __shfl(v, k, kWave); mx[k] = __shfl(v, 3 + k, kWave); }
+    sign = (uint32_t)__shfl(v, 6, kWave);
   }
-  for (int k = 1; k < kBoxThreads / kWave; ++k) sign |= rsign[k];
-  if (e <= b) {
-    for (int d = 0; d < 3; ++d) { mn[d] = 0.0; mx[d] = 1.0; }
+  if (clear) {
+    static_assert(sizeof(DevScalars) % 4 == 0 && offsetof(DevScalars, flags) == 0,
+                  "cleared by words, the flags by the lane that sets them");
+    for (unsigned k = d; k < sizeof(DevScalars) / 4; k += kWave) reinterpret_cast<uint32_t*>(sc)[k] = 0u;
   }
+  if (d != 0) return;
+  if (e <= b)
+    for (int k = 0; k < 3; ++k) { mn[k] = 0.0; mx[k] = 1.0; }
   box_finalize(mn, mx, sign, force_cubic, boxes + sid, sc);
 }
 
@@ -269,22 +261,18 @@ void launch_sink_groups(hipStream_t s, int64_t m, int g, uint32_t* gfirst, uint3
   sink_groups_kernel<<<(unsigned)b, 256, 0, s>>>(m, g, gfirst, gcount);
 }
 
-int box_partial_blocks(int64_t n) {
-  int64_t b = (n + kBoxThreads * 16 - 1) / (kBoxThreads * 16);
-  return (int)(b < 1 ? 1 : (b > 1024 ? 1024 : b));
-}
-
-void launch_box(hipStream_t s, int64_t n, const double* x, const double* y, const double* z,
-                const double* q, int force_cubic, double* partial, DevBox* box, DevScalars* sc) {
-  const int nb = box_partial_blocks(n);
-  box_partial_kernel<<<nb, kBoxThreads, 0, s>>>(n, x, y, z, q, partial, sc);
-  box_final_kernel<<<1, kWave, 0, s>>>(nb, partial, force_cubic, box, sc);
-}
-
-void launch_box_batch(hipStream_t s, int nsys, const int64_t* soff, const double* x,
-                      const double* y, const double* z, const double* q, int force_cubic,
-                      DevBox* boxes, uint32_t* sys, DevScalars* sc) {
-  box_segment_kernel<<<nsys, kBoxThreads, 0, s>>>(nsys, soff, x, y, z, q, force_cubic, boxes, sys, sc);
+void launch_box(hipStream_t s, int64_t n, int nsys, const int64_t* soff, const double* x,
+                const double* y, const double* z, const double* q, int force_cubic,
+                double* partial, uint32_t* tickets, DevBox* boxes, uint32_t* sys, DevScalars* sc) {
+  // 16 particles a thread, as far as the partial results have room
+  int64_t parts = (n / nsys + kBoxThreads * 16 - 1) / (kBoxThreads * 16);
+  const int64_t most = nsys > 1 ? kBoxParts / nsys : 1024;
+  if (nsys > 1) parts *= 4;   // the largest system may be several times the mean
+  parts = parts < 1 ? 1 : parts;
+  parts = parts > most ? (most < 1 ? 1 : most) : parts;
+  box_kernel<<<(unsigned)(parts * nsys), kBoxThreads, 0, s>>>(
+      n, (int)parts, nsys > 1 ? soff : nullptr, x, y, z, q, force_cubic, partial, tickets, boxes,
+      nsys > 1 ? sys : nullptr, sc, nsys == 1);
 }
 
 void launch_keys(hipStream_t s, int64_t n, const double* x, const double* y, const double* z,

@@ -61,6 +61,7 @@ struct Ctx {
   uint32_t *hist = nullptr, *bsum = nullptr;
   int64_t hist_cap = 0, bsum_cap = 0;
   double* partial = nullptr;
+  uint32_t* box_tickets = nullptr;
   DevBox* box = nullptr;
   DevScalars* sc = nullptr;
   DevScalars* sc_host = nullptr;    // pinned
@@ -251,7 +252,7 @@ void free_all(Ctx* c) {
                   c->gfirst, c->gcount, c->gstat, c->queue, c->np2p, c->nm2p, c->res[0], c->res[1],
                   c->res[2], c->res[3], c->res[4], c->tab, c->ntype, c->kidtwig,
                   c->fc_rank, c->node_rank, c->nfirst, c->link, c->geom,
-                  c->mom64, c->wm32, c->wm64, c->hist, c->bsum, c->partial, c->box, c->sc,
+                  c->mom64, c->wm32, c->wm64, c->hist, c->bsum, c->partial, c->box_tickets, c->box, c->sc,
                   c->sys, c->soff, c->sysroot, c->label, c->tlabel, c->ehist, c->ecount,
                   c->nadj, c->parent, c->leafof, c->aqueue, c->lcount, c->loff, c->lent,
                   c->ltotal, c->nparent, c->echunk, c->esyschunk, c->epartial, c->prec4,
@@ -425,11 +426,9 @@ int grow_device_impl(Ctx* c, int64_t n, const double* x, const double* y, const 
   const uint32_t* sys = nsys > 1 ? c->sys : nullptr;
   hipStream_t s = c->stream;
   RECORD(c, 0);
-  reset_scalars_kernel<<<1, 64, 0, s>>>(c->sc);
-  if (nsys > 1)
-    launch_box_batch(s, (int)nsys, c->soff, x, y, z, q, c->cfg.force_cubic_domain, c->box, c->sys, c->sc);
-  else
-    launch_box(s, n, x, y, z, q, c->cfg.force_cubic_domain, c->partial, c->box, c->sc);
+  if (nsys > 1) reset_scalars_kernel<<<1, 64, 0, s>>>(c->sc);
+  launch_box(s, n, (int)nsys, c->soff, x, y, z, q, c->cfg.force_cubic_domain, c->partial,
+             c->box_tickets, c->box, c->sys, c->sc);
   launch_keys(s, n, x, y, z, q, c->box, sys, c->k0, c->v0, c->prec4);
   launch_sort_keys(s, c->k0, c->v0, c->k1, c->v1, n, c->hist, c->bsum, sys, nsys);
   launch_dup_detect(s, n, c->k0, sys, c->sc);
@@ -445,7 +444,7 @@ int grow_device_impl(Ctx* c, int64_t n, const double* x, const double* y, const 
   t.cap = c->mcap;
   t.keys = c->k0;
   t.x = c->xs; t.y = c->ys; t.z = c->zs; t.q = c->qs;
-  t.lo = c->lo; t.hi = c->hi; t.cnt = c->cnt;
+  t.lo = c->lo; t.hi = c->hi;
   t.tab = c->tab; t.fc_rank = c->fc_rank; t.ntype = c->ntype; t.kidtwig = c->kidtwig;
   t.node_rank = c->node_rank; t.nfirst = c->nfirst; t.link = c->link; t.geom = c->geom;
   t.parent = c->nparent;
@@ -490,7 +489,6 @@ int traverse_device_impl(Ctx* c, double* ex, double* ey, double* ez, double* pot
     return fail(c, PEPC_GPU_EINVAL, "traverse: periodic boundaries need a single system");
   a.nbox = c->periodic ? c->nbox : 1;
   a.vbox = c->periodic ? c->vbox : nullptr;
-  launch_walk_reset(s, a);
   RECORD(c, 2);
   launch_walk(s, a, c->cfg.precision, c->walk_blocks, c->cfg.list_tile,
               std::max(c->cfg.group_size, c->cfg.group_pack));
@@ -506,7 +504,9 @@ int traverse_device_impl(Ctx* c, double* ex, double* ey, double* ez, double* pot
 }
 
 int sync_impl(Ctx* c, pepc_gpu_stats* st) {
-  HIPCHECK(c, hipMemcpyAsync(c->sc_host, c->sc, sizeof(DevScalars), hipMemcpyDeviceToHost, c->stream));
+  HIPCHECK(c, hipSetDevice(c->cfg.device));
+  launch_publish(c->stream, c->sc, c->sc_host);
+  HIPCHECK(c, hipGetLastError());
   HIPCHECK(c, hipStreamSynchronize(c->stream));
   const DevScalars& h = *c->sc_host;
   if (st) {
@@ -629,9 +629,9 @@ int traverse_sinks_run(Ctx* c, const SinkBufs& b, int64_t m, const double* x, co
   }
   a.tx = tx; a.ty = ty; a.tz = tz;
   a.ex = out[0]; a.ey = out[1]; a.ez = out[2]; a.pot = out[3]; a.work = out[4];
-  launch_queue_reset(s, c->queue);
   launch_walk(s, a, c->cfg.precision, c->walk_blocks, c->cfg.list_tile,
               mode == PEPC_GPU_SINKS_GROUPED ? c->cfg.group_size : 1);
+  launch_zero_words(s, c->queue, kQueueWords);
   if (c->periodic && c->far_field) {
     launch_lattice_sources(s, c->n, c->xs, c->ys, c->zs, c->qs, c->lgeom, c->ml, c->fact, c->lpart,
                            c->ldpart, c->lom, c->ldip, c->mu, c->fict, c->lcoef);
@@ -696,7 +696,8 @@ int pepc_gpu_create(void** out, const pepc_gpu_config* cfg) {
       delete c;
       return PEPC_GPU_EHIP;
     }
-  if (dalloc(c, &c->box, 1) || dalloc(c, &c->sc, 1) || dalloc(c, &c->partial, 1024 * kBoxPartial) ||
+  if (dalloc(c, &c->box, 1) || dalloc(c, &c->sc, 1) || dalloc(c, &c->partial, kBoxParts * kBoxPartial) ||
+      dalloc(c, &c->box_tickets, kBoxParts) ||
       dalloc(c, &c->queue, kQueueWords) ||
       hipHostMalloc((void**)&c->sc_host, sizeof(DevScalars), hipHostMallocDefault) != hipSuccess) {
     free_all(c);
@@ -711,6 +712,8 @@ int pepc_gpu_create(void** out, const pepc_gpu_config* cfg) {
     }
     c->nxcd = nx < 1 ? 1 : (nx > kMaxQueues ? kMaxQueues : nx);
   }
+  launch_zero_words(c->stream, c->queue, kQueueWords);
+  launch_zero_words(c->stream, c->box_tickets, kBoxParts);
   c->walk_blocks = cfg->walk_blocks > 0
                        ? cfg->walk_blocks
                        : walk_default_blocks(cfg->precision == PEPC_GPU_FP64 ? kWalkFP64 : kWalkFP32Kahan,

@@ -62,33 +62,6 @@ __device__ __forceinline__ bool tree_broken(const DevScalars* sc) {
   return (sc->flags & (kFlagNodeOverflow | kFlagDupKeys | kFlagBadBox)) != 0u;
 }
 
-// A system boundary acts like the ends of the array: the first particle of a
-// system owns that system's root (level 0).
-__global__ void levels_kernel(int64_t n, const unsigned long long* __restrict__ keys,
-                              const uint32_t* __restrict__ sys,
-                              uint8_t* __restrict__ lo, uint8_t* __restrict__ hi,
-                              uint32_t* __restrict__ gmark, DevScalars* __restrict__ sc) {
-  for (int64_t a = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; a < n;
-       a += (int64_t)gridDim.x * blockDim.x) {
-    int la = 0, lb = 0;
-    bool dup = false;
-    if (a > 0 && same_sys(sys, a - 1, a)) {
-      if (keys[a - 1] == keys[a]) dup = true; else la = split_level(keys[a - 1], keys[a]);
-    }
-    if (a + 1 < n && same_sys(sys, a, a + 1)) {
-      if (keys[a + 1] == keys[a]) dup = true; else lb = split_level(keys[a], keys[a + 1]);
-    }
-    if (dup) {
-      atomicOr(&sc->flags, kFlagDupKeys);
-      la = lb = 0;
-    }
-    const int lam = la > lb ? la : lb;
-    lo[a] = (uint8_t)la;
-    hi[a] = (uint8_t)lam;
-    gmark[a] = 0;   // group marks start cleared (group_mark_kernel sets them)
-  }
-}
-
 // ---- BFS node numbering
 // Tiles of bfs_tile(n) sorted particles; wave w of a tile owns the w-th
 // quarter of them and takes them 64 at a time,
@@ -112,10 +85,10 @@ __host__ __device__ constexpr int bfs_tile(int64_t n) {
 constexpr int kLevels = kMaxLevel + 1;
 
 // The wave's node and twig counts per level over its particles: lane l
-// accumulates level l (levels < 21 <= 64 lanes).
-__device__ __forceinline__ void bfs_wave_counts(int64_t n, int64_t base,
-                                                const uint8_t* __restrict__ lo,
-                                                const uint8_t* __restrict__ hi, uint32_t& cn,
+// accumulates level l (levels < 21 <= 64 lanes).  levels(a, l0, l1) gives the
+// first and last level of the nodes that particle a < n owns.
+template <class F>
+__device__ __forceinline__ void bfs_wave_counts(int64_t n, int64_t base, F levels, uint32_t& cn,
                                                 uint32_t& ct) {
   const int lane = lane_id();
   const int passes = bfs_tile(n) / (kBfsWaves * kWave);
@@ -123,8 +96,8 @@ __device__ __forceinline__ void bfs_wave_counts(int64_t n, int64_t base,
   ct = 0;
   for (int it = 0; it < passes; ++it) {
     const int64_t a = base + (int64_t)it * kWave + lane;
-    const bool valid = a < n;
-    const int l0 = valid ? lo[a] : kLevels, l1 = valid ? hi[a] : -1;
+    int l0 = kLevels, l1 = -1;
+    if (a < n) levels(a, l0, l1);
     const int lmin = -wave_max_i32(-l0), lmax = wave_max_i32(l1);
     for (int l = lmin; l <= lmax; ++l) {
       const uint32_t c = (uint32_t)popc64(__ballot(l0 <= l && l <= l1));
@@ -134,16 +107,41 @@ __device__ __forceinline__ void bfs_wave_counts(int64_t n, int64_t base,
   }
 }
 
-__global__ __launch_bounds__(kT) void bfs_count_kernel(int64_t n, const uint8_t* __restrict__ lo,
-                                                      const uint8_t* __restrict__ hi,
+// Levels of every particle's nodes (a system boundary acts like the ends of
+// the array: the first particle of a system owns that system's root, level
+// 0), their counts, and cleared group marks, which group_mark_kernel sets.
+// The levels come straight from the keys: they cost a launch of their own
+// before (2 us in every grow, and 17 us of memory traffic at 4,194,304
+// particles).  Counts nothing that later kernels use once a flag is raised.
+__global__ __launch_bounds__(kT) void bfs_count_kernel(int64_t n,
+                                                      const unsigned long long* __restrict__ keys,
+                                                      const uint32_t* __restrict__ sys,
+                                                      uint8_t* __restrict__ lo,
+                                                      uint8_t* __restrict__ hi,
+                                                      uint32_t* __restrict__ gmark,
                                                       uint32_t* __restrict__ tab, int64_t nb,
-                                                      const DevScalars* __restrict__ sc) {
-  if (tree_broken(sc)) return;
+                                                      DevScalars* __restrict__ sc) {
   __shared__ uint32_t wn[kBfsWaves][kLevels], wt[kBfsWaves][kLevels];
   const int w = threadIdx.x / kWave, lane = lane_id();
   uint32_t cn, ct;
   const int64_t per_wave = bfs_tile(n) / kBfsWaves;
-  bfs_wave_counts(n, ((int64_t)blockIdx.x * kBfsWaves + w) * per_wave, lo, hi, cn, ct);
+  const auto levels = [&](int64_t a, int& l0, int& l1) {
+    const unsigned long long key = keys[a];
+    const bool prev = a > 0 && same_sys(sys, a - 1, a), next = a + 1 < n && same_sys(sys, a, a + 1);
+    const unsigned long long kp = prev ? keys[a - 1] : ~key, kn = next ? keys[a + 1] : ~key;
+    if (kp == key || kn == key) {   // equal keys left: no tree
+      atomicOr(&sc->flags, kFlagDupKeys);
+      l0 = l1 = 0;
+    } else {
+      l0 = prev ? split_level(kp, key) : 0;
+      l1 = next ? split_level(key, kn) : 0;
+      l1 = l0 > l1 ? l0 : l1;
+    }
+    lo[a] = (uint8_t)l0;
+    hi[a] = (uint8_t)l1;
+    gmark[a] = 0;
+  };
+  bfs_wave_counts(n, ((int64_t)blockIdx.x * kBfsWaves + w) * per_wave, levels, cn, ct);
   if (lane < kLevels) { wn[w][lane] = cn; wt[w][lane] = ct; }
   __syncthreads();
   if (threadIdx.x < kLevels) {
@@ -269,7 +267,7 @@ __global__ __launch_bounds__(kT) void bfs_emit_kernel(
   const int64_t per_wave = bfs_tile(n) / kBfsWaves;
   const int64_t base = ((int64_t)blockIdx.x * kBfsWaves + w) * per_wave;
   uint32_t rn, rt;   // lane l: next node index / twig rank of level l for this wave
-  bfs_wave_counts(n, base, lo, hi, rn, rt);
+  bfs_wave_counts(n, base, [&](int64_t a, int& l0, int& l1) { l0 = lo[a]; l1 = hi[a]; }, rn, rt);
   if (lane < kLevels) { wn[w][lane] = rn; wt[w][lane] = rt; }
   __syncthreads();
   if (lane < kLevels) {
@@ -894,20 +892,6 @@ __global__ void group_mark_kernel(int group_size, int pack, const NodeLink* __re
   }
 }
 
-__global__ void group_emit_kernel(int64_t n, const uint32_t* __restrict__ gmark,
-                                  const uint32_t* __restrict__ rank, uint32_t* __restrict__ gfirst,
-                                  uint32_t* __restrict__ gcount) {
-  for (int64_t a = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; a < n;
-       a += (int64_t)gridDim.x * blockDim.x) {
-    const uint32_t c = gmark[a];
-    if (c) {
-      const uint32_t g = rank[a];
-      gfirst[g] = (uint32_t)a;
-      gcount[g] = c;
-    }
-  }
-}
-
 // Root node of each system (level-0 nodes, one per non-empty system).
 __global__ void sysroot_kernel(const uint32_t* __restrict__ sys, const uint32_t* __restrict__ nfirst,
                                uint32_t* __restrict__ sysroot, const DevScalars* __restrict__ sc) {
@@ -947,8 +931,8 @@ int64_t bfs_table_words(int64_t n) {
 
 void launch_tree_build(hipStream_t s, const TreeBuffers& t, int group_size, int group_pack) {
   const int64_t n = t.n, cap = t.cap, nb = bfs_tiles(n);
-  levels_kernel<<<grid_for(n), kT, 0, s>>>(n, t.keys, t.sys, t.lo, t.hi, t.gmark, t.sc);
-  bfs_count_kernel<<<(unsigned)nb, kT, 0, s>>>(n, t.lo, t.hi, t.tab, nb, t.sc);
+  bfs_count_kernel<<<(unsigned)nb, kT, 0, s>>>(n, t.keys, t.sys, t.lo, t.hi, t.gmark, t.tab, nb,
+                                               t.sc);
   bfs_scan_kernel<<<2 * kLevels, kBfsScanT, 0, s>>>(t.tab, nb, cap, t.sc);
   bfs_emit_kernel<<<(unsigned)nb, kT, 0, s>>>(n, t.lo, t.hi, t.tab, nb, t.x, t.y, t.z, t.q, t.geom,
                                               t.link, t.nfirst, t.ntype, t.fc_rank, t.node_rank,
@@ -956,8 +940,7 @@ void launch_tree_build(hipStream_t s, const TreeBuffers& t, int group_size, int 
   launch_upward(s, t);
   group_mark_kernel<<<grid_for(n), kT, 0, s>>>(group_size, group_pack, t.link, t.nfirst, t.node_rank,
                                                t.gmark, t.sc);
-  launch_scan(s, t.gmark, t.cnt, n, t.bsum, &t.sc->ngroups, true);
-  group_emit_kernel<<<grid_for(n), kT, 0, s>>>(n, t.gmark, t.cnt, t.gfirst, t.gcount);
+  launch_group_list(s, n, t.gmark, t.bsum, t.gfirst, t.gcount, &t.sc->ngroups);
   if (t.sys) sysroot_kernel<<<grid_for(t.nsys), kT, 0, s>>>(t.sys, t.nfirst, t.sysroot, t.sc);
 }
 

@@ -253,6 +253,14 @@ void walk_kernel(WalkArgs a) {
   const double theta2 = a.theta2;
   const double t_acc = theta2 * (1.0 - 1e-12), t_rej = theta2 * (1.0 + 1e-12);
   const uint32_t ngroups = SINK ? a.nsink_groups : a.sc->ngroups;
+  if (!SINK && blockIdx.x == 0 && lane == 0) {   // the sums of walk_stats_kernel
+    a.sc->interactions = 0;
+    a.sc->mac_evals = 0;
+    a.sc->p2p = 0;
+    a.sc->m2p = 0;
+    a.sc->amb_nodes = 0;
+    a.sc->walk_steps = 0;
+  }
   const double* __restrict__ TX = SINK ? a.tx : a.x;
   const double* __restrict__ TY = SINK ? a.ty : a.y;
   const double* __restrict__ TZ = SINK ? a.tz : a.z;
@@ -665,9 +673,13 @@ void walk_kernel(WalkArgs a) {
 
 // Sums the per-group records into the device scalars (walk statistics of
 // tree_walk_statistics, module_tree_walk_simple.f90:63-115).
+// Also leaves the work-queue heads at zero for the next walk; the walk itself
+// clears the sums, which saves a launch before it.
 __global__ __launch_bounds__(256) void walk_stats_kernel(const uint32_t* __restrict__ gstat,
-                                                        DevScalars* __restrict__ sc) {
+                                                        DevScalars* __restrict__ sc,
+                                                        uint32_t* __restrict__ queue) {
   const int64_t ng = sc->ngroups;
+  if (blockIdx.x == 0 && threadIdx.x < kMaxQueues) queue[kQueueStride * threadIdx.x] = 0;
   unsigned long long v[6] = {0, 0, 0, 0, 0, 0};
   for (int64_t g = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; g < ng;
        g += (int64_t)gridDim.x * blockDim.x) {
@@ -700,20 +712,13 @@ __global__ __launch_bounds__(256) void walk_stats_kernel(const uint32_t* __restr
   }
 }
 
-__global__ void walk_reset_kernel(DevScalars* sc, uint32_t* queue) {
-  if (threadIdx.x < kMaxQueues) queue[kQueueStride * threadIdx.x] = 0;
-  if (threadIdx.x == 0) {
-    sc->interactions = 0;
-    sc->mac_evals = 0;
-    sc->p2p = 0;
-    sc->m2p = 0;
-    sc->amb_nodes = 0;
-    sc->walk_steps = 0;
-  }
+__global__ __launch_bounds__(256) void zero_words_kernel(uint32_t* words, int n) {
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) words[i] = 0;
 }
 
-__global__ void queue_reset_kernel(uint32_t* queue) {
-  if (threadIdx.x < kMaxQueues) queue[kQueueStride * threadIdx.x] = 0;
+__global__ void publish_kernel(const DevScalars* __restrict__ src, DevScalars* __restrict__ dst) {
+  for (unsigned k = threadIdx.x; k < sizeof(DevScalars) / 4; k += blockDim.x)
+    reinterpret_cast<uint32_t*>(dst)[k] = reinterpret_cast<const uint32_t*>(src)[k];
 }
 
 // FP64 direct sum (src/utils/module_directsum.f90:34-172): all sources
@@ -835,11 +840,13 @@ int walk_default_blocks(int precision, int list_tile) {
   return cus * per;
 }
 
-void launch_walk_reset(hipStream_t s, const WalkArgs& a) {
-  walk_reset_kernel<<<1, 64, 0, s>>>(a.sc, a.queue);
+void launch_zero_words(hipStream_t s, uint32_t* words, int n) {
+  zero_words_kernel<<<(n + 255) / 256, 256, 0, s>>>(words, n);
 }
 
-void launch_queue_reset(hipStream_t s, uint32_t* queue) { queue_reset_kernel<<<1, 64, 0, s>>>(queue); }
+void launch_publish(hipStream_t s, const DevScalars* src, DevScalars* dst) {
+  publish_kernel<<<1, 64, 0, s>>>(src, dst);
+}
 
 bool walk_list_tile_ok(int precision, int list_tile) {
   if (list_tile == 0) return true;
@@ -882,7 +889,7 @@ void launch_walk(hipStream_t s, const WalkArgs& a, int precision, int blocks, in
 }
 
 void launch_walk_stats(hipStream_t s, const WalkArgs& a) {
-  walk_stats_kernel<<<256, 256, 0, s>>>(a.gstat, a.sc);
+  walk_stats_kernel<<<256, 256, 0, s>>>(a.gstat, a.sc, a.queue);
 }
 
 // About kDirectBlocks blocks: eight of four waves for each of the 256 CUs.  A
