@@ -47,6 +47,8 @@ void launch_radix_pass_dev(hipStream_t s, const unsigned long long* kin, const u
                            unsigned long long* kout, uint32_t* vout, int64_t n, const uint32_t* ndev,
                            int shift, int nbits, uint32_t* hist, uint32_t* bsum,
                            const uint32_t* dsrc);
+// launch_sort_keys takes its input in (k1, v1) instead of (k0, v0).
+bool sort_input_second(int64_t n, bool batched);
 void launch_sort_keys(hipStream_t s, unsigned long long* k0, uint32_t* v0, unsigned long long* k1,
                       uint32_t* v1, int64_t n, uint32_t* hist, uint32_t* bsum,
                       const uint32_t* sysid, int64_t nsys);

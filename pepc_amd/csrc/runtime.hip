@@ -429,7 +429,8 @@ int grow_device_impl(Ctx* c, int64_t n, const double* x, const double* y, const 
   if (nsys > 1) reset_scalars_kernel<<<1, 64, 0, s>>>(c->sc);
   launch_box(s, n, (int)nsys, c->soff, x, y, z, q, c->cfg.force_cubic_domain, c->partial,
              c->box_tickets, c->box, c->sys, c->sc);
-  launch_keys(s, n, x, y, z, q, c->box, sys, c->k0, c->v0, c->prec4);
+  const bool second = sort_input_second(n, sys != nullptr);
+  launch_keys(s, n, x, y, z, q, c->box, sys, second ? c->k1 : c->k0, second ? c->v1 : c->v0, c->prec4);
   launch_sort_keys(s, c->k0, c->v0, c->k1, c->v1, n, c->hist, c->bsum, sys, nsys);
   launch_dup_detect(s, n, c->k0, sys, c->sc);
   // equal keys into the reference presort's order and apart (the sort's
@@ -613,7 +614,8 @@ int traverse_sinks_run(Ctx* c, const SinkBufs& b, int64_t m, const double* x, co
   const double *tx = x, *ty = y, *tz = z;
   double* out[5] = {ex, ey, ez, pot, work};
   if (mode == PEPC_GPU_SINKS_GROUPED) {
-    launch_sink_keys(s, m, x, y, z, c->box, b.k0, b.v0);
+    const bool second = sort_input_second(m, false);
+    launch_sink_keys(s, m, x, y, z, c->box, second ? b.k1 : b.k0, second ? b.v1 : b.v0);
     launch_sort_keys(s, b.k0, b.v0, b.k1, b.v1, m, b.hist, b.bsum, nullptr, 1);
     // the fourth gathered array is a scratch copy of x (gather4 moves four)
     launch_gather4(s, m, b.v0, x, y, z, x, b.x, b.y, b.z, b.res[4]);
