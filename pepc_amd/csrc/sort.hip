@@ -434,7 +434,10 @@ __global__ __launch_bounds__(kRankT) void rank_block_kernel(
 
 // Runs of `run` elements (the last may be shorter), four to a group: element
 // i of a run moves behind the elements of the group's earlier runs that are
-// not greater and of its later runs that are smaller.
+// not greater and of its later runs that are smaller.  The searches are a
+// chain of loads, so PAIR takes two steps at a time, for half as many loads
+// again; that is the shorter way until the loads themselves fill the chip.
+template <bool PAIR>
 __global__ __launch_bounds__(256) void merge4_kernel(const unsigned long long* __restrict__ kin,
                                                      const uint32_t* __restrict__ vin,
                                                      unsigned long long* __restrict__ kout,
@@ -449,14 +452,39 @@ __global__ __launch_bounds__(256) void merge4_kernel(const unsigned long long* _
   for (int q = 0; q < 3; ++q) {
     const int other = first + q + (first + q >= r ? 1 : 0);
     const int64_t b = (int64_t)other * run;
-    begin[q] = b < n ? (int)b : n;
-    len[q] = n - begin[q] < run ? n - begin[q] : run;
+    // an empty run reads element 0 and takes nothing from it
+    begin[q] = b < n ? (int)b : 1;
+    len[q] = b < n ? (n - begin[q] < run ? n - begin[q] : run) : 0;
     bound[q] = other < r ? key + 1ull : key;
   }
-  for (int s = run; s > 0; s >>= 1) {
+  if constexpr (PAIR) {
+    // two binary steps at a time (run is 2^11 times a power of four: 12, 14, ...
+    // steps): their three pivots are loaded together
+    for (int s = run; s > 1; s >>= 2) {
+      const int h = s >> 1;
+      unsigned long long a[3], b[3], c[3];
 #pragma unroll
-    for (int q = 0; q < 3; ++q)
-      if (pos[q] + s <= len[q] && kin[begin[q] + pos[q] + s - 1] < bound[q]) pos[q] += s;
+      for (int q = 0; q < 3; ++q) {
+        const unsigned long long* p = kin + begin[q];
+        const int last = len[q] - 1;
+        const int ia = pos[q] + h - 1, ib = pos[q] + s - 1, ic = pos[q] + s + h - 1;
+        a[q] = p[ia < last ? ia : last];
+        b[q] = p[ib < last ? ib : last];
+        c[q] = p[ic < last ? ic : last];
+      }
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        const bool up = pos[q] + s <= len[q] && b[q] < bound[q];
+        pos[q] += up ? s : 0;
+        if (pos[q] + h <= len[q] && (up ? c[q] : a[q]) < bound[q]) pos[q] += h;
+      }
+    }
+  } else {
+    for (int s = run; s > 0; s >>= 1) {
+#pragma unroll
+      for (int q = 0; q < 3; ++q)
+        if (pos[q] + s <= len[q] && kin[begin[q] + pos[q] + s - 1] < bound[q]) pos[q] += s;
+    }
   }
   const int64_t out = (int64_t)first * run + (i - r * run) + pos[0] + pos[1] + pos[2];
   kout[out] = key;
@@ -1036,6 +1064,10 @@ constexpr int64_t kMergeMax = 524288;
 // same 234 and of 262,144 306 and 283.
 constexpr int64_t kRankMax = 65536;
 
+// Largest array merged with two search steps at a time (grow of 32,768
+// particles 155 -> 145 us, 131,072 232 -> 222, but 524,288 346 -> 356).
+constexpr int64_t kMergePairMax = 131072;
+
 static int merge_launches(int64_t n) {
   int merges = 0;
   for (int64_t run = kMergeN; run < n; run *= 4) ++merges;
@@ -1058,7 +1090,8 @@ static void launch_merge_sort(hipStream_t s, unsigned long long* k0, uint32_t* v
     merge_block_kernel<<<(unsigned)((n + kMergeN - 1) / kMergeN), kMergeT, 0, s>>>(k0, v0, ka, va, n);
   int run = kMergeN;
   for (int m = 0; m < merges; ++m, run *= 4) {
-    merge4_kernel<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(ka, va, kb, vb, (int)n, run);
+    auto* merge = n <= kMergePairMax ? merge4_kernel<true> : merge4_kernel<false>;
+    merge<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(ka, va, kb, vb, (int)n, run);
     std::swap(ka, kb);
     std::swap(va, vb);
   }
