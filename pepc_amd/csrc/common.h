@@ -166,4 +166,62 @@ __device__ __forceinline__ int split_level(unsigned long long a, unsigned long l
   return kMaxLevel - msb / 3;
 }
 
+// Work queues of the persistent kernels, one per XCD: the items (in key
+// order) are cut into nq contiguous ranges and workgroup b, which the
+// dispatcher places on XCD b mod nq, takes items from range b mod nq first, so
+// the waves sharing an XCD's L2 work on neighbouring items and reuse the same
+// nodes.  A used-up range sends the wave on to the next one.
+// The first items of a range belong to its workgroups by number, only the
+// others are counted out by the range's head, and the first wave that finds a
+// range used up says so in the last word, which a wave reads once, when its
+// own range has ended.  Atomics on one address are served one after another
+// (15 ns each), and every wave used to ask all eight heads at its end: 4,096
+// waves spent 60 us of every walk that way (487 groups: 92 -> 28 us; 8,400:
+// 198 -> 146; 134,000: 1.63 -> 1.59 ms).  Reading a head before asking it is
+// worse (98 ns per item), and so is handing out several items at once, whose
+// nodes the neighbouring waves then no longer share (4 at a time, 4,194,304
+// particles: 5.13 -> 5.45 ms).
+constexpr int kMaxQueues = 8;
+constexpr int kQueueStride = 16;   // words: a 64-byte line for each head
+constexpr int kQueueWords = (kMaxQueues + 1) * kQueueStride;   // zero at a kernel's start
+
+struct GroupQueue {
+  uint32_t nq, q, todo;   // queues, position, ranges to look at
+  uint32_t mine;          // the item by number, then ~0
+  bool looked;
+
+  __device__ __forceinline__ void init(uint32_t queues) {
+    nq = queues;
+    q = blockIdx.x % nq;
+    todo = (1u << nq) - 1u;
+    mine = blockIdx.x / nq;
+    looked = false;
+  }
+  // One lane of the workgroup: the next of n items, or n when there is none.
+  __device__ __forceinline__ uint32_t next(uint32_t* heads, uint32_t n) {
+    while (todo) {
+      if ((todo >> q) & 1u) {
+        const uint32_t lo = (uint32_t)((uint64_t)n * q / nq);
+        const uint32_t size = (uint32_t)((uint64_t)n * (q + 1) / nq) - lo;
+        const uint32_t given = (gridDim.x - q + nq - 1u) / nq;   // workgroups of this range
+        uint32_t r = mine;
+        mine = ~0u;
+        if (r >= size && size > given) {
+          r = given + atomicAdd(heads + kQueueStride * q, 1u);
+          if (r == size) atomicOr(heads + kQueueStride * kMaxQueues, 1u << q);
+        }
+        if (r < size) return lo + r;
+        todo &= ~(1u << q);
+        if (!looked) {
+          todo &= ~__hip_atomic_load(heads + kQueueStride * kMaxQueues, __ATOMIC_RELAXED,
+                                     __HIP_MEMORY_SCOPE_AGENT);
+          looked = true;
+        }
+      }
+      q = q + 1 == nq ? 0u : q + 1;
+    }
+    return n;
+  }
+};
+
 }  // namespace pepc

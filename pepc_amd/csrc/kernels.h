@@ -165,11 +165,6 @@ struct WalkArgs {
   const double *tx = nullptr, *ty = nullptr, *tz = nullptr;
   uint32_t nsink_groups = 0;
 };
-// Work queues of the persistent walk: up to kMaxQueues heads, each on a
-// 64-byte line of its own (kQueueWords words in all).
-constexpr int kMaxQueues = 8;
-constexpr int kQueueStride = 16;
-constexpr int kQueueWords = kMaxQueues * kQueueStride;
 // Zeroes n words.  The work-queue heads are zero between walks: launch_walk_stats
 // leaves them so, and a walk of sinks is followed by this.
 void launch_zero_words(hipStream_t s, uint32_t* words, int n);

@@ -265,25 +265,11 @@ void walk_kernel(WalkArgs a) {
   const double* __restrict__ TY = SINK ? a.ty : a.y;
   const double* __restrict__ TZ = SINK ? a.tz : a.z;
 
-  // Work queues, one per XCD: the groups (in key order) are cut into nqueue
-  // contiguous ranges and workgroup b, which the dispatcher places on XCD
-  // b mod nqueue, takes groups from range b mod nqueue first, so the waves
-  // sharing an XCD's L2 walk neighbouring groups and reuse the same nodes.
-  // An exhausted range sends the wave on to the next one.
-  const uint32_t nq = (uint32_t)a.nqueue;
-  uint32_t q = blockIdx.x % nq, qleft = nq;   // lane 0's position in the queues
+  GroupQueue work;
+  work.init((uint32_t)a.nqueue);
   for (;;) {
     uint32_t gg = ngroups;
-    if (lane == 0) {
-      while (qleft) {
-        const uint32_t lo = (uint32_t)((uint64_t)ngroups * q / nq);
-        const uint32_t hi = (uint32_t)((uint64_t)ngroups * (q + 1) / nq);
-        const uint32_t r = atomicAdd(a.queue + kQueueStride * q, 1u);
-        if (r < hi - lo) { gg = lo + r; break; }
-        q = q + 1 == nq ? 0u : q + 1;
-        --qleft;
-      }
-    }
+    if (lane == 0) gg = work.next(a.queue, ngroups);
     const uint32_t g = uniform(gg);
     if (g >= ngroups) break;
 
@@ -679,7 +665,7 @@ __global__ __launch_bounds__(256) void walk_stats_kernel(const uint32_t* __restr
                                                         DevScalars* __restrict__ sc,
                                                         uint32_t* __restrict__ queue) {
   const int64_t ng = sc->ngroups;
-  if (blockIdx.x == 0 && threadIdx.x < kMaxQueues) queue[kQueueStride * threadIdx.x] = 0;
+  if (blockIdx.x == 0 && threadIdx.x <= kMaxQueues) queue[kQueueStride * threadIdx.x] = 0;
   unsigned long long v[6] = {0, 0, 0, 0, 0, 0};
   for (int64_t g = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; g < ng;
        g += (int64_t)gridDim.x * blockDim.x) {
