@@ -257,8 +257,9 @@ int pepc_gpu_direct(void *ctx, int64_t n, const double *x, const double *y, cons
                     const double *q, int64_t ntest, const int64_t *testidx, double eps2,
                     double sign, double *ex, double *ey, double *ez, double *pot);
 
-/* Device timing of the last grow and traverse in milliseconds (HIP events
- * on the context's stream, recorded by the *_device and host forms). */
+/* Device timing of the last grow and traverse in milliseconds, by the
+ * device's constant clock (10 ns) at the start and end of their kernels; -1
+ * for one that has not run yet. */
 int pepc_gpu_timings(void *ctx, double *t_grow_ms, double *t_walk_ms);
 
 /* ---------------------------------------------------------------------------

@@ -166,6 +166,10 @@ __device__ __forceinline__ int split_level(unsigned long long a, unsigned long l
   return kMaxLevel - msb / 3;
 }
 
+// Device clock at the ends of a grow and of a walk, written by their own
+// first and last kernels: four events on the stream took 14 us of every solve.
+enum { kClockGrow = 0, kClockGrown, kClockWalk, kClockWalked, kClocks };
+
 // Work queues of the persistent kernels, one per XCD: the items (in key
 // order) are cut into nq contiguous ranges and workgroup b, which the
 // dispatcher places on XCD b mod nq, takes items from range b mod nq first, so

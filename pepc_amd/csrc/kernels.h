@@ -14,7 +14,8 @@ constexpr int kBoxParts = 4096;  // blocks of launch_box with partial results
 // tickets: kBoxParts words, zero between calls.
 void launch_box(hipStream_t s, int64_t n, int nsys, const int64_t* soff, const double* x,
                 const double* y, const double* z, const double* q, int force_cubic,
-                double* partial, uint32_t* tickets, DevBox* boxes, uint32_t* sys, DevScalars* sc);
+                double* partial, uint32_t* tickets, DevBox* boxes, uint32_t* sys, DevScalars* sc,
+                unsigned long long* clock);
 // sys == nullptr: one system with boxes[0].
 // Also writes rec[i] = {x, y, z, q} (input order) for launch_gather_rec.
 void launch_keys(hipStream_t s, int64_t n, const double* x, const double* y, const double* z,
@@ -37,7 +38,8 @@ void launch_scan(hipStream_t s, const uint32_t* in, uint32_t* out, int64_t n, ui
 // Group g is the g-th nonzero mark: gfirst[g] its particle, gcount[g] its
 // value; *ngroups their number.
 void launch_group_list(hipStream_t s, int64_t n, const uint32_t* gmark, uint32_t* bsum,
-                       uint32_t* gfirst, uint32_t* gcount, uint32_t* ngroups);
+                       uint32_t* gfirst, uint32_t* gcount, uint32_t* ngroups,
+                       unsigned long long* clock);
 void launch_radix_pass(hipStream_t s, const unsigned long long* kin, const uint32_t* vin,
                        unsigned long long* kout, uint32_t* vout, int64_t n, int shift, int nbits,
                        uint32_t* hist, uint32_t* bsum);
@@ -118,6 +120,7 @@ struct TreeBuffers {
   const int64_t* soff;               // system ranges, nsys + 1 entries
   uint32_t* sysroot;                 // root node per system
   int64_t nsys;
+  unsigned long long* clock;         // kClocks device clocks
 };
 
 void launch_dup_detect(hipStream_t s, int64_t n, const unsigned long long* keys, const uint32_t* sys,
@@ -153,6 +156,7 @@ struct WalkArgs {
   uint32_t* nm2p;
   uint32_t* gstat;                   // 8 words per group: mac, p2p, m2p, amb, steps, count
   uint32_t* queue;                   // work-queue heads, kQueueStride words apart
+  unsigned long long* clock = nullptr;   // kClocks device clocks (not for sinks)
   int nqueue = 1;                    // queues: one contiguous range of groups per XCD
   const uint32_t* sys;               // batched systems: system per particle (else nullptr)
   const uint32_t* sysroot;           // batched systems: root node per system

@@ -72,7 +72,9 @@ __global__ __launch_bounds__(kBoxThreads) void box_kernel(
     int64_t n, int parts, const int64_t* __restrict__ soff, const double* __restrict__ x,
     const double* __restrict__ y, const double* __restrict__ z, const double* __restrict__ q,
     int force_cubic, double* partial, uint32_t* tickets, DevBox* __restrict__ boxes,
-    uint32_t* __restrict__ sys, DevScalars* __restrict__ sc, bool clear) {
+    uint32_t* __restrict__ sys, DevScalars* __restrict__ sc, bool clear,
+    unsigned long long* __restrict__ clock) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) clock[kClockGrow] = wall_clock64();
   const unsigned sid = blockIdx.x / (unsigned)parts, part = blockIdx.x % (unsigned)parts;
   const int64_t b = soff ? soff[sid] : 0, e = soff ? soff[sid + 1] : n;
   double mn[3] = {INFINITY, INFINITY, INFINITY};
@@ -263,7 +265,8 @@ void launch_sink_groups(hipStream_t s, int64_t m, int g, uint32_t* gfirst, uint3
 
 void launch_box(hipStream_t s, int64_t n, int nsys, const int64_t* soff, const double* x,
                 const double* y, const double* z, const double* q, int force_cubic,
-                double* partial, uint32_t* tickets, DevBox* boxes, uint32_t* sys, DevScalars* sc) {
+                double* partial, uint32_t* tickets, DevBox* boxes, uint32_t* sys, DevScalars* sc,
+                unsigned long long* clock) {
   // 16 particles a thread, as far as the partial results have room
   int64_t parts = (n / nsys + kBoxThreads * 16 - 1) / (kBoxThreads * 16);
   const int64_t most = nsys > 1 ? kBoxParts / nsys : 1024;
@@ -272,7 +275,7 @@ void launch_box(hipStream_t s, int64_t n, int nsys, const int64_t* soff, const d
   parts = parts > most ? (most < 1 ? 1 : most) : parts;
   box_kernel<<<(unsigned)(parts * nsys), kBoxThreads, 0, s>>>(
       n, (int)parts, nsys > 1 ? soff : nullptr, x, y, z, q, force_cubic, partial, tickets, boxes,
-      nsys > 1 ? sys : nullptr, sc, nsys == 1);
+      nsys > 1 ? sys : nullptr, sc, nsys == 1, clock);
 }
 
 void launch_keys(hipStream_t s, int64_t n, const double* x, const double* y, const double* z,

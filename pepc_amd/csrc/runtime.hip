@@ -65,7 +65,9 @@ struct Ctx {
   DevBox* box = nullptr;
   DevScalars* sc = nullptr;
   DevScalars* sc_host = nullptr;    // pinned
-  hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
+  unsigned long long* clock = nullptr;   // kClocks device clocks
+  bool timed_grow = false, timed_walk = false;   // run outside a capture
+  double clock_ms = 0.0;                 // per tick
   TreeBuffers tb;                   // buffers of the last grow
   // batched systems
   int64_t nsys = 1, sys_cap = 0;
@@ -252,7 +254,7 @@ void free_all(Ctx* c) {
                   c->gfirst, c->gcount, c->gstat, c->queue, c->np2p, c->nm2p, c->res[0], c->res[1],
                   c->res[2], c->res[3], c->res[4], c->tab, c->ntype, c->kidtwig,
                   c->fc_rank, c->node_rank, c->nfirst, c->link, c->geom,
-                  c->mom64, c->wm32, c->wm64, c->hist, c->bsum, c->partial, c->box_tickets, c->box, c->sc,
+                  c->mom64, c->wm32, c->wm64, c->hist, c->bsum, c->partial, c->box_tickets, c->clock, c->box, c->sc,
                   c->sys, c->soff, c->sysroot, c->label, c->tlabel, c->ehist, c->ecount,
                   c->nadj, c->parent, c->leafof, c->aqueue, c->lcount, c->loff, c->lent,
                   c->ltotal, c->nparent, c->echunk, c->esyschunk, c->epartial, c->prec4,
@@ -390,16 +392,17 @@ int check_flags(Ctx* c, uint32_t f) {
 
 Ctx* as_ctx(void* p) { return reinterpret_cast<Ctx*>(p); }
 
-int record(Ctx* c, int k) {
-  if (!c->capturing) HIPCHECK(c, hipEventRecord(c->ev[k], c->stream));
-  return 0;
+// Milliseconds of the last grow and walk by the device's clock (its stream
+// synchronized); false when they cannot be read.
+bool read_clock(Ctx* c, double* grow, double* walk) {
+  unsigned long long t[kClocks];
+  if (hipMemcpyAsync(t, c->clock, sizeof(t), hipMemcpyDeviceToHost, c->stream) != hipSuccess ||
+      hipStreamSynchronize(c->stream) != hipSuccess)
+    return false;
+  *grow = (double)(t[kClockGrown] - t[kClockGrow]) * c->clock_ms;
+  *walk = (double)(t[kClockWalked] - t[kClockWalk]) * c->clock_ms;
+  return true;
 }
-
-#define RECORD(c, k)              \
-  do {                            \
-    int _r = record((c), (k));    \
-    if (_r) return _r;            \
-  } while (0)
 
 // nsys == 1: one system (no offsets needed).  nsys > 1: particles of system s
 // occupy [off[s], off[s+1]) on input and, sorted by key, on output.
@@ -425,10 +428,9 @@ int grow_device_impl(Ctx* c, int64_t n, const double* x, const double* y, const 
   }
   const uint32_t* sys = nsys > 1 ? c->sys : nullptr;
   hipStream_t s = c->stream;
-  RECORD(c, 0);
   if (nsys > 1) reset_scalars_kernel<<<1, 64, 0, s>>>(c->sc);
   launch_box(s, n, (int)nsys, c->soff, x, y, z, q, c->cfg.force_cubic_domain, c->partial,
-             c->box_tickets, c->box, c->sys, c->sc);
+             c->box_tickets, c->box, c->sys, c->sc, c->clock);
   const bool second = sort_input_second(n, sys != nullptr);
   launch_keys(s, n, x, y, z, q, c->box, sys, second ? c->k1 : c->k0, second ? c->v1 : c->v0, c->prec4);
   launch_sort_keys(s, c->k0, c->v0, c->k1, c->v1, n, c->hist, c->bsum, sys, nsys);
@@ -458,15 +460,16 @@ int grow_device_impl(Ctx* c, int64_t n, const double* x, const double* y, const 
   t.soff = nsys > 1 ? c->soff : nullptr;
   t.sysroot = c->sysroot;
   t.nsys = nsys;
+  t.clock = c->clock;
   c->tb = t;
   launch_tree_build(s, t, c->cfg.group_size, c->cfg.group_pack);
   HIPCHECK(c, hipGetLastError());
-  RECORD(c, 1);
   c->n = n;
   c->nsys = nsys;
   c->frozen = false;
   c->grown = true;
   c->walked = false;
+  if (!c->capturing) c->timed_grow = true;
   return 0;
 }
 
@@ -483,6 +486,7 @@ int traverse_device_impl(Ctx* c, double* ex, double* ey, double* ez, double* pot
   a.theta2 = c->cfg.theta2; a.eps2 = c->cfg.eps2; a.sign = c->cfg.sign;
   a.ex = ex; a.ey = ey; a.ez = ez; a.pot = pot; a.work = work;
   a.np2p = c->np2p; a.nm2p = c->nm2p; a.gstat = c->gstat; a.queue = c->queue; a.nqueue = c->nxcd;
+  a.clock = c->clock;
   a.sys = c->nsys > 1 ? c->sys : nullptr;
   a.sysroot = c->sysroot;
   a.boxes = c->box;
@@ -490,17 +494,16 @@ int traverse_device_impl(Ctx* c, double* ex, double* ey, double* ez, double* pot
     return fail(c, PEPC_GPU_EINVAL, "traverse: periodic boundaries need a single system");
   a.nbox = c->periodic ? c->nbox : 1;
   a.vbox = c->periodic ? c->vbox : nullptr;
-  RECORD(c, 2);
   launch_walk(s, a, c->cfg.precision, c->walk_blocks, c->cfg.list_tile,
               std::max(c->cfg.group_size, c->cfg.group_pack));
   if (c->periodic && c->far_field)
     launch_lattice_far(s, c->n, c->xs, c->ys, c->zs, c->qs, c->lgeom, c->ml, c->fact, c->linv,
                        c->cfg.sign, c->lpart, c->ldpart, c->lom, c->ldip, c->mu,
                        c->fict, c->lcoef, ex, ey, ez, pot);
-  RECORD(c, 3);
   launch_walk_stats(s, a);
   HIPCHECK(c, hipGetLastError());
   c->walked = true;
+  if (!c->capturing) c->timed_walk = true;
   return 0;
 }
 
@@ -693,13 +696,8 @@ int pepc_gpu_create(void** out, const pepc_gpu_config* cfg) {
     return PEPC_GPU_EHIP;
   }
   c->own_stream = true;
-  for (auto& e : c->ev)
-    if (hipEventCreate(&e) != hipSuccess) {
-      delete c;
-      return PEPC_GPU_EHIP;
-    }
   if (dalloc(c, &c->box, 1) || dalloc(c, &c->sc, 1) || dalloc(c, &c->partial, kBoxParts * kBoxPartial) ||
-      dalloc(c, &c->box_tickets, kBoxParts) ||
+      dalloc(c, &c->box_tickets, kBoxParts) || dalloc(c, &c->clock, kClocks) ||
       dalloc(c, &c->queue, kQueueWords) ||
       hipHostMalloc((void**)&c->sc_host, sizeof(DevScalars), hipHostMallocDefault) != hipSuccess) {
     free_all(c);
@@ -713,6 +711,15 @@ int pepc_gpu_create(void** out, const pepc_gpu_config* cfg) {
       nx = 1;
     }
     c->nxcd = nx < 1 ? 1 : (nx > kMaxQueues ? kMaxQueues : nx);
+  }
+  {
+    int khz = 0;
+    if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, cfg->device) != hipSuccess ||
+        khz <= 0) {
+      (void)hipGetLastError();
+      khz = 100000;   // gfx9's constant clock
+    }
+    c->clock_ms = 1.0 / khz;
   }
   launch_zero_words(c->stream, c->queue, kQueueWords);
   launch_zero_words(c->stream, c->box_tickets, kBoxParts);
@@ -732,8 +739,6 @@ int pepc_gpu_destroy(void* p) {
   if (c->stream) (void)hipStreamSynchronize(c->stream);
   free_all(c);
   if (c->sc_host) (void)hipHostFree(c->sc_host);
-  for (auto& e : c->ev)
-    if (e) (void)hipEventDestroy(e);
   if (c->own_stream && c->stream) (void)hipStreamDestroy(c->stream);
   delete c;
   return 0;
@@ -1234,23 +1239,12 @@ int pepc_gpu_timings(void* p, double* t_grow_ms, double* t_walk_ms) {
   Ctx* c = as_ctx(p);
   if (!c) return PEPC_GPU_EINVAL;
   HIPCHECK(c, hipStreamSynchronize(c->stream));
-  float a = 0.f, b = 0.f;
-  // an interval whose events were not recorded reads -1; the failed query's
-  // error is cleared so that the next call's launch check does not see it
-  if (t_grow_ms) {
-    *t_grow_ms = -1.0;
-    if (c->grown) {
-      if (hipEventElapsedTime(&a, c->ev[0], c->ev[1]) == hipSuccess) *t_grow_ms = a;
-      else (void)hipGetLastError();
-    }
-  }
-  if (t_walk_ms) {
-    *t_walk_ms = -1.0;
-    if (c->walked) {
-      if (hipEventElapsedTime(&b, c->ev[2], c->ev[3]) == hipSuccess) *t_walk_ms = b;
-      else (void)hipGetLastError();
-    }
-  }
+  // what has not run outside a capture reads -1
+  double a = -1.0, b = -1.0;
+  if (c->timed_grow && !read_clock(c, &a, &b))
+    return fail(c, PEPC_GPU_EHIP, "timings: device clocks could not be read");
+  if (t_grow_ms) *t_grow_ms = c->grown && c->timed_grow ? a : -1.0;
+  if (t_walk_ms) *t_walk_ms = c->walked && c->timed_walk ? b : -1.0;
   return 0;
 }
 
@@ -1623,18 +1617,17 @@ int pepc_gpu_autotune(void* p, int64_t n, int64_t nsys, const int64_t* offsets, 
       r = grow_device_impl(c, n, x, y, z, q, ns, nsys > 1 ? offsets : nullptr);
       if (!r) r = traverse_device_impl(c, c->res[0], c->res[1], c->res[2], c->res[3], c->res[4]);
       if (!r) r = sync_impl(c, nullptr);
-      float tg = 0.f, tw = 0.f;
-      if (!r && (hipEventElapsedTime(&tg, c->ev[0], c->ev[1]) != hipSuccess ||
-                 hipEventElapsedTime(&tw, c->ev[2], c->ev[3]) != hipSuccess))
-        r = fail(c, PEPC_GPU_EHIP, "autotune: event timing failed");
+      double tg = 0.0, tw = 0.0;
+      if (!r && !read_clock(c, &tg, &tw))
+        r = fail(c, PEPC_GPU_EHIP, "autotune: device clocks could not be read");
       if (r) {
         c->cfg = saved;
         c->walk_blocks = saved_wb;
         c->grown = false;
         return r;
       }
-      if (rep > 0 && (double)tg + (double)tw < tbest) {
-        tbest = (double)tg + (double)tw;
+      if (rep > 0 && tg + tw < tbest) {
+        tbest = tg + tw;
         cd.tg = tg;
         cd.tw = tw;
       }

@@ -122,7 +122,8 @@ __global__ __launch_bounds__(kScanThreads) void scan_apply_kernel(const uint32_t
 // launches of 2 us fewer in every grow.
 __global__ __launch_bounds__(kScanThreads) void group_list_kernel(
     int64_t n, const uint32_t* __restrict__ gmark, const uint32_t* __restrict__ bsum, bool scanned,
-    uint32_t* __restrict__ gfirst, uint32_t* __restrict__ gcount, uint32_t* __restrict__ ngroups) {
+    uint32_t* __restrict__ gfirst, uint32_t* __restrict__ gcount, uint32_t* __restrict__ ngroups,
+    unsigned long long* __restrict__ clock) {
   __shared__ uint32_t tile[kScanTile];
   const int64_t base = (int64_t)blockIdx.x * kScanTile;
   uint32_t before = 0;
@@ -151,7 +152,10 @@ __global__ __launch_bounds__(kScanThreads) void group_list_kernel(
     gcount[g] = c[j];
     ++g;
   }
-  if (blockIdx.x + 1 == gridDim.x && threadIdx.x == 0) *ngroups = start + tot;
+  if (blockIdx.x + 1 == gridDim.x && threadIdx.x == 0) {
+    *ngroups = start + tot;
+    clock[kClockGrown] = wall_clock64();
+  }
 }
 
 // ---------------------------------------------------------------- radix sort
@@ -1023,13 +1027,14 @@ void launch_scan(hipStream_t s, const uint32_t* in, uint32_t* out, int64_t n, ui
 constexpr int64_t kGroupSumBlocks = 2048;
 
 void launch_group_list(hipStream_t s, int64_t n, const uint32_t* gmark, uint32_t* bsum,
-                       uint32_t* gfirst, uint32_t* gcount, uint32_t* ngroups) {
+                       uint32_t* gfirst, uint32_t* gcount, uint32_t* ngroups,
+                       unsigned long long* clock) {
   const int64_t nb = scan_blocks(n);
   const bool scanned = nb > kGroupSumBlocks;
   scan_reduce_kernel<<<(unsigned)nb, kScanThreads, 0, s>>>(gmark, n, bsum, true);
   if (scanned) scan_small_kernel<<<1, kScanThreads, 0, s>>>(bsum, (int)nb, nullptr);
   group_list_kernel<<<(unsigned)nb, kScanThreads, 0, s>>>(n, gmark, bsum, scanned, gfirst, gcount,
-                                                          ngroups);
+                                                          ngroups, clock);
 }
 
 // One stable pass over bits [shift, shift + nbits), output in (kout, vout).

@@ -894,7 +894,9 @@ __global__ void group_mark_kernel(int group_size, int pack, const NodeLink* __re
 
 // Root node of each system (level-0 nodes, one per non-empty system).
 __global__ void sysroot_kernel(const uint32_t* __restrict__ sys, const uint32_t* __restrict__ nfirst,
-                               uint32_t* __restrict__ sysroot, const DevScalars* __restrict__ sc) {
+                               uint32_t* __restrict__ sysroot, const DevScalars* __restrict__ sc,
+                               unsigned long long* __restrict__ clock) {
+  if (blockIdx.x + 1 == gridDim.x && threadIdx.x == 0) clock[kClockGrown] = wall_clock64();
   if (tree_broken(sc)) return;
   const int64_t nroot = sc->level_offset[1];
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < nroot;
@@ -940,8 +942,8 @@ void launch_tree_build(hipStream_t s, const TreeBuffers& t, int group_size, int 
   launch_upward(s, t);
   group_mark_kernel<<<grid_for(n), kT, 0, s>>>(group_size, group_pack, t.link, t.nfirst, t.node_rank,
                                                t.gmark, t.sc);
-  launch_group_list(s, n, t.gmark, t.bsum, t.gfirst, t.gcount, &t.sc->ngroups);
-  if (t.sys) sysroot_kernel<<<grid_for(t.nsys), kT, 0, s>>>(t.sys, t.nfirst, t.sysroot, t.sc);
+  launch_group_list(s, n, t.gmark, t.bsum, t.gfirst, t.gcount, &t.sc->ngroups, t.clock);
+  if (t.sys) sysroot_kernel<<<grid_for(t.nsys), kT, 0, s>>>(t.sys, t.nfirst, t.sysroot, t.sc, t.clock);
 }
 
 void launch_upward(hipStream_t s, const TreeBuffers& t) {

@@ -260,6 +260,7 @@ void walk_kernel(WalkArgs a) {
     a.sc->m2p = 0;
     a.sc->amb_nodes = 0;
     a.sc->walk_steps = 0;
+    a.clock[kClockWalk] = wall_clock64();
   }
   const double* __restrict__ TX = SINK ? a.tx : a.x;
   const double* __restrict__ TY = SINK ? a.ty : a.y;
@@ -663,7 +664,9 @@ void walk_kernel(WalkArgs a) {
 // clears the sums, which saves a launch before it.
 __global__ __launch_bounds__(256) void walk_stats_kernel(const uint32_t* __restrict__ gstat,
                                                         DevScalars* __restrict__ sc,
-                                                        uint32_t* __restrict__ queue) {
+                                                        uint32_t* __restrict__ queue,
+                                                        unsigned long long* __restrict__ clock) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) clock[kClockWalked] = wall_clock64();   // walk over
   const int64_t ng = sc->ngroups;
   if (blockIdx.x == 0 && threadIdx.x <= kMaxQueues) queue[kQueueStride * threadIdx.x] = 0;
   unsigned long long v[6] = {0, 0, 0, 0, 0, 0};
@@ -875,7 +878,7 @@ void launch_walk(hipStream_t s, const WalkArgs& a, int precision, int blocks, in
 }
 
 void launch_walk_stats(hipStream_t s, const WalkArgs& a) {
-  walk_stats_kernel<<<256, 256, 0, s>>>(a.gstat, a.sc, a.queue);
+  walk_stats_kernel<<<256, 256, 0, s>>>(a.gstat, a.sc, a.queue, a.clock);
 }
 
 // About kDirectBlocks blocks: eight of four waves for each of the 256 CUs.  A
