@@ -267,10 +267,17 @@ void launch_box(hipStream_t s, int64_t n, int nsys, const int64_t* soff, const d
                 const double* y, const double* z, const double* q, int force_cubic,
                 double* partial, uint32_t* tickets, DevBox* boxes, uint32_t* sys, DevScalars* sc,
                 unsigned long long* clock) {
-  // 16 particles a thread, as far as the partial results have room
-  int64_t parts = (n / nsys + kBoxThreads * 16 - 1) / (kBoxThreads * 16);
+  // Four particles a thread (a batch's largest system may be several times the
+  // mean), for one system only until there is a block per CU, then sixteen:
+  // the tickets are served one by one.  Four in place of sixteen: grow of
+  // 32,768 particles 140 -> 137 us, of 65,536 172 -> 166.
+  const int64_t mean = n / nsys;
+  int64_t parts = (mean + kBoxThreads * 4 - 1) / (kBoxThreads * 4);
+  if (nsys == 1 && parts > 256) {
+    parts = (mean + kBoxThreads * 16 - 1) / (kBoxThreads * 16);
+    if (parts < 256) parts = 256;
+  }
   const int64_t most = nsys > 1 ? kBoxParts / nsys : 1024;
-  if (nsys > 1) parts *= 4;   // the largest system may be several times the mean
   parts = parts < 1 ? 1 : parts;
   parts = parts > most ? (most < 1 ? 1 : most) : parts;
   box_kernel<<<(unsigned)(parts * nsys), kBoxThreads, 0, s>>>(
