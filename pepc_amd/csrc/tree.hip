@@ -660,12 +660,13 @@ __device__ __forceinline__ void quad_moments(const QuadTwig& t, int level, const
 // only workgroup barriers between, and a second kernel of one block the twigs
 // that cross tile ends: two launches in place of one per level.
 // Upward pass 91 -> 42 us for 1,777 particles, 134 -> 63 for 32,768 (with a
-// thread per twig, 95); grow 372 -> 358 us for 131,072.  Larger trees have
-// enough twigs per level for thread-per-twig launches, which need fewer lanes
-// per twig (1,048,576 particles: 333 us by thread-per-twig tiles, 223 by level).
+// thread per twig, 95).  Larger trees have enough twigs per level for launches
+// by level: with four lanes per twig in both, a grow of 65,536 particles takes
+// 168 us by tiles and 179 by level, of 131,072 215 and 197.
 constexpr int kUpT = 512;
-constexpr int kUpTiles = 256;
-constexpr int64_t kUpTilesMax = (int64_t)kUpTiles * kBfsTileSmall;   // 131,072 particles
+constexpr int kUpTiles = 128;
+constexpr int64_t kUpTilesMax = (int64_t)kUpTiles * kBfsTileSmall;   // 65,536 particles
+static_assert(kUpTiles % kWave == 0, "the crossing twigs are looked for by whole waves");
 
 struct UpTiles {
   const uint32_t* twig;   // [level][tile] rank of the tile's first twig of the level, level-major
@@ -762,9 +763,21 @@ __global__ __launch_bounds__(kUpT) void upward_cross_kernel(UpTiles t, UpArgs u)
 // The launch boundary orders a level's writes before the next level's reads
 // on every XCD; a single-launch scheme would need an agent-scope release per
 // node, which writes back the L2 of its XCD.
+// Levels of up to kUpQuadTwigs twigs, most of a large tree's, take four lanes
+// per twig as small trees do: the launch's quads hold them all at once, and a
+// level then costs the shorter chain.  Grow 262,144 particles 278 -> 245 us,
+// 1,048,576 clustered 569 -> 520, 4,194,304 1,384 -> 1,346; four lanes per
+// twig at every level 510 and 1,427.
+constexpr int64_t kUpQuadTwigs = 98304;   // 1,536 blocks of 64 quads
+
 __global__ __launch_bounds__(kT) void upward_level_kernel(int level, UpArgs u) {
   if (tree_broken(u.sc)) return;
   const int64_t tb = u.sc->twig_offset[level], te = u.sc->twig_offset[level + 1];
+  if (te - tb <= kUpQuadTwigs) {
+    const int64_t r = tb + (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) / 4;
+    if (r < te) quad_moments(quad_twig((uint32_t)r, u), level, u);
+    return;
+  }
   for (int64_t r = tb + blockIdx.x * (int64_t)blockDim.x + threadIdx.x; r < te;
        r += (int64_t)gridDim.x * blockDim.x) {
     const int64_t i = u.node_rank[r];
@@ -969,6 +982,7 @@ void launch_upward(hipStream_t s, const TreeBuffers& t) {
   // MI355X) with a twig-stride loop: the large levels keep every CU busy and
   // the many small levels launch few idle blocks.
   constexpr unsigned kUpBlocks = 1536;
+  static_assert(kUpQuadTwigs * 4 <= (int64_t)kUpBlocks * kT, "one quad per twig of a small level");
   for (int l = kMaxLevel; l >= 0; --l)
     upward_level_kernel<<<kUpBlocks, kT, 0, s>>>(l, u);
 }
