@@ -202,7 +202,7 @@ struct LatticeGeom {
   // Fictitious-charge correction: the neighbour boxes' fictitious charges
   // merged by lattice point, the points where all of them meet (and cancel)
   // left out.  fpt[4k..4k+2] = integer lattice coordinates of point k,
-  // fpt[4k+3] = mask of the charges there; lattice_mu_kernel writes
+  // fpt[4k+3] = mask of the charges there; lattice_coef_kernel writes
   // fpos[4k..4k+3] = {x, y, z, merged charge}.  nfpt = 0 otherwise.
   const int* fpt;
   double* fpos;
@@ -219,7 +219,7 @@ void launch_lattice_coefficients(hipStream_t s, const double* vec, int nb, doubl
                                  const double* fact, double2* mstar, double2* lstar,
                                  int maxiter, double2* ml);
 int lattice_moment_blocks(int64_t n);
-// Recurrence constants: inv[l(l+1)/2 + m] = 1 / ((l-m)(l+m)) for l > m,
+// Recurrence constants: inv[l(l+1)/2 + m] = b_lm (lattice.hip),
 // inv[kLatticeNM + m] = 1 / (2m); kLatticeNM + 21 doubles.
 void launch_lattice_inv(hipStream_t s, double* inv);
 // Per-step moments, mu and the field added to ex..pot (sign applied).
