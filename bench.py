@@ -63,7 +63,7 @@ def run_gpu(sys_, precision, group, steps, warmup, dev_inputs, pack=0):
     t1 = time.perf_counter()
     st = sol.sync()
     ms = (t1 - t0) * 1e3 / steps
-    # per-kernel device times (HIP events on the context stream), outside the timed region
+    # device times of grow and walk (pepc_gpu_timings), outside the timed region
     tg, tw = [], []
     for _ in range(min(steps, 5)):
         sol.grow(x, y, z, q, sync=False)

@@ -332,7 +332,7 @@ int pepc_gpu_replay_device(void *ctx, const double *x, const double *y, const do
  * device arrays (one system, or nsys batched systems with host offsets) for
  * every candidate of group size {16, 32, 64} x group pack {0, 32, 64} x list tile
  * (FP32 {64, 128}, FP64 {32, 64}) x persistent grid {full, half}: one
- * warm-up and reps timed runs each, device time (HIP events), best of reps.
+ * warm-up and reps timed runs each, device time (pepc_gpu_timings), best of reps.
  * The fastest becomes the context's configuration (read it back with
  * pepc_gpu_get_config); the tree is invalidated, so grow again.  out[0] is
  * the winner, out[1..] every candidate in the order tried (up to cap

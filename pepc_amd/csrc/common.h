@@ -32,7 +32,7 @@ struct DevBox {
   double cell[3];               // boxsize / 2^20, the refinement length
   double b2[kMaxLevel + 1];     // maxval(boxsize)^2 / 4^l
   uint32_t qsign;               // kQPositive | kQNegative: signs among the charges
-  uint32_t pad;
+  uint32_t mixed;               // both signs at the grow: FP32 walk records in the second form below
 };
 
 // A system whose charges all have one sign has no dipole moments: a node's
@@ -79,6 +79,8 @@ struct __align__(16) NodeLink {
 // quadrupole B = -3 (A2 - 2/3 tr I) with A2 = {2 quad, off-diagonals}, the
 // trace of quad, the dipole and the charge.
 // Slots: 0..2 Bxx Byy Bzz | 3 Bxy | 4 Byz | 5 Bzx | 6 tr | 7..9 p | 10 q
+// FP32 records of a system with charges of both signs (DevBox::mixed), the
+// reference's terms: 0 q | 1..3 p | 4..6 2 quad | 7 xy | 8 yz | 9 zx | 10 tr
 template <typename R>
 struct __align__(16) NodeMoments {
   R v[16];

@@ -52,6 +52,7 @@ __device__ void box_finalize(double mn[3], double mx[3], uint32_t sign, int forc
   box->b2[0] = m * m;
   for (int l = 1; l <= kMaxLevel; ++l) box->b2[l] = box->b2[l - 1] / 4.0;
   box->qsign = sign & (kQPositive | kQNegative);
+  box->mixed = box->qsign == (kQPositive | kQNegative) ? 1u : 0u;
   if (bad) atomicOr(&sc->flags, kFlagBadBox);
 }
 

@@ -333,7 +333,7 @@ __device__ __forceinline__ double walk_b2(const double* m, double boxlength2, in
   return INFINITY;
 }
 
-__device__ __forceinline__ void write_walk_forms(int64_t i, const double* m, double b2, int prec,
+__device__ __forceinline__ void write_walk_forms(int64_t i, const double* m, double b2, int prec, bool mixed,
                                                  NodeGeom* geom, NodeMoments<float>* wm32,
                                                  NodeMoments<double>* wm64) {
   NodeGeom g;
@@ -354,6 +354,13 @@ __device__ __forceinline__ void write_walk_forms(int64_t i, const double* m, dou
     o[2] = make_double4(w[8], w[9], w[10], w[11]);
   } else {
     float4* o = reinterpret_cast<float4*>(&wm32[i]);
+    if (mixed) {
+      w[0] = m[M_Q];
+      w[1] = m[M_PX]; w[2] = m[M_PY]; w[3] = m[M_PZ];
+      w[4] = 2.0 * m[M_QX]; w[5] = 2.0 * m[M_QY]; w[6] = 2.0 * m[M_QZ];
+      w[7] = m[M_XY]; w[8] = m[M_YZ]; w[9] = m[M_ZX];
+      w[10] = tr;
+    }
     o[0] = make_float4((float)w[0], (float)w[1], (float)w[2], (float)w[3]);
     o[1] = make_float4((float)w[4], (float)w[5], (float)w[6], (float)w[7]);
     o[2] = make_float4((float)w[8], (float)w[9], (float)w[10], 0.0f);
@@ -384,7 +391,8 @@ struct UpArgs {
 };
 
 __device__ void twig_moments(int64_t i, uint32_t c0, uint32_t nc, int level, const UpArgs& u) {
-  const double b2 = u.boxes[u.sys ? u.sys[u.nfirst[i]] : 0u].b2[level];
+  const DevBox& box = u.boxes[u.sys ? u.sys[u.nfirst[i]] : 0u];
+  const double b2 = box.b2[level];
   // The children's kinds come first (one byte each, one line); then every
   // child's charge, |charge| and centre are requested together, a leaf
   // child's from its geometry record (its particle's position and charge), a
@@ -480,7 +488,7 @@ __device__ void twig_moments(int64_t i, uint32_t c0, uint32_t nc, int level, con
   double2* out = reinterpret_cast<double2*>(u.mom + i * 16);
 #pragma unroll
   for (int k = 0; k < 8; ++k) out[k] = make_double2(m[2 * k], m[2 * k + 1]);
-  write_walk_forms(i, m, walk_b2(m, b2, u.mac_select), u.prec, u.geom, u.wm32, u.wm64);
+  write_walk_forms(i, m, walk_b2(m, b2, u.mac_select), u.prec, box.mixed != 0u, u.geom, u.wm32, u.wm64);
 }
 
 // ---- small trees: four lanes per twig, by tiles of particles
@@ -529,7 +537,9 @@ __device__ __forceinline__ QuadTwig quad_twig(uint32_t r, const UpArgs& u) {
 __device__ __forceinline__ void quad_moments(const QuadTwig& t, int level, const UpArgs& u) {
   const uint32_t lane = threadIdx.x & 3u;
   const uint32_t a = lane < 3u ? lane : 0u;   // lane 3 repeats component x
-  const double b2 = u.boxes[u.sys ? u.sys[u.nfirst[t.i]] : 0u].b2[level];
+  const DevBox& box = u.boxes[u.sys ? u.sys[u.nfirst[t.i]] : 0u];
+  const double b2 = box.b2[level];
+  const bool mixed = box.mixed != 0u && u.prec != kWalkFP64;
   double ca[8], cq[8], cw[8], pa[8], qa[8], oa[8];
 #pragma unroll
   for (uint32_t j = 0; j < 8; ++j) {
@@ -624,8 +634,8 @@ __device__ __forceinline__ void quad_moments(const QuadTwig& t, int level, const
     o[M_QX + a] = quad;
     o[M_XY + a] = off;
     g[a] = coc;
-    w[0] = 2.0 * tr - 6.0 * quad;
-    w[1] = -3.0 * off;
+    w[0] = mixed ? 2.0 * quad : 2.0 * tr - 6.0 * quad;
+    w[1] = mixed ? off : -3.0 * off;
     w[2] = dip;
   } else {
     o[M_Q] = charge;
@@ -642,7 +652,12 @@ __device__ __forceinline__ void quad_moments(const QuadTwig& t, int level, const
     u.link[t.i].count = count;
     u.kidtwig[t.i] = (uint8_t)(~t.leafmask & ((1u << t.nc) - 1u));
   }
-  const uint32_t k0 = lane < 3u ? a : 6u, k1 = lane < 3u ? 3u + a : 10u, k2 = lane < 3u ? 7u + a : 11u;
+  uint32_t k0 = lane < 3u ? a : 6u, k1 = lane < 3u ? 3u + a : 10u, k2 = lane < 3u ? 7u + a : 11u;
+  if (mixed) {
+    k0 = lane < 3u ? 4u + a : 10u;
+    k1 = lane < 3u ? 7u + a : 0u;
+    k2 = lane < 3u ? 1u + a : 11u;
+  }
   if (u.prec == kWalkFP64) {
     double* v = u.wm64[t.i].v;
     v[k0] = w[0]; v[k1] = w[1]; v[k2] = w[2];

@@ -19,7 +19,8 @@
 // appended to M2P / P2P lists staged in LDS and evaluated in batches: every
 // lane reads the same entry (LDS broadcast) and evaluates it for its target.
 //
-// Precision.  FP32 path: coordinates relative to the group's first particle
+// Precision.  FP32 path (of systems whose charges have one sign; the others
+// keep an evaluation of their own, see walk_group_mixed): coordinates relative to the group's first particle
 // (differences taken in FP64 once per node, then rounded), FP32 kernels with
 // fused multiply-add, FP32 partial sums per batch added to FP64 running sums
 // (more exact than the compensated FP32 sums they replace, with half the
@@ -221,6 +222,403 @@ __device__ __forceinline__ Span span_of(double lo, double hi) {
   return r;
 }
 
+// ---- FP32 groups of systems with charges of both signs
+// Close pairs of opposite charges make a trajectory of such a system amplify
+// any change of rounding, so its FP32 forces keep one fixed evaluation: the
+// reference's grouping of the terms, one target per lane, lists emptied whole,
+// Kahan sums, slices added in order.  With the form used for one-signed
+// systems, 20 steps of 8,192 to 262,144 thermal particles differed from this
+// one by 1e-5 in the velocities (their own FP32 error is 3e-5), and some pairs
+// and their order by far more; a single solve by 1e-7.
+// That form is the faster one (256 systems: 5.34 against 5.58 ms per solve;
+// 65,536 particles: 392 against 417 us); the sums of many slices by lane
+// instead of by shuffles took 65,536 sinks from 904 to 662 us.
+struct MixedAcc {
+  float s[4];  // running sums   ex, ey, ez, pot
+  float c[4];  // compensation
+  float p[4];  // partial sums of the current batch
+};
+
+// Entry {cx,cy,cz,q | px,py,pz,2qx | 2qy,2qz,xy,yz | zx,tr,-,-}.  With w = 1/r^2,
+// A2 = [[2qx,xy,zx],[xy,2qy,yz],[zx,yz,2qz]], g = A2 d, S2 = d.g, a = d.p + tr:
+//   phi = (1/r) (q - w (a - 1.5 w S2))
+//   E   = (w/r) (c d + p - 3 w g),   c = q - 3 w (a - 2.5 w S2)
+__device__ __forceinline__ void m2p_mixed(float dx, float dy, float dz, const Prec<float>::V4& b,
+                                          const Prec<float>::V4& c, const Prec<float>::V4& d, float q,
+                                          float eps2, float* p) {
+  using R = float;
+  using P = Prec<R>;
+  const R r2 = P::fm(dz, dz, P::fm(dy, dy, P::fm(dx, dx, eps2)));
+  const R rd = P::rsq(r2);
+  const R w = rd * rd;
+  const R rd3 = rd * w;
+  const R px = b.x, py = b.y, pz = b.z, qx2 = b.w;
+  const R qy2 = c.x, qz2 = c.y, xy = c.z, yz = c.w;
+  const R zx = d.x, tr = d.y;
+  const R gx = P::fm(qx2, dx, P::fm(xy, dy, zx * dz));
+  const R gy = P::fm(qy2, dy, P::fm(xy, dx, yz * dz));
+  const R gz = P::fm(qz2, dz, P::fm(yz, dy, zx * dx));
+  const R s2 = P::fm(dz, gz, P::fm(dy, gy, dx * gx));
+  const R av = P::fm(dz, pz, P::fm(dy, py, P::fm(dx, px, tr)));
+  const R bv = w * s2;
+  p[3] = P::fm(rd, P::fm(-w, P::fm(R(-1.5), bv, av), q), p[3]);
+  const R w3 = R(3) * w;
+  const R cc = P::fm(-w3, P::fm(R(-2.5), bv, av), q);
+  p[0] = P::fm(rd3, P::fm(cc, dx, P::fm(-w3, gx, px)), p[0]);
+  p[1] = P::fm(rd3, P::fm(cc, dy, P::fm(-w3, gy, py)), p[1]);
+  p[2] = P::fm(rd3, P::fm(cc, dz, P::fm(-w3, gz, pz)), p[2]);
+}
+
+// Kahan step on the batch's partial sums.
+__device__ __forceinline__ void fold_mixed(MixedAcc& a) {
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const float y = a.p[k] - a.c[k];
+    const float t = a.s[k] + y;
+    a.c[k] = (t - a.s[k]) - y;
+    a.s[k] = t;
+    a.p[k] = 0.0f;
+  }
+}
+
+// One group (targets a0 .. a0 + cnt - 1) of walk_kernel<float>, whose LDS
+// arrays it uses; traversal, decisions, counts and records are the same.
+template <int LM, bool PER, bool SINK>
+__device__ __forceinline__ void walk_group_mixed(const WalkArgs& a, uint32_t g, uint32_t a0,
+                                                 uint32_t cnt, uint32_t* stack,
+                                                 Prec<float>::V4 (*lm)[4], Prec<float>::V4* lp,
+                                                 uint32_t* lpi, uint2* opened) {
+  using R = float;
+  using V4 = Prec<float>::V4;
+  constexpr int kCap = kStackCap32;
+  const int lane = threadIdx.x;
+  const R eps2 = (R)a.eps2;
+  const double theta2 = a.theta2;
+  const double t_acc = theta2 * (1.0 - 1e-12), t_rej = theta2 * (1.0 + 1e-12);
+  const double* __restrict__ TX = SINK ? a.tx : a.x;
+  const double* __restrict__ TY = SINK ? a.ty : a.y;
+  const double* __restrict__ TZ = SINK ? a.tz : a.z;
+  // Lanes s*cnt .. s*cnt+cnt-1 form slice s (s < S = 64/cnt) and hold the
+  // group's targets in order; the 64 - S*cnt remaining lanes hold copies
+  // of targets for the box and take no part in the sums.
+  const uint32_t T = cnt;
+  const uint32_t S = kWave / T;
+  const uint32_t s = (uint32_t)lane / T;
+  const uint32_t t = (uint32_t)lane - s * T;
+  const bool valid = s < S;
+  const uint32_t tid = a0 + t;
+  const double xt = TX[tid], yt = TY[tid], zt = TZ[tid];
+  const double ox = uniform(xt), oy = uniform(yt), oz = uniform(zt);   // lane 0: target a0
+  const double lox = uniform_min(xt), loy = uniform_min(yt), loz = uniform_min(zt);
+  const double hix = -uniform_min(-xt), hiy = -uniform_min(-yt), hiz = -uniform_min(-zt);
+  // target position in the kernel's frame (FP64: set per box below)
+  R tx = R(0), ty = R(0), tz = R(0);
+  tx = (R)(xt - ox); ty = (R)(yt - oy); tz = (R)(zt - oz);
+
+  MixedAcc acc;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) { acc.s[k] = R(0); acc.c[k] = R(0); acc.p[k] = R(0); }
+
+  uint32_t sp = 0, nm = 0, np = 0, cnt_p2p = 0, cnt_m2p = 0, namb = 0, nsteps = 0;
+  uint32_t mac_lane = 0;   // this lane's MAC evaluations, summed over the wave at the end
+  bool overflow = false;
+  const uint32_t root = (!SINK && a.sys) ? a.sysroot[a.sys[a0]] : 0u;   // the group's own root
+  double sx = xt, sy = yt, sz = zt;    // targets of the current box: x - vbox
+
+  // Batches: entry k goes to slice k mod S; the loop count is uniform.
+  // FP32: two entries per pass (their LDS reads issued together), then the
+  // tail; FP64 keeps one entry per pass (register pressure).
+  auto flush_m2p = [&]() {
+    uint32_t kk = 0;
+    constexpr bool kPair = true;
+    const uint32_t n2 = (kPair && nm >= 2 * S) ? nm - 2 * S + 1 : 0;
+    if (kPair && valid) {
+      for (; kk < n2; kk += 2 * S) {
+        const uint32_t k = kk + s, k2 = k + S;
+        const V4 e0 = lm[k][0], e1 = lm[k][1], e2 = lm[k][2], e3 = lm[k][3];
+        const V4 f0 = lm[k2][0], f1 = lm[k2][1], f2 = lm[k2][2], f3 = lm[k2][3];
+        m2p_mixed(tx - (R)e0.x, ty - (R)e0.y, tz - (R)e0.z, e1, e2, e3, (R)e0.w, eps2, acc.p);
+        m2p_mixed(tx - (R)f0.x, ty - (R)f0.y, tz - (R)f0.z, f1, f2, f3, (R)f0.w, eps2, acc.p);
+      }
+    }
+    kk = n2 ? ((n2 - 1) / (2 * S) + 1) * 2 * S : 0;
+    for (; kk < nm; kk += S) {
+      const uint32_t k = kk + s;
+      if (valid && k < nm) {
+        const V4 e0 = lm[k][0], e1 = lm[k][1], e2 = lm[k][2], e3 = lm[k][3];
+        m2p_mixed(tx - (R)e0.x, ty - (R)e0.y, tz - (R)e0.z, e1, e2, e3, (R)e0.w, eps2, acc.p);
+      }
+    }
+    fold_mixed(acc);
+  };
+  // self term: the reference's rule (a zero separation from the leaf's
+  // particle) for sinks, the particle index for the grown particles
+  auto p2p_self = [&](uint32_t k) -> bool {
+    if constexpr (SINK) {
+      const uint32_t j = lpi[k];
+      return sx == a.x[j] && sy == a.y[j] && sz == a.z[j];
+    } else {
+      return lpi[k] == tid;   // mirror-box entries hold ~0u
+    }
+  };
+  // FP32: two entries per pass as for M2P (same per-lane order of terms)
+  auto flush_p2p = [&]() {
+    uint32_t kk = 0;
+    constexpr bool kPair = true;
+    const uint32_t n2 = (kPair && np >= 2 * S) ? np - 2 * S + 1 : 0;
+    if (kPair && valid) {
+      for (; kk < n2; kk += 2 * S) {
+        const uint32_t k = kk + s, k2 = k + S;
+        const V4 e = lp[k], f = lp[k2];
+        const bool self1 = p2p_self(k), self2 = p2p_self(k2);
+        p2p<R>(tx - (R)e.x, ty - (R)e.y, tz - (R)e.z, (R)e.w, eps2, self1, acc.p);
+        p2p<R>(tx - (R)f.x, ty - (R)f.y, tz - (R)f.z, (R)f.w, eps2, self2, acc.p);
+      }
+    }
+    kk = n2 ? ((n2 - 1) / (2 * S) + 1) * 2 * S : 0;
+    for (; kk < np; kk += S) {
+      const uint32_t k = kk + s;
+      if (valid && k < np) {
+        const V4 e = lp[k];
+        p2p<R>(tx - (R)e.x, ty - (R)e.y, tz - (R)e.z, (R)e.w, eps2, p2p_self(k), acc.p);
+      }
+    }
+    fold_mixed(acc);
+  };
+
+  const int nbox = PER ? a.nbox : 1;
+  for (int box = 0; box < nbox && !overflow; ++box) {
+  double vx = 0.0, vy = 0.0, vz = 0.0;
+  if constexpr (PER) { vx = a.vbox[3 * box]; vy = a.vbox[3 * box + 1]; vz = a.vbox[3 * box + 2]; }
+  const bool central = !PER || (vx == 0.0 && vy == 0.0 && vz == 0.0);
+  // targets of this box: x - vbox; group box likewise (rounding is monotone,
+  // so the shifted extremes are the extremes of the shifted targets)
+  sx = xt - vx; sy = yt - vy; sz = zt - vz;
+  const Span bx = span_of(lox - vx, hix - vx), by = span_of(loy - vy, hiy - vy),
+             bz = span_of(loz - vz, hiz - vz);
+  const double fox = ox - vx, foy = oy - vy, foz = oz - vz;   // FP32 node frame
+  if (lane == 0) stack[0] = root | kTwigBit;
+  sp = 1;
+  wave_order();
+  while (sp > 0) {
+    // Up to min(64, LM) nodes are read from the top of the stack (so one
+    // step's appends always fit an emptied list, positions nm + rank < LM);
+    // after the box test only the longest run of them whose pushes fit
+    // below the cap is visited, the rest stay on the stack.
+    constexpr uint32_t kPop = (uint32_t)(LM < kWave ? LM : kWave);
+    static_assert(kListP >= kWave, "P2P list must hold one full step");
+    const uint32_t m = sp < kPop ? sp : kPop;
+    if (nm + m > (uint32_t)LM) { wave_order(); flush_m2p(); nm = 0; }
+    if (np + m > (uint32_t)kListP) { wave_order(); flush_p2p(); np = 0; }
+    const bool has = (uint32_t)lane < m;
+    const uint32_t entry = has ? stack[sp - 1 - lane] : 0u;
+    const uint32_t node = entry & ~kTwigBit;
+    const bool twig_entry = (entry & kTwigBit) != 0u;
+    wave_order();
+    ++nsteps;
+
+    // All of a node's data is requested at once, before any decision, so a
+    // traversal step waits for one memory round trip.  A twig also brings
+    // its walk moments and its children's kinds; a leaf has neither.
+    NodeGeom gm = {0.0, 0.0, 0.0, 0.0};
+    NodeLink lk = {0u, 0u, 0u, 0u};
+    V4 w0, w1, w2;
+    uint32_t kids = 0u;
+    if (has) {
+      gm = a.geom[node];
+      lk = a.link[node];
+    }
+    if (has && twig_entry) {
+      kids = a.kidtwig[node];
+      const V4* src;
+      src = reinterpret_cast<const V4*>(&a.wm32[node]);
+      w0 = src[0]; w1 = src[1]; w2 = src[2];
+    }
+    // Decide from the group's bounding box when possible (margins cover
+    // every rounding of the exact per-target test below).
+    bool acc_ok = false, rej = false;
+    uint32_t macc = 0;
+    if (has && lk.nchild != 0u) {
+#pragma clang fp contract(fast)
+      const double dx = fabs(gm.cx - bx.c), dy = fabs(gm.cy - by.c), dz = fabs(gm.cz - bz.c);
+      const double ex = fmax(dx - bx.h, 0.0), ey = fmax(dy - by.h, 0.0), ez = fmax(dz - bz.h, 0.0);
+      const double fx = dx + bx.h, fy = dy + by.h, fz = dz + bz.h;
+      const double dmin2 = ex * ex + ey * ey + ez * ez;
+      const double dmax2 = fx * fx + fy * fy + fz * fz;
+      acc_ok = t_acc * dmin2 > gm.b2;
+      rej = !acc_ok && t_rej * dmax2 <= gm.b2;
+      macc = acc_ok ? cnt : (rej ? 1u : 0u);
+    }
+    // Visit lanes 0 .. k-1 for the largest k whose step leaves at most kCap
+    // entries: sp - k + (children of lanes < k, counted for every twig the
+    // box did not accept) <= kCap.  k >= 1 always, so the stack passes the
+    // cap only by the one-node steps of a depth-first descent (within
+    // kStackSlack), and k is never below the worst-case count
+    // (kCap - sp) / 7.  Nodes k .. m-1 stay on the stack unvisited: none of
+    // their decisions is counted.
+    // While the worst case fits (7 net pushes per node), all m are visited
+    // without the search.
+    uint32_t k = m;
+    if ((int)(7u * m) > (int)kCap - (int)sp) {
+      const uint32_t pmax = (has && lk.nchild != 0u && !acc_ok) ? lk.nchild : 0u;
+      uint32_t ptot;
+      const uint32_t pex = wave_exclusive_scan16(pmax, &ptot);
+      const bool fits = has && (int)(pex + pmax) - (lane + 1) <= (int)kCap - (int)sp;
+      const unsigned long long fm = __ballot(fits);
+      k = fm ? 64u - (uint32_t)__clzll((long long)fm) : 1u;
+    }
+    const bool keep = (uint32_t)lane < k;
+    sp -= k;
+    const bool leaf = keep && lk.nchild == 0u;
+    const bool twig = keep && lk.nchild != 0u;
+    // Undecided nodes: exact per-target test.  Every slice holds all the
+    // targets, so slice s tests the s-th undecided node of the batch and S
+    // nodes are settled per pass.  The nodes' centres and b^2 are staged in
+    // the free tail of the M2P list (entries nm .. nm + m - 1, which this
+    // step's appends overwrite only after the tests), so each slice reads
+    // its node with one broadcast load per pass.
+    const bool amb_me = twig && !acc_ok && !rej;
+    const unsigned long long amb = __ballot(amb_me);
+    const uint32_t na = (uint32_t)popc64(amb);
+    namb += na;
+    if (na) {
+      const uint32_t my_rank = mask_rank(amb);
+      if (amb_me) {
+        double2* st = reinterpret_cast<double2*>(&lm[nm + my_rank][0]);
+        st[0] = make_double2(gm.cx, gm.cy);
+        st[1] = make_double2(gm.cz, gm.b2);
+      }
+      wave_order();
+      for (uint32_t base = 0; base < na; base += S) {
+        const uint32_t r = base + s;
+        const bool active = valid && r < na;
+        double2 c0 = make_double2(0.0, 0.0), c1 = c0;
+        if (active) {
+          const double2* st = reinterpret_cast<const double2*>(&lm[nm + r][0]);
+          c0 = st[0];
+          c1 = st[1];
+        }
+        const bool fail = active && mac_fails(sx, sy, sz, c0.x, c0.y, c1.x, c1.y, theta2);
+        const unsigned long long ball = __ballot(fail);
+        if (amb_me && my_rank >= base && my_rank < base + S) {
+          const uint32_t rr = my_rank - base;
+          const unsigned long long fm =
+              (ball >> (rr * T)) & (T == 64 ? ~0ull : ((1ull << T) - 1ull));
+          if (fm == 0ull) { acc_ok = true; macc = cnt; }
+          else { rej = true; macc = (uint32_t)__ffsll((long long)fm); }
+        }
+      }
+      wave_order();
+    }
+    mac_lane += twig ? macc : 0u;
+
+    const bool take_m = twig && acc_ok;
+    const unsigned long long am = __ballot(take_m);
+    const unsigned long long pm = __ballot(leaf);
+    if (take_m) {
+      const uint32_t pos = nm + mask_rank(am);
+      V4 e0;
+      e0 = V4{(float)(gm.cx - fox), (float)(gm.cy - foy), (float)(gm.cz - foz), 0.0f};
+      // w0 = {q, px, py, pz}, w1 = {2qx, 2qy, 2qz, xy}, w2 = {yz, zx, tr, -}
+      e0.w = w0.x;
+      V4 e1, e2, e3;
+      e1.x = w0.y; e1.y = w0.z; e1.z = w0.w; e1.w = w1.x;
+      e2.x = w1.y; e2.y = w1.z; e2.z = w1.w; e2.w = w2.x;
+      e3.x = w2.y; e3.y = w2.z; e3.z = 0; e3.w = 0;
+      lm[pos][0] = e0; lm[pos][1] = e1; lm[pos][2] = e2; lm[pos][3] = e3;
+    }
+    if (leaf) {
+      const uint32_t pos = np + mask_rank(pm);
+      V4 e;
+      e = V4{(float)(gm.cx - fox), (float)(gm.cy - foy), (float)(gm.cz - foz), (float)gm.b2};
+      lp[pos] = e;
+      lpi[pos] = (SINK || central) ? lk.first : ~0u;
+    }
+    const uint32_t nma = (uint32_t)popc64(am), npa = (uint32_t)popc64(pm);
+    nm += nma; np += npa; cnt_m2p += nma; cnt_p2p += npa;
+
+    // children of the opened nodes, as in walk_kernel
+    const bool open = twig && !acc_ok;
+    const unsigned long long om = __ballot(open);
+    if (open) opened[mask_rank(om)] = make_uint2(lk.first, lk.nchild | (kids << 8));
+    wave_order();
+    const int no = (int)popc64(om);
+    for (int o = 0; o < no; o += 8) {
+      const int j = o + (lane >> 3);
+      const uint32_t c = (uint32_t)lane & 7u;
+      const uint2 rec = opened[j & (kWave - 1)];
+      const bool child = j < no && c < (rec.y & 0xFFu);
+      const unsigned long long cm = __ballot(child);
+      const uint32_t nc = (uint32_t)popc64(cm);
+      if (sp + nc > (uint32_t)(kCap + kStackSlack)) { overflow = true; break; }
+      if (child) stack[sp + mask_rank(cm)] = (rec.x + c) | (((rec.y >> (8u + c)) & 1u) << 31);
+      sp += nc;
+    }
+    if (overflow) break;
+    wave_order();
+  }
+  if constexpr (PER && SINK) {   // next box shifts the targets
+    wave_order();
+    if (nm) flush_m2p();
+    if (np) flush_p2p();
+    nm = 0; np = 0;
+  }
+  }   // boxes
+  wave_order();
+  if (nm) flush_m2p();
+  if (np) flush_p2p();
+
+  // Combine the slices in FP64, in order (target t lives in lanes t, t+T, ...):
+  // many slices through the list's LDS, one lane per sum, few by shuffles.
+  double out[4];
+  const bool by_lane = S > 4u;   // then 4 T sums fit the wave
+#pragma unroll
+  for (int k = 0; k < 4; ++k) out[k] = (double)acc.s[k] - (double)acc.c[k];
+  if (by_lane) {
+    double* sums = reinterpret_cast<double*>(&lm[0][0]);   // 4 x 64: 2 KB of the list
+    static_assert(sizeof(V4) * 4 * LM >= 4 * kWave * sizeof(double), "the list holds the sums");
+    wave_order();
+#pragma unroll
+    for (int k = 0; k < 4; ++k) sums[k * kWave + lane] = out[k];
+    wave_order();
+    const uint32_t k = s < 4u ? s : 3u;   // lane k T + t: component k of target t
+    double v = sums[k * kWave + t];
+    for (uint32_t o = 1; o < S; ++o) v += sums[k * kWave + t + o * T];
+    double* dst = k == 0u ? a.ex : k == 1u ? a.ey : k == 2u ? a.ez : a.pot;
+    if (s < 4u) dst[tid] = v * a.sign;
+    wave_order();
+  } else {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const double v0 = out[k];
+      double v = v0;
+      for (uint32_t o = 1; o < S; ++o) v += __shfl(v0, (int)(t + o * T));
+      out[k] = v * a.sign;
+    }
+  }
+  if (overflow) {
+    if (lane == 0) atomicOr(&a.sc->flags, kFlagStackOverflow);
+  }
+  if (s == 0 && valid) {
+    if (!by_lane) {
+      a.ex[tid] = out[0];
+      a.ey[tid] = out[1];
+      a.ez[tid] = out[2];
+      a.pot[tid] = out[3];
+    }
+    a.work[tid] = (SINK ? 0.0 : 1.0) + (double)(cnt_p2p + cnt_m2p);
+    a.np2p[tid] = cnt_p2p;
+    a.nm2p[tid] = cnt_m2p;
+  }
+  const unsigned long long nmac = SINK ? 0ull : wave_sum((unsigned long long)mac_lane);
+  if (!SINK && lane == 0) {   // per-group record, summed by walk_stats_kernel
+    uint4* gs = reinterpret_cast<uint4*>(a.gstat + 8 * (size_t)g);
+    gs[0] = make_uint4((uint32_t)nmac, cnt_p2p, cnt_m2p, namb);
+    gs[1] = make_uint4(nsteps, cnt, 0u, 0u);
+  }
+  wave_order();
+}
+
 // LM: capacity of the M2P list staged in LDS (the list tile); the P2P list
 // holds kListP entries.  The default tiles (LM * sizeof(R) = 256 bytes per
 // float component: FP32 64, FP64 32) leave LDS for four one-wave workgroups
@@ -282,6 +680,13 @@ void walk_kernel(WalkArgs a) {
     uint32_t a0, cnt;
     if (!SINK || a.gfirst) { a0 = uniform(a.gfirst[g]); cnt = uniform(a.gcount[g]); }
     else { a0 = g; cnt = 1u; }
+    const DevBox& sbox = a.boxes[(!SINK && a.sys) ? a.sys[a0] : 0u];   // the group's system
+    if constexpr (sizeof(R) == 4) {
+      if (uniform(sbox.mixed)) {
+        walk_group_mixed<LM, PER, SINK>(a, g, a0, cnt, stack, lm, lp, lpi, opened);
+        continue;
+      }
+    }
     const uint32_t T = cnt;
     const uint32_t W = (T + (uint32_t)NT - 1u) / (uint32_t)NT;
     const bool two = NT == 2 && T > 1u;
@@ -317,7 +722,7 @@ void walk_kernel(WalkArgs a) {
     // Kept remainders (fewer than S entries) shorten the next steps' lists;
     // above 16 slices, where a list is a few passes at most, lists are emptied.
     const bool keep_rest = S <= 16u;
-    const bool dipoles = uniform(a.boxes[(!SINK && a.sys) ? a.sys[a0] : 0u].qsign) == 3u;
+    const bool dipoles = uniform(sbox.qsign) == 3u;
     uint32_t sp = 0, nm = 0, np = 0, cnt_p2p = 0, cnt_m2p = 0, namb = 0, nsteps = 0;
     uint32_t mac_lane = 0;   // this lane's MAC evaluations, summed over the wave at the end
     bool overflow = false;
