@@ -230,9 +230,11 @@ __device__ __forceinline__ Span span_of(double lo, double hi) {
 // systems, 20 steps of 8,192 to 262,144 thermal particles differed from this
 // one by 1e-5 in the velocities (their own FP32 error is 3e-5), and some pairs
 // and their order by far more; a single solve by 1e-7.
-// That form is the faster one (256 systems: 5.34 against 5.58 ms per solve;
-// 65,536 particles: 392 against 417 us); the sums of many slices by lane
-// instead of by shuffles took 65,536 sinks from 904 to 662 us.
+// That form is the faster one (256 systems: 5.34 against 5.53 ms per solve;
+// 65,536 particles: 392 against 409 us); the sums of many slices by lane
+// instead of by shuffles took 65,536 sinks from 904 to 662 us.  The children
+// are pushed by their parent's lane: eight lanes per parent, as in
+// walk_kernel, spill here (256 systems 5.53 -> 5.67 ms).
 struct MixedAcc {
   float s[4];  // running sums   ex, ey, ez, pot
   float c[4];  // compensation
@@ -287,7 +289,7 @@ template <int LM, bool PER, bool SINK>
 __device__ __forceinline__ void walk_group_mixed(const WalkArgs& a, uint32_t g, uint32_t a0,
                                                  uint32_t cnt, uint32_t* stack,
                                                  Prec<float>::V4 (*lm)[4], Prec<float>::V4* lp,
-                                                 uint32_t* lpi, uint2* opened) {
+                                                 uint32_t* lpi) {
   using R = float;
   using V4 = Prec<float>::V4;
   constexpr int kCap = kStackCap32;
@@ -537,24 +539,13 @@ __device__ __forceinline__ void walk_group_mixed(const WalkArgs& a, uint32_t g, 
     const uint32_t nma = (uint32_t)popc64(am), npa = (uint32_t)popc64(pm);
     nm += nma; np += npa; cnt_m2p += nma; cnt_p2p += npa;
 
-    // children of the opened nodes, as in walk_kernel
-    const bool open = twig && !acc_ok;
-    const unsigned long long om = __ballot(open);
-    if (open) opened[mask_rank(om)] = make_uint2(lk.first, lk.nchild | (kids << 8));
-    wave_order();
-    const int no = (int)popc64(om);
-    for (int o = 0; o < no; o += 8) {
-      const int j = o + (lane >> 3);
-      const uint32_t c = (uint32_t)lane & 7u;
-      const uint2 rec = opened[j & (kWave - 1)];
-      const bool child = j < no && c < (rec.y & 0xFFu);
-      const unsigned long long cm = __ballot(child);
-      const uint32_t nc = (uint32_t)popc64(cm);
-      if (sp + nc > (uint32_t)(kCap + kStackSlack)) { overflow = true; break; }
-      if (child) stack[sp + mask_rank(cm)] = (rec.x + c) | (((rec.y >> (8u + c)) & 1u) << 31);
-      sp += nc;
-    }
-    if (overflow) break;
+    const uint32_t nc = (twig && !acc_ok) ? lk.nchild : 0u;   // at most 8
+    uint32_t tot;
+    const uint32_t excl = wave_exclusive_scan16(nc, &tot);
+    if (sp + tot > (uint32_t)(kCap + kStackSlack)) { overflow = true; break; }
+    for (uint32_t k = 0; k < nc; ++k)
+      stack[sp + excl + k] = (lk.first + k) | (((kids >> k) & 1u) ? kTwigBit : 0u);
+    sp += tot;
     wave_order();
   }
   if constexpr (PER && SINK) {   // next box shifts the targets
@@ -683,7 +674,7 @@ void walk_kernel(WalkArgs a) {
     const DevBox& sbox = a.boxes[(!SINK && a.sys) ? a.sys[a0] : 0u];   // the group's system
     if constexpr (sizeof(R) == 4) {
       if (uniform(sbox.mixed)) {
-        walk_group_mixed<LM, PER, SINK>(a, g, a0, cnt, stack, lm, lp, lpi, opened);
+        walk_group_mixed<LM, PER, SINK>(a, g, a0, cnt, stack, lm, lp, lpi);
         continue;
       }
     }
