@@ -75,10 +75,10 @@ struct __align__(16) NodeLink {
   uint32_t level;
 };
 
-// Moments in the form the M2P kernel evaluates (see walk.hip): the traceless
-// quadrupole B = -3 (A2 - 2/3 tr I) with A2 = {2 quad, off-diagonals}, the
-// trace of quad, the dipole and the charge.
-// Slots: 0..2 Bxx Byy Bzz | 3 Bxy | 4 Byz | 5 Bzx | 6 tr | 7..9 p | 10 q
+// Moments in the form the M2P kernel evaluates (see walk.hip): -3 times the
+// quadrupole matrix A2 = {2 quad, off-diagonals}, twice the trace of quad, the
+// dipole and the charge.
+// Slots: 0..2 -3 A2 xx yy zz | 3 xy | 4 yz | 5 zx | 6 2 tr | 7..9 p | 10 q
 // FP32 records of a system with charges of both signs (DevBox::mixed), the
 // reference's terms: 0 q | 1..3 p | 4..6 2 quad | 7 xy | 8 yz | 9 zx | 10 tr
 template <typename R>

@@ -341,9 +341,9 @@ __device__ __forceinline__ void write_walk_forms(int64_t i, const double* m, dou
   geom[i] = g;
   double w[12];
   const double tr = (m[M_QX] + m[M_QY]) + m[M_QZ];
-  w[0] = 2.0 * tr - 6.0 * m[M_QX]; w[1] = 2.0 * tr - 6.0 * m[M_QY]; w[2] = 2.0 * tr - 6.0 * m[M_QZ];
+  w[0] = -6.0 * m[M_QX]; w[1] = -6.0 * m[M_QY]; w[2] = -6.0 * m[M_QZ];
   w[3] = -3.0 * m[M_XY]; w[4] = -3.0 * m[M_YZ]; w[5] = -3.0 * m[M_ZX];
-  w[6] = tr;
+  w[6] = 2.0 * tr;
   w[7] = m[M_PX]; w[8] = m[M_PY]; w[9] = m[M_PZ];
   w[10] = m[M_Q];
   w[11] = 0.0;
@@ -634,7 +634,7 @@ __device__ __forceinline__ void quad_moments(const QuadTwig& t, int level, const
     o[M_QX + a] = quad;
     o[M_XY + a] = off;
     g[a] = coc;
-    w[0] = mixed ? 2.0 * quad : 2.0 * tr - 6.0 * quad;
+    w[0] = mixed ? 2.0 * quad : -6.0 * quad;
     w[1] = mixed ? off : -3.0 * off;
     w[2] = dip;
   } else {
@@ -645,7 +645,7 @@ __device__ __forceinline__ void quad_moments(const QuadTwig& t, int level, const
     double m[16];
     m[M_BMAX] = bmax;
     g[3] = walk_b2(m, b2, u.mac_select);
-    w[0] = tr;
+    w[0] = mixed ? tr : 2.0 * tr;
     w[1] = charge;
     w[2] = 0.0;
     u.link[t.i].nchild = t.nc;

@@ -31,10 +31,10 @@
 // issues an FP32 instruction every 3 clocks per SIMD and every other kind
 // (FP64, integer, compares, any with a scalar operand) every 4.3 to 4.8; the
 // 4.2M-particle explosion at theta 0.6 issued 4.36e9 VALU instructions at
-// 3.0 clocks each.  So the design counts instructions: traceless moments and
-// no dipole terms for one-signed charges (41 -> 35 per pair), list remainders
-// kept so that passes are full, one ballot transposition for the exact tests
-// and one for the pushes.  3.76e9 instructions, walk 5.88 -> 5.24 ms (FP64
+// 3.0 clocks each.  So the design counts instructions: no dipole
+// terms for one-signed charges (41 -> 36 per pair), list remainders kept so
+// that passes are full, one ballot transposition for the exact tests and one
+// for the pushes.  3.76e9 instructions, walk 5.88 -> 5.24 ms (FP64
 // 11.56 -> 10.52, theta 0.3 at 500,009 particles 2.90 -> 2.58).
 //
 // Periodic systems (PER): the group walks the tree once per lattice vector
@@ -95,14 +95,18 @@ struct Acc {
   R p[4];       // partial sums of the current batch
 };
 
-// M2P.  With w = 1/r^2, the node's traceless quadrupole B = -3 (A2 - 2/3 tr I)
-// (A2 = 2 Qt, tr = trace Qt), g = B d, X = d.g + 2 tr eps^2 and p = the dipole:
-//   phi = (1/r) (q - w (d.p + 0.5 w X))
-//   E   = (w/r) (c d + p + w g),   c = q - w (3 d.p + 2.5 w X)
-// which is phi and -grad phi of module_coulomb_kernels.f90:60-145: the trace
-// terms of that form cancel against the trace part of d.A2 d up to eps^2.
-// The separation d is target minus centre of charge.
-// Entry: {cx,cy,cz,q | Bxx,Byy,Bzz,Bxy | Byz,Bzx,2 tr eps^2,px | py,pz,-,-}.
+// M2P.  With w = 1/r^2, A2 = 2 Qt, tr = trace Qt, h = -3 w A2 d, y = d.h + 2 tr
+// and p = the dipole:
+//   phi = (1/r) (q - w (d.p + 0.5 y))
+//   E   = (w/r) (c d + p + h),   c = q - w (3 d.p + 2.5 y - 2 tr)
+// which is phi and -grad phi of module_coulomb_kernels.f90:60-145.  The
+// separation d is target minus centre of charge.
+// Every factor lies between r^-3 and the moments times r, so for charges near
+// one FP32 holds separations and softenings from 1e-11 to 1e12.  E summed as
+// r^-3 c d + r^-5 B d with a traceless B is an instruction shorter (4,194,304
+// particles: solve 6.62 ms against 6.66), but r^-5 leaves FP32 below a
+// separation of 2e-8 and above 4e7.
+// Entry: {cx,cy,cz,q | -3 A2: xx,yy,zz,xy | yz,zx, 2 tr,px | py,pz,-,-}.
 // Without a dipole (DIP = false) its terms and its words are left out.
 template <typename R, bool DIP>
 __device__ __forceinline__ void m2p(R dx, R dy, R dz, R q, const typename Prec<R>::V4& b,
@@ -112,28 +116,25 @@ __device__ __forceinline__ void m2p(R dx, R dy, R dz, R q, const typename Prec<R
   const R rd = P::rsq(r2);
   const R w = rd * rd;
   const R rd3 = rd * w;
-  const R gx = P::fm(b.x, dx, P::fm(b.w, dy, c.y * dz));
-  const R gy = P::fm(b.y, dy, P::fm(b.w, dx, c.x * dz));
-  const R gz = P::fm(b.z, dz, P::fm(c.x, dy, c.y * dx));
-  const R x = P::fm(dz, gz, P::fm(dy, gy, P::fm(dx, gx, c.z)));
-  const R y = w * x;
+  const R hx = w * P::fm(b.x, dx, P::fm(b.w, dy, c.y * dz));
+  const R hy = w * P::fm(b.y, dy, P::fm(b.w, dx, c.x * dz));
+  const R hz = w * P::fm(b.z, dz, P::fm(c.x, dy, c.y * dx));
+  const R y = P::fm(dz, hz, P::fm(dy, hy, P::fm(dx, hx, c.z)));
+  R vx = hx, vy = hy, vz = hz, cc;
   if constexpr (DIP) {
     const R px = c.w;
     const R av = P::fm(dz, pz, P::fm(dy, py, dx * px));
     p[3] = P::fm(rd, P::fm(-w, P::fm(R(0.5), y, av), q), p[3]);
-    const R cc = P::fm(-w, P::fm(R(2.5), y, R(3) * av), q);
-    p[0] = P::fm(rd3, P::fm(cc, dx, P::fm(w, gx, px)), p[0]);
-    p[1] = P::fm(rd3, P::fm(cc, dy, P::fm(w, gy, py)), p[1]);
-    p[2] = P::fm(rd3, P::fm(cc, dz, P::fm(w, gz, pz)), p[2]);
+    cc = P::fm(-w, P::fm(R(2.5), y, P::fm(R(3), av, -c.z)), q);
+    vx += px; vy += py; vz += pz;
   } else {
     const R y2 = w * y;
     p[3] = P::fm(rd, P::fm(R(-0.5), y2, q), p[3]);
-    const R e1 = rd3 * P::fm(R(-2.5), y2, q);
-    const R e5 = rd3 * w;
-    p[0] = P::fm(e5, gx, P::fm(e1, dx, p[0]));
-    p[1] = P::fm(e5, gy, P::fm(e1, dy, p[1]));
-    p[2] = P::fm(e5, gz, P::fm(e1, dz, p[2]));
+    cc = P::fm(w, c.z, P::fm(R(-2.5), y2, q));
   }
+  p[0] = P::fm(rd3, P::fm(cc, dx, vx), p[0]);
+  p[1] = P::fm(rd3, P::fm(cc, dy, vy), p[1]);
+  p[2] = P::fm(rd3, P::fm(cc, dz, vz), p[2]);
 }
 
 // P2P (module_coulomb_kernels.f90:242-257): phi = q/r, E = q d / r^3.
@@ -638,7 +639,7 @@ void walk_kernel(WalkArgs a) {
 
   const int lane = threadIdx.x;
   constexpr bool kPair = sizeof(R) == 4 && NT == 1;
-  const R eps2 = (R)a.eps2, eps22 = (R)(2.0 * a.eps2);
+  const R eps2 = (R)a.eps2;
   const double theta2 = a.theta2;
   const double t_acc = theta2 * (1.0 - 1e-12), t_rej = theta2 * (1.0 + 1e-12);
   const uint32_t ngroups = SINK ? a.nsink_groups : a.sc->ngroups;
@@ -953,15 +954,13 @@ void walk_kernel(WalkArgs a) {
       const unsigned long long pm = __ballot(leaf);
       if (take_m) {
         const uint32_t pos = nm + mask_rank(am);
-        // w0 = {Bxx,Byy,Bzz,Bxy}, w1 = {Byz,Bzx,tr,px}, w2 = {py,pz,q,-}
+        // the record is the entry's words in order, with q behind pz
         V4 e0;
         if constexpr (sizeof(R) == 4)
           e0 = V4{(float)(gm.cx - fox), (float)(gm.cy - foy), (float)(gm.cz - foz), w2.z};
         else
           e0 = V4{gm.cx, gm.cy, gm.cz, w2.z};
-        V4 e2 = w1;
-        e2.z *= eps22;
-        lm[pos][0] = e0; lm[pos][1] = w0; lm[pos][2] = e2; lm[pos][3] = w2;
+        lm[pos][0] = e0; lm[pos][1] = w0; lm[pos][2] = w1; lm[pos][3] = w2;
       }
       if (leaf) {
         const uint32_t pos = np + mask_rank(pm);
