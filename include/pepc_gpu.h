@@ -243,7 +243,10 @@ int pepc_gpu_read_walk(void *ctx, int64_t gcap, uint32_t *gfirst, uint32_t *gcou
  * periodic form: every source in every mirror box, self only in the central
  * box (:80-93), plus the lattice far field at the targets from all sources
  * (:130-137), after which pepc_gpu_lattice_get reports these sources'
- * moments.  Asynchronous on the context's stream. */
+ * moments.  Asynchronous on the context's stream.  The first call that splits
+ * the sum over the sources allocates 32 MB, which the context keeps; calls on
+ * different streams take turns at it.  On a stream under capture (and without
+ * memory) the sum is not split and uses none of it. */
 int pepc_gpu_direct_device(void *ctx, int64_t n, const double *x, const double *y,
                            const double *z, const double *q, int64_t ntest,
                            const int64_t *testidx, double eps2, double sign, double *ex,

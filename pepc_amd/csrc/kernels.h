@@ -324,7 +324,14 @@ struct DirectPlan {
   int span;
   int64_t tblocks, ranges, range, partials;
 };
+constexpr int kDirectT = 256;             // threads per block
+constexpr int64_t kDirectBlocks = 2048;   // blocks aimed at
 DirectPlan direct_plan(int64_t n, int64_t ntest);
+// Doubles that hold the partial sums of every split: four per thread, and a
+// plan with several partials per target has fewer than 2 kDirectBlocks blocks
+// (ranges are rounded up: at most kDirectBlocks + tblocks, tblocks below
+// kDirectBlocks).
+constexpr int64_t kDirectWork = 4 * kDirectT * 2 * kDirectBlocks;
 // nbox mirror-box vectors vbox (nullptr: open boundaries).  work: room for
 // 4 * ntest * direct_plan(n, ntest).partials doubles, or nullptr (slower).
 void launch_direct(hipStream_t s, int64_t n, const double* x, const double* y, const double* z,

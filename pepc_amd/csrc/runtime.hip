@@ -114,7 +114,7 @@ struct Ctx {
   double2* lom = nullptr;
   // direct sum: partial sums
   double* dwork = nullptr;
-  int64_t dwork_cap = 0;
+  hipEvent_t dwork_used = nullptr;   // behind its last use
   // sinks (traversal of other particles)
   int64_t scap = 0, sk_m = 0;
   int sk_mode = 0;
@@ -739,6 +739,7 @@ int pepc_gpu_destroy(void* p) {
   if (c->stream) (void)hipStreamSynchronize(c->stream);
   free_all(c);
   if (c->sc_host) (void)hipHostFree(c->sc_host);
+  if (c->dwork_used) (void)hipEventDestroy(c->dwork_used);
   if (c->own_stream && c->stream) (void)hipStreamDestroy(c->stream);
   delete c;
   return 0;
@@ -1130,31 +1131,41 @@ int pepc_gpu_read_walk(void* p, int64_t gcap, uint32_t* gfirst, uint32_t* gcount
   return 0;
 }
 
-// Partial sums of the split direct sum: kept by the context, at most about
-// 19 MB (256 targets x 2304 blocks x 4 sums) plus one sum per target.  nullptr
-// (the unsplit form) when there is no memory for them or when they would have
-// to be allocated on a stream under capture.
+// Partial sums of the split direct sum: one block of kDirectWork doubles, kept
+// by the context from the first call that splits and never moved.  Calls on
+// different streams take turns: each waits on its stream for the event that
+// the one before recorded behind its kernels (direct_release).  nullptr (the
+// unsplit form) without memory, and on every stream under capture: a graph
+// would hold the block's address and write it beside later calls.
 static double* direct_workspace(Ctx* c, hipStream_t s, int64_t n, int64_t ntest) {
   if (ntest <= 0) return nullptr;
   const int64_t partials = direct_plan(n, ntest).partials;
-  if (partials == 1) return nullptr;
-  const int64_t need = 4 * ntest * partials;
-  if (need <= c->dwork_cap) return c->dwork;
+  if (partials == 1 || 4 * ntest * partials > kDirectWork) return nullptr;
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(s, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) {
     (void)hipGetLastError();
     return nullptr;
   }
-  // kernels of earlier calls may still use the smaller buffer: hipFree waits
-  if (c->dwork) (void)hipFree(c->dwork);
-  c->dwork_cap = 0;
-  if (hipMalloc((void**)&c->dwork, sizeof(double) * (size_t)need) != hipSuccess) {
+  if (c->dwork) {
+    if (hipStreamWaitEvent(s, c->dwork_used, 0) == hipSuccess) return c->dwork;
     (void)hipGetLastError();
-    c->dwork = nullptr;
     return nullptr;
   }
-  c->dwork_cap = need;
+  // an allocation would break a capture that runs on some other stream
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  (void)hipThreadExchangeStreamCaptureMode(&mode);
+  if ((!c->dwork_used && hipEventCreateWithFlags(&c->dwork_used, hipEventDisableTiming) != hipSuccess) ||
+      hipMalloc((void**)&c->dwork, sizeof(double) * kDirectWork) != hipSuccess) {
+    (void)hipGetLastError();
+    c->dwork = nullptr;
+  }
+  (void)hipThreadExchangeStreamCaptureMode(&mode);
   return c->dwork;
+}
+
+// The workspace's kernels of this call are enqueued.
+static void direct_release(Ctx* c, hipStream_t s) {
+  if (hipEventRecord(c->dwork_used, s) != hipSuccess) (void)hipStreamSynchronize(s);
 }
 
 // directforce (src/utils/module_directsum.f90:34-172): with periodic
@@ -1169,10 +1180,12 @@ static void enqueue_direct(Ctx* c, hipStream_t s, int64_t n, const double* x, co
   double* work = direct_workspace(c, s, n, ntest);
   if (!c->periodic) {
     launch_direct(s, n, x, y, z, q, ntest, testidx, eps2, sign, ex, ey, ez, pot, work);
+    if (work) direct_release(c, s);
     return;
   }
   launch_direct(s, n, x, y, z, q, ntest, testidx, eps2, sign, ex, ey, ez, pot, work, c->nbox,
                 c->vbox);
+  if (work) direct_release(c, s);
   if (c->far_field && ntest > 0) {
     launch_lattice_sources(s, n, x, y, z, q, c->lgeom, c->ml, c->fact, c->lpart, c->ldpart, c->lom,
                            c->ldip, c->mu, c->fict, c->lcoef);

@@ -1117,8 +1117,6 @@ __global__ void publish_kernel(const DevScalars* __restrict__ src, DevScalars* _
 // writes its own partial sums, which direct_reduce_kernel adds in a fixed
 // order.  4096 targets against 1,048,576 sources: 4.2 ms; 178 ms with one
 // block per 256 targets (16 blocks) and a square root and a division per pair.
-constexpr int kDirectT = 256;
-
 __global__ __launch_bounds__(kDirectT) void direct_kernel(
     int64_t n, const double* __restrict__ x, const double* __restrict__ y,
     const double* __restrict__ z, const double* __restrict__ q, int64_t ntest,
@@ -1279,8 +1277,6 @@ void launch_walk_stats(hipStream_t s, const WalkArgs& a) {
 // About kDirectBlocks blocks: eight of four waves for each of the 256 CUs.  A
 // block never has fewer than 512 sources, and at most 65,535 ranges are used
 // (the grid's second dimension).  Without a workspace: whole targets.
-constexpr int64_t kDirectBlocks = 2048;
-
 DirectPlan direct_plan(int64_t n, int64_t ntest) {
   DirectPlan p;
   p.span = kDirectT;
