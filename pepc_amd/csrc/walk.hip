@@ -1142,7 +1142,8 @@ __global__ __launch_bounds__(kDirectT) void direct_kernel(
     const int self = tj >= base && tj < base + lim ? (int)(tj - base) : -1;
     double part[4] = {0.0, 0.0, 0.0, 0.0};
     auto term = [&](const double4& c, double px, double py, double pz, bool skip) {
-      const double dx = px - c.x, dy = py - c.y, dz = pz - c.z;
+      // (a skipped pair adds zero, also where the position is not finite)
+      const double dx = skip ? 0.0 : px - c.x, dy = skip ? 0.0 : py - c.y, dz = skip ? 0.0 : pz - c.z;
       const double r2 = dx * dx + dy * dy + dz * dz + eps2;
       const double rd = rsqrt(skip ? 1.0 : r2);
       const double qr = (skip ? 0.0 : c.w) * rd;
