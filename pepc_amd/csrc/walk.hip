@@ -103,9 +103,9 @@ struct Acc {
 // separation d is target minus centre of charge.
 // Every factor lies between r^-3 and the moments times r, so for charges near
 // one FP32 holds separations and softenings from 1e-11 to 1e12.  E summed as
-// r^-3 c d + r^-5 B d with a traceless B is an instruction shorter (4,194,304
-// particles: solve 6.62 ms against 6.66), but r^-5 leaves FP32 below a
-// separation of 2e-8 and above 4e7.
+// r^-3 c d + r^-5 B d with a traceless B is an instruction shorter (solve of
+// 4,194,304 particles 6.66 ms against 6.76, clustered 1,048,576 3.49 against
+// 3.53), but r^-5 leaves FP32 below a separation of 2e-8 and above 4e7.
 // Entry: {cx,cy,cz,q | -3 A2: xx,yy,zz,xy | yz,zx, 2 tr,px | py,pz,-,-}.
 // Without a dipole (DIP = false) its terms and its words are left out.
 template <typename R, bool DIP>
