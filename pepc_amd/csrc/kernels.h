@@ -40,15 +40,6 @@ void launch_scan(hipStream_t s, const uint32_t* in, uint32_t* out, int64_t n, ui
 void launch_group_list(hipStream_t s, int64_t n, const uint32_t* gmark, uint32_t* bsum,
                        uint32_t* gfirst, uint32_t* gcount, uint32_t* ngroups,
                        unsigned long long* clock);
-void launch_radix_pass(hipStream_t s, const unsigned long long* kin, const uint32_t* vin,
-                       unsigned long long* kout, uint32_t* vout, int64_t n, int shift, int nbits,
-                       uint32_t* hist, uint32_t* bsum);
-// One stable pass; afterwards bsum[0..255] holds the element count of each
-// digit value.
-void launch_radix_pass_dev(hipStream_t s, const unsigned long long* kin, const uint32_t* vin,
-                           unsigned long long* kout, uint32_t* vout, int64_t n, const uint32_t* ndev,
-                           int shift, int nbits, uint32_t* hist, uint32_t* bsum,
-                           const uint32_t* dsrc);
 // launch_sort_keys takes its input in (k1, v1) instead of (k0, v0).
 bool sort_input_second(int64_t n, bool batched);
 void launch_sort_keys(hipStream_t s, unsigned long long* k0, uint32_t* v0, unsigned long long* k1,

@@ -175,9 +175,8 @@ __device__ __forceinline__ uint32_t radix_digit(unsigned long long key, uint32_t
 
 __global__ __launch_bounds__(kSortThreads) void radix_hist_kernel(
     const unsigned long long* __restrict__ keys, const uint32_t* __restrict__ vals,
-    const uint32_t* __restrict__ dsrc, int64_t n, const uint32_t* __restrict__ ndev,
-    int shift, uint32_t mask, uint32_t* __restrict__ hist, int nblocks) {
-  if (ndev && (int64_t)*ndev < n) n = *ndev;
+    const uint32_t* __restrict__ dsrc, int64_t n, int shift, uint32_t mask,
+    uint32_t* __restrict__ hist, int nblocks) {
   __shared__ uint32_t cnt[kRadix];
   cnt[threadIdx.x] = 0;
   __syncthreads();
@@ -200,12 +199,10 @@ __global__ __launch_bounds__(kSortThreads) void radix_hist_kernel(
 __global__ __launch_bounds__(kSortThreads) void radix_scatter_kernel(
     const unsigned long long* __restrict__ kin, const uint32_t* __restrict__ vin,
     unsigned long long* __restrict__ kout, uint32_t* __restrict__ vout,
-    const uint32_t* __restrict__ dsrc, int64_t n,
-    const uint32_t* __restrict__ ndev, int shift, int nbits, const uint32_t* __restrict__ hscan,
-    const uint32_t* __restrict__ dtot, int nblocks, bool scan_here) {
-  if (ndev && (int64_t)*ndev < n) n = *ndev;
+    const uint32_t* __restrict__ dsrc, int64_t n, int shift, int nbits,
+    const uint32_t* __restrict__ hscan, const uint32_t* __restrict__ dtot, int nblocks,
+    bool scan_here) {
   const int64_t tile0 = (int64_t)blockIdx.x * kSortTile;
-  if (tile0 >= n) return;
   __shared__ uint32_t wcnt[kSortWaves][kRadix];
   __shared__ uint32_t lbase[kRadix];
   __shared__ uint32_t gbase[kRadix];
@@ -1037,28 +1034,20 @@ void launch_group_list(hipStream_t s, int64_t n, const uint32_t* gmark, uint32_t
                                                           ngroups, clock);
 }
 
-// One stable pass over bits [shift, shift + nbits), output in (kout, vout).
-// With ndev != nullptr the element count is min(n, *ndev), read on the device
-// (n then only sizes the grid), so no host round trip is needed.
-void launch_radix_pass_dev(hipStream_t s, const unsigned long long* kin, const uint32_t* vin,
-                           unsigned long long* kout, uint32_t* vout, int64_t n, const uint32_t* ndev,
-                           int shift, int nbits, uint32_t* hist, uint32_t* bsum,
-                           const uint32_t* dsrc) {
+// One stable pass over bits [shift, shift + nbits) of the keys (or, with dsrc,
+// of dsrc[value]), output in (kout, vout).
+static void launch_radix_pass(hipStream_t s, const unsigned long long* kin, const uint32_t* vin,
+                              unsigned long long* kout, uint32_t* vout, int64_t n, int shift,
+                              int nbits, uint32_t* hist, uint32_t* bsum, const uint32_t* dsrc) {
   const int nb = (int)sort_blocks(n);
-  radix_hist_kernel<<<nb, kSortThreads, 0, s>>>(kin, vin, dsrc, n, ndev, shift, (1u << nbits) - 1u,
-                                                hist, nb);
+  radix_hist_kernel<<<nb, kSortThreads, 0, s>>>(kin, vin, dsrc, n, shift, (1u << nbits) - 1u, hist,
+                                                nb);
   // Few blocks: each scatter block sums its digits' rows itself, one launch
   // fewer per pass.  Otherwise bsum[0..255] holds the digit totals.
   const bool scan_here = nb <= kScanHereBlocks;
   if (!scan_here) digit_scan_kernel<<<kRadix, kSortThreads, 0, s>>>(hist, nb, bsum);
-  radix_scatter_kernel<<<nb, kSortThreads, 0, s>>>(kin, vin, kout, vout, dsrc, n, ndev, shift, nbits,
-                                                   hist, bsum, nb, scan_here);
-}
-
-void launch_radix_pass(hipStream_t s, const unsigned long long* kin, const uint32_t* vin,
-                       unsigned long long* kout, uint32_t* vout, int64_t n, int shift, int nbits,
-                       uint32_t* hist, uint32_t* bsum) {
-  launch_radix_pass_dev(s, kin, vin, kout, vout, n, nullptr, shift, nbits, hist, bsum, nullptr);
+  radix_scatter_kernel<<<nb, kSortThreads, 0, s>>>(kin, vin, kout, vout, dsrc, n, shift, nbits, hist,
+                                                   bsum, nb, scan_here);
 }
 
 // Largest array sorted by merging.
@@ -1120,14 +1109,14 @@ void launch_sort_keys(hipStream_t s, unsigned long long* k0, uint32_t* v0, unsig
   static const int widths[8] = {8, 8, 8, 8, 8, 8, 8, 4};
   for (int p = 0; p < 8; ++p) {
     if (p % 2 == 0)
-      launch_radix_pass(s, k0, v0, k1, v1, n, shifts[p], widths[p], hist, bsum);
+      launch_radix_pass(s, k0, v0, k1, v1, n, shifts[p], widths[p], hist, bsum, nullptr);
     else
-      launch_radix_pass(s, k1, v1, k0, v0, n, shifts[p], widths[p], hist, bsum);
+      launch_radix_pass(s, k1, v1, k0, v0, n, shifts[p], widths[p], hist, bsum, nullptr);
   }
   if (sysid) {
-    launch_radix_pass_dev(s, k0, v0, k1, v1, n, nullptr, 0, 8, hist, bsum, sysid);
+    launch_radix_pass(s, k0, v0, k1, v1, n, 0, 8, hist, bsum, sysid);
     if (nsys > 256) {
-      launch_radix_pass_dev(s, k1, v1, k0, v0, n, nullptr, 8, 8, hist, bsum, sysid);
+      launch_radix_pass(s, k1, v1, k0, v0, n, 8, 8, hist, bsum, sysid);
     } else {
       launch_copy_pairs(s, k1, v1, k0, v0, n);
     }
