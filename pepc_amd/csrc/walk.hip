@@ -314,9 +314,8 @@ __device__ __forceinline__ void walk_group_mixed(const WalkArgs& a, uint32_t g, 
   const double ox = uniform(xt), oy = uniform(yt), oz = uniform(zt);   // lane 0: target a0
   const double lox = uniform_min(xt), loy = uniform_min(yt), loz = uniform_min(zt);
   const double hix = -uniform_min(-xt), hiy = -uniform_min(-yt), hiz = -uniform_min(-zt);
-  // target position in the kernel's frame (FP64: set per box below)
-  R tx = R(0), ty = R(0), tz = R(0);
-  tx = (R)(xt - ox); ty = (R)(yt - oy); tz = (R)(zt - oz);
+  // target position relative to the group's first particle
+  const R tx = (R)(xt - ox), ty = (R)(yt - oy), tz = (R)(zt - oz);
 
   MixedAcc acc;
 #pragma unroll
@@ -329,13 +328,11 @@ __device__ __forceinline__ void walk_group_mixed(const WalkArgs& a, uint32_t g, 
   double sx = xt, sy = yt, sz = zt;    // targets of the current box: x - vbox
 
   // Batches: entry k goes to slice k mod S; the loop count is uniform.
-  // FP32: two entries per pass (their LDS reads issued together), then the
-  // tail; FP64 keeps one entry per pass (register pressure).
+  // Two entries per pass (their LDS reads issued together), then the tail.
   auto flush_m2p = [&]() {
     uint32_t kk = 0;
-    constexpr bool kPair = true;
-    const uint32_t n2 = (kPair && nm >= 2 * S) ? nm - 2 * S + 1 : 0;
-    if (kPair && valid) {
+    const uint32_t n2 = nm >= 2 * S ? nm - 2 * S + 1 : 0;
+    if (valid) {
       for (; kk < n2; kk += 2 * S) {
         const uint32_t k = kk + s, k2 = k + S;
         const V4 e0 = lm[k][0], e1 = lm[k][1], e2 = lm[k][2], e3 = lm[k][3];
@@ -364,12 +361,11 @@ __device__ __forceinline__ void walk_group_mixed(const WalkArgs& a, uint32_t g, 
       return lpi[k] == tid;   // mirror-box entries hold ~0u
     }
   };
-  // FP32: two entries per pass as for M2P (same per-lane order of terms)
+  // Two entries per pass as for M2P (same per-lane order of terms).
   auto flush_p2p = [&]() {
     uint32_t kk = 0;
-    constexpr bool kPair = true;
-    const uint32_t n2 = (kPair && np >= 2 * S) ? np - 2 * S + 1 : 0;
-    if (kPair && valid) {
+    const uint32_t n2 = np >= 2 * S ? np - 2 * S + 1 : 0;
+    if (valid) {
       for (; kk < n2; kk += 2 * S) {
         const uint32_t k = kk + s, k2 = k + S;
         const V4 e = lp[k], f = lp[k2];
@@ -399,7 +395,7 @@ __device__ __forceinline__ void walk_group_mixed(const WalkArgs& a, uint32_t g, 
   sx = xt - vx; sy = yt - vy; sz = zt - vz;
   const Span bx = span_of(lox - vx, hix - vx), by = span_of(loy - vy, hiy - vy),
              bz = span_of(loz - vz, hiz - vz);
-  const double fox = ox - vx, foy = oy - vy, foz = oz - vz;   // FP32 node frame
+  const double fox = ox - vx, foy = oy - vy, foz = oz - vz;   // node frame
   if (lane == 0) stack[0] = root | kTwigBit;
   sp = 1;
   wave_order();
@@ -433,8 +429,7 @@ __device__ __forceinline__ void walk_group_mixed(const WalkArgs& a, uint32_t g, 
     }
     if (has && twig_entry) {
       kids = a.kidtwig[node];
-      const V4* src;
-      src = reinterpret_cast<const V4*>(&a.wm32[node]);
+      const V4* src = reinterpret_cast<const V4*>(&a.wm32[node]);
       w0 = src[0]; w1 = src[1]; w2 = src[2];
     }
     // Decide from the group's bounding box when possible (margins cover
@@ -520,10 +515,8 @@ __device__ __forceinline__ void walk_group_mixed(const WalkArgs& a, uint32_t g, 
     const unsigned long long pm = __ballot(leaf);
     if (take_m) {
       const uint32_t pos = nm + mask_rank(am);
-      V4 e0;
-      e0 = V4{(float)(gm.cx - fox), (float)(gm.cy - foy), (float)(gm.cz - foz), 0.0f};
       // w0 = {q, px, py, pz}, w1 = {2qx, 2qy, 2qz, xy}, w2 = {yz, zx, tr, -}
-      e0.w = w0.x;
+      const V4 e0 = V4{(float)(gm.cx - fox), (float)(gm.cy - foy), (float)(gm.cz - foz), w0.x};
       V4 e1, e2, e3;
       e1.x = w0.y; e1.y = w0.z; e1.z = w0.w; e1.w = w1.x;
       e2.x = w1.y; e2.y = w1.z; e2.z = w1.w; e2.w = w2.x;
@@ -532,8 +525,7 @@ __device__ __forceinline__ void walk_group_mixed(const WalkArgs& a, uint32_t g, 
     }
     if (leaf) {
       const uint32_t pos = np + mask_rank(pm);
-      V4 e;
-      e = V4{(float)(gm.cx - fox), (float)(gm.cy - foy), (float)(gm.cz - foz), (float)gm.b2};
+      const V4 e = V4{(float)(gm.cx - fox), (float)(gm.cy - foy), (float)(gm.cz - foz), (float)gm.b2};
       lp[pos] = e;
       lpi[pos] = (SINK || central) ? lk.first : ~0u;
     }
