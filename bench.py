@@ -3,7 +3,7 @@
 
 Workload: the Coulomb explosion system, N = 4,194,304 equal positive ions
 (q = 1/N) uniform in the unit ball, eps = 1e-3, theta = 0.6, quadrupole
-moments; FP32 + Kahan kernels (FP64 upward pass and acceptance tests).
+moments; FP32 kernels with FP64 running sums (FP64 upward pass and acceptance tests).
 A step is one grow + traverse of the whole system (keys, sort, tree build,
 upward pass, walk and P2P/M2P) with the particles already resident in HBM.
 
@@ -17,8 +17,10 @@ Usage: python bench.py [--gpus 1] [--steps K] [--warmup W]
 from __future__ import annotations
 
 import argparse
+import hashlib
 import json
 import os
+import re
 import sys
 import time
 
@@ -279,10 +281,34 @@ def tree_error(out, ref):
             "median_rel_pot_err": float(np.median(prel))}
 
 
+def walk_sources_sha16(csrc=os.path.join(ROOT, "pepc_amd", "csrc")):
+    """Hash of the sources that the walk kernel is compiled from, without
+    comments and white space."""
+    h = hashlib.sha256()
+    for name in ("walk.hip", "common.h", "kernels.h"):
+        with open(os.path.join(csrc, name)) as f:
+            text = re.sub(r"/\*.*?\*/|//[^\n]*", " ", f.read(), flags=re.S)
+        h.update(" ".join(text.split()).encode() + b"\0")
+    return h.hexdigest()[:16]
+
+
+def walk_counters(path, sha16):
+    """(HBM bytes, VALU instructions) per walk launch from the counter profile
+    at path; (None, None) unless it was taken from the walk sources sha16."""
+    try:
+        with open(path) as f:
+            rec = json.load(f)
+        if rec.get("walk_sources_sha16") != sha16:
+            return None, None
+        return rec.get("hbm_bytes_per_launch"), rec.get("sq_insts_valu_per_launch")
+    except (OSError, ValueError, AttributeError):
+        return None, None
+
+
 def valu_issue(insts, t_walk_ms):
     """Wave64 VALU instructions per walk launch (SQ_INSTS_VALU, from the
-    committed counter profile of the same workload) over this run's walk time,
-    against the issue rate the FP32 peak implies."""
+    committed counter profile of the same workload and the same sources) over
+    this run's walk time, against the issue rate the FP32 peak implies."""
     if not insts:
         return None
     rate = insts / (t_walk_ms * 1e-3)
@@ -455,15 +481,8 @@ def main():
         f"sampled energy rel err {energy['rel_err']:.3e}")
     flops = walk_flops(st)
     achieved = flops / (t_walk_ms * 1e-3) / 1e12
-    traffic = valu_insts = None
-    tp = os.path.join(ROOT, "profiles", "walk_explosion4m_traffic.json")
-    if os.path.exists(tp):
-        try:
-            rec = json.load(open(tp))
-            traffic = rec.get("hbm_bytes_per_launch")
-            valu_insts = rec.get("sq_insts_valu_per_launch")
-        except Exception:
-            traffic = valu_insts = None
+    traffic, valu_insts = walk_counters(
+        os.path.join(ROOT, "profiles", "walk_explosion4m_traffic.json"), walk_sources_sha16())
     sol.close()
 
     fp64 = None
