@@ -1134,8 +1134,7 @@ __global__ __launch_bounds__(kDirectT) void direct_kernel(
     const int self = tj >= base && tj < base + lim ? (int)(tj - base) : -1;
     double part[4] = {0.0, 0.0, 0.0, 0.0};
     auto term = [&](const double4& c, double px, double py, double pz, bool skip) {
-      // (a skipped pair adds zero, also where the position is not finite)
-      const double dx = skip ? 0.0 : px - c.x, dy = skip ? 0.0 : py - c.y, dz = skip ? 0.0 : pz - c.z;
+      const double dx = px - c.x, dy = py - c.y, dz = pz - c.z;
       const double r2 = dx * dx + dy * dy + dz * dz + eps2;
       const double rd = rsqrt(skip ? 1.0 : r2);
       const double qr = (skip ? 0.0 : c.w) * rd;
@@ -1299,8 +1298,12 @@ void launch_direct(hipStream_t s, int64_t n, const double* x, const double* y, c
     p.ranges = 1;
     work = nullptr;
   }
+  // A skipped pair adds zero times its separation, which is NaN for a target
+  // that is not at a finite position.  Any other source makes that component NaN
+  // too; a particle alone has no other, and its sums are empty.
+  const int64_t sources = n == 1 && !vbox ? 0 : n;
   direct_kernel<<<dim3((unsigned)p.tblocks, (unsigned)p.ranges), kDirectT, 0, s>>>(
-      n, x, y, z, q, ntest, testidx, eps2, sign, ex, ey, ez, pot, nbox, vbox, p.span, p.range, work);
+      sources, x, y, z, q, ntest, testidx, eps2, sign, ex, ey, ez, pot, nbox, vbox, p.span, p.range, work);
   if (work)
     direct_reduce_kernel<<<(unsigned)((4 * ntest + kDirectT / kWave - 1) / (kDirectT / kWave)),
                            kDirectT, 0, s>>>(ntest, (int)p.partials, work, sign, ex, ey, ez, pot);
