@@ -292,13 +292,14 @@ def walk_sources_sha16(csrc=os.path.join(ROOT, "pepc_amd", "csrc")):
     return h.hexdigest()[:16]
 
 
-def walk_counters(path, sha16):
+def walk_counters(path, sha16, workload):
     """(HBM bytes, VALU instructions) per walk launch from the counter profile
-    at path; (None, None) unless it was taken from the walk sources sha16."""
+    at path; (None, None) unless it was taken from the walk sources sha16 on
+    the same workload."""
     try:
         with open(path) as f:
             rec = json.load(f)
-        if rec.get("walk_sources_sha16") != sha16:
+        if rec.get("walk_sources_sha16") != sha16 or rec.get("workload") != workload:
             return None, None
         return rec.get("hbm_bytes_per_launch"), rec.get("sq_insts_valu_per_launch")
     except (OSError, ValueError, AttributeError):
@@ -482,7 +483,8 @@ def main():
     flops = walk_flops(st)
     achieved = flops / (t_walk_ms * 1e-3) / 1e12
     traffic, valu_insts = walk_counters(
-        os.path.join(ROOT, "profiles", "walk_explosion4m_traffic.json"), walk_sources_sha16())
+        os.path.join(ROOT, "profiles", "walk_explosion4m_traffic.json"), walk_sources_sha16(),
+        f"coulomb_explosion_n{s.n}_theta{args.theta} G={args.group} pack={args.pack} {args.precision}")
     sol.close()
 
     fp64 = None

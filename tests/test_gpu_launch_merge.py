@@ -1,8 +1,9 @@
 """Boxes, levels and groups at the edges of the blocks that produce them.
 
-Box: one block up to 4,096 particles of a system, several above (the block
-that finishes last joins them); batches from one system per block to many
-blocks per system.  The box is the coordinates' extrema with the margin of
+Box: from one block (up to 1,024 particles of a system) to many (the block that
+finishes last joins them; the edges of their rule are in
+test_gpu_box_blocks.py); batches from one system per block to many blocks per
+system.  The box is the coordinates' extrema with the margin of
 1/10000 of the extent, computed with the same operations, so it is compared
 exactly.  Groups: tiles of 4,096 marks; they cover the particles in order
 without gaps.  Repeated solves equal the first bit for bit (nothing that a

@@ -1,6 +1,7 @@
 """Tree build and upward pass at the edges of their tiles (512 particles, one
-tile more or less, the largest tree formed by tiles and the first formed by
-levels): node set and FP64 moments bit-exact against the oracle."""
+tile more or less) and at larger trees of both forms, by tiles and by levels
+(the edges between the forms are in test_gpu_upward_levels.py): node set and
+FP64 moments bit-exact against the oracle."""
 import numpy as np
 import pytest
 
