@@ -34,8 +34,8 @@
 // 3.0 clocks each.  So the design counts instructions: no dipole
 // terms for one-signed charges (41 -> 36 per pair), list remainders kept so
 // that passes are full, one ballot transposition for the exact tests and one
-// for the pushes.  3.76e9 instructions, walk 5.88 -> 5.24 ms (FP64
-// 11.56 -> 10.52, theta 0.3 at 500,009 particles 2.90 -> 2.58).
+// for the pushes.  Now 3.87e9 instructions at 3.0 clocks, FP64 4.97e9 at 4.8
+// (walk 5.13 and 10.2 ms).
 //
 // Periodic systems (PER): the group walks the tree once per lattice vector
 // vbox of the mirror boxes, with its targets shifted to x - vbox
